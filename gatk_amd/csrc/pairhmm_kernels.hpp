@@ -253,9 +253,10 @@ struct SwBatch {
     const int32_t *alt_len;
     int32_t match, mismatch, open, extend;  // SWParameters
     int32_t strategy;                       // 0 SOFTCLIP, 1 INDEL, 2 LEADING_INDEL, 3 IGNORE
-    int32_t max_ref_len;
-    uint8_t *scratch;                       // per wave: backtrack codes, last column, bottom row
-    size_t scratch_per_wave, bt_bytes_per_wave;
+    int32_t max_ref_len, max_alt_len;
+    uint8_t *scratch;                       // per wave: four bits per cell for the traceback
+    size_t scratch_per_wave;
+    uint32_t *queue_head;                   // next pair to take, 0 before the launch
     uint32_t *elems;                        // CIGAR elements (len << 2 | op), reference list order
     const int64_t *elem_off;                // per pair; capacity ref_len + alt_len + 4
     uint32_t *elems_short;                  // the first kSwShortElems elements of pair p at p * kSwShortElems
@@ -265,8 +266,7 @@ struct SwBatch {
 // Elements per pair in the compact copy the host reads back; a pair with more (rare: every element
 // but a clip consumes an indel or a run of matches) is read from the full list.
 constexpr int kSwShortElems = 16;
-size_t sw_lds_bytes(int max_ref_len);
-size_t sw_bt_bytes_per_wave(int max_ref_len, int max_alt_len);
+int sw_max_ref_len();
 size_t sw_scratch_bytes_per_wave(int max_ref_len, int max_alt_len);
 hipError_t launch_sw(const SwBatch &batch, uint32_t n_pairs, int grid_blocks, hipStream_t stream);
 

@@ -95,7 +95,7 @@ int32_t sw_run_batch(pairhmm_context *ctx, int64_t n_pairs, const uint8_t *ref_b
         alt_end = std::max(alt_end, alt_off[p] + alt_len[p]);
         elem_total += ref_len[p] + alt_len[p] + 4;
     }
-    if (sw_lds_bytes(max_r) > max_lds_per_block())
+    if (max_r > sw_max_ref_len())
         return fail(PAIRHMM_ERR_BAD_ARG, "reference of " + std::to_string(max_r) + " bases exceeds the LDS budget");
 
     size_t off = 0;
@@ -105,7 +105,8 @@ int32_t sw_run_batch(pairhmm_context *ctx, int64_t n_pairs, const uint8_t *ref_b
         return o;
     };
     const size_t o_rb = take(ref_end), o_ab = take(alt_end), o_roff = take(8 * n_pairs), o_rlen = take(4 * n_pairs),
-                 o_aoff = take(8 * n_pairs), o_alen = take(4 * n_pairs), o_eoff = take(8 * n_pairs);
+                 o_aoff = take(8 * n_pairs), o_alen = take(4 * n_pairs), o_eoff = take(8 * n_pairs),
+                 o_head = take(sizeof(uint32_t));
     const size_t in_bytes = off;
     const size_t o_short = take(4 * static_cast<size_t>(kSwShortElems) * n_pairs), o_n = take(4 * n_pairs),
                  o_off = take(4 * n_pairs);
@@ -113,8 +114,8 @@ int32_t sw_run_batch(pairhmm_context *ctx, int64_t n_pairs, const uint8_t *ref_b
     const size_t o_elems = take(4 * static_cast<size_t>(elem_total));  // device only
     const size_t per_wave = sw_scratch_bytes_per_wave(max_r, max_a);
     const int cus = std::max(ctx->num_cus, 1);
-    // 20 waves per CU: the 12-byte LDS row records of 600-base references allow it, and the sweep's
-    // lane-to-lane dependency chain needs many resident waves to hide its latency.
+    // 20 waves per CU, what the kernel's 96 VGPRs allow; a wave takes its pairs from a queue, so pairs of
+    // uneven size spread over the waves.
     int64_t waves = std::min<int64_t>(n_pairs, static_cast<int64_t>(cus) * 20);
     waves = std::max<int64_t>(1, std::min<int64_t>(waves, static_cast<int64_t>(kSwScratchBudget / per_wave)));
     const size_t o_scratch = take(per_wave * static_cast<size_t>(waves));
@@ -135,6 +136,7 @@ int32_t sw_run_batch(pairhmm_context *ctx, int64_t n_pairs, const uint8_t *ref_b
         eoff[p] = e;
         e += ref_len[p] + alt_len[p] + 4;
     }
+    *reinterpret_cast<uint32_t *>(hs + o_head) = 0u;
     uint8_t *ds = static_cast<uint8_t *>(ctx->stage_dev.ptr);
     HIP_TRY(hipMemcpyAsync(ds, hs, in_bytes, hipMemcpyHostToDevice, ctx->stream), PAIRHMM_ERR_KERNEL);
 
@@ -151,9 +153,10 @@ int32_t sw_run_batch(pairhmm_context *ctx, int64_t n_pairs, const uint8_t *ref_b
     b.extend = params->gap_extend_penalty;
     b.strategy = overhang_strategy;
     b.max_ref_len = max_r;
+    b.max_alt_len = max_a;
     b.scratch = ds + o_scratch;
     b.scratch_per_wave = per_wave;
-    b.bt_bytes_per_wave = sw_bt_bytes_per_wave(max_r, max_a);
+    b.queue_head = reinterpret_cast<uint32_t *>(ds + o_head);
     b.elems = reinterpret_cast<uint32_t *>(ds + o_elems);
     b.elem_off = reinterpret_cast<const int64_t *>(ds + o_eoff);
     b.elems_short = reinterpret_cast<uint32_t *>(ds + o_short);

@@ -156,3 +156,25 @@ def test_packed_text_too_small_is_an_error(binding):
                                                     ends.ctypes.data, offs.ctypes.data)
     assert st != 0
     assert (text[5:] == 0x7F).all()
+
+
+@pytest.mark.parametrize("strategy", list(SWOverhangStrategy))
+def test_sweep_edges(binding, strategy):
+    """Alternates at the edges of a lane's columns (64 K) and of a sweep (256), references at the edges of
+    the wave's fill and of its 8-step blocks, and gaps around the traceback's 64-cell fetch."""
+    rng = np.random.default_rng(int(strategy))
+    base = lambda n: bytes(np.frombuffer(b"ACGT", np.uint8)[rng.integers(0, 4, n)])  # noqa: E731
+    refs, alts = [], []
+    for A in (1, 64, 65, 128, 129, 192, 193, 255, 256, 257, 511, 512, 513):
+        for R in (1, 7, 8, 9, 62, 63, 64, 65, 72, 500):
+            ref = base(R)
+            refs.append(ref)
+            alts.append((ref + base(A))[:A] if rng.random() < 0.7 else base(A))
+    for gap in (1, 62, 63, 64, 65, 66, 128, 129, 200):
+        left, right, mid = base(90), base(90), base(gap)
+        refs += [left + mid + right, left + right]
+        alts += [left + right, left + mid + right]
+    params = NEW_SW_PARAMETERS
+    print(f"[sw] edges strategy={strategy.name} pairs={len(refs)}", flush=True)
+    for k, (r, a, g) in enumerate(zip(refs, alts, binding.align_batch(refs, alts, params, strategy))):
+        assert g == oracle.sw_align(r, a, _p(params), strategy.name), (k, len(r), len(a))
