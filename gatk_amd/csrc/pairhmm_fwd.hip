@@ -21,8 +21,8 @@
 //     ready-made sums per column, A(c) (its diagonal term) and B(c) (its vertical term), 8 columns
 //     per LDS read ahead of use, and the DPP products leave lane 0's preloaded value in place
 //     (wave_shr:1 without bound_ctrl), so no step waits on LDS.  FP32 forms A and B in a side pass
-//     over the three planes lane 63 left (M, I, S = I + D); FP64, whose planes are twice as large,
-//     has lane 63 form them directly into two planes.
+//     over the planes lane 63 left; FP64, whose planes are twice as large, has every row form the
+//     sums of the row below it, and gives a lane up to four rows.
 //   * Rows past R on the last stripe pass the last row down (M = D = 0, I = M + I of the row
 //     above), so the last stripe's planes end up holding M(R,c) + I(R,c).
 //   * Cells with c <= 0 or c > H are computed too (they are exact zeros, resp. never read by a real
@@ -261,16 +261,29 @@ __device__ double forward_pair_f32(const WaveLds<T> &L, int lane, int H, int R, 
     return wave_sum(acc);
 }
 
-// FP64 pass.  Each lane forms the sums the row below it needs from its own new M, S and I, with the
-// transitions of the row below (the next lane's row; for lane 63 the next stripe's first row):
-//   A(c+1) = M(c) MM' + S(c) GM'   and   B(c) = M(c) MI' + I(c) II',
-// and the row below takes them one lane over: B at the next step (same column), A two steps later
-// (the next column).  So two doubles cross lanes per step (four 32-bit DPP moves) where the
-// products over the row above would move four (M and S two steps back, M and I one step back), and
-// a lane needs only the next row's MM, GM, MI, II and its own MD, DD and priors.  Lane 63's sums are
-// lane 0's A and B of the next stripe; after the last stripe the next row is the pass-through row
-// (MM = GM = 0, MI = II = 1), so the B plane ends up holding M(R,c) + I(R,c).  Lane 0 takes A and B
-// as the old values of the DPP moves (wave_shr:1 without bound_ctrl leaves lane 0 unwritten).
+// FP64 pass.  A lane owns kRows consecutive rows and computes the same column of all of them at a
+// step: 4 rows (a stripe of 256) while more than 192 are left, then 2, then 1 for a last part of up to
+// 64, so a read is padded to 64 rows as with one row per lane.
+// Each row forms the sums the row below it needs from its own new M, S and I, with the transitions
+// of the row below:
+//   A(c+1) = M(c) MM' + S(c) GM'   and   B(c) = M(c) MI' + I(c) II'.
+// Within a lane the row below takes B at once and A at the next step; the next lane's first row takes
+// them one lane over: B at the next step (same column), A two steps later (the next column).  So two
+// doubles cross lanes per step (four 32-bit DPP moves) for kRows cells.  The last row's
+// sums of lane 63 are lane 0's A and B of the next stripe; after the last stripe the next row is the
+// pass-through row (MM = GM = 0, MI = II = 1), so the B plane ends up holding M(R,c) + I(R,c).  Lane 0
+// takes A and B as the old values of the DPP moves (wave_shr:1 without bound_ctrl leaves lane 0
+// unwritten).
+//
+// The prior: a row's match prior pm is folded into the transitions that form its A, so that a match
+// leaves M = A and only a mismatch multiplies, by px / pm, in the lanes that have one (an EXEC mask
+// around one product: two VALU instructions where a compare, two selects and a product were four).
+// An 'N' in the haplotype and qualities whose pm or MM is near 0 take the selects (kGeneric).
+//
+// Bound by VALU issue: 33 instructions per step of four cells and about 2 of block overhead, where one
+// row per lane and selected priors took 15 a cell.  Precision stress (40 regions, 1.07e11 cells, all
+// launches): 67.1 ms then, 49.2 with two rows per lane at 4 waves per SIMD, 45.2 with four at 3
+// (168 VGPRs), 43.2 with M's factor folded.
 //
 // Every lane stores its (B(c), A(c+1)) at its own column c = t - lane into an LDS ring at step t (no
 // one-lane exec mask in the step); lane 63 writes column c last, at step c + 63.  After each block
@@ -288,81 +301,217 @@ __device__ double forward_pair_f32(const WaveLds<T> &L, int lane, int H, int R, 
 // is reloaded with the next block's first four columns, after step 7 the second half.  A wait for
 // the wave's stores at each stripe start orders the previous stripe's stores before these loads;
 // all accesses come from one wave on one CU, so its L1 holds no stale copy.
-template <int kCols, bool kHapHasN>
-__device__ double forward_pair_f64(const WaveLds<double> &L, int lane, int H, int R, const uint8_t *__restrict__ rb,
-                                   const uint8_t *__restrict__ rq, const uint8_t *__restrict__ ri,
-                                   const uint8_t *__restrict__ rd, const uint8_t *__restrict__ rg,
-                                   const DeviceTables &tab) {
-    const int n_stripes = (R + kWave - 1) / kWave;
-    const int steps = round_up(H + kWave, kUnroll);
-    double *P = L.bm;  // A(c) at 2 (kLdsPad + c), B(c) at 2 (kLdsPad + c) + 1
-    using lds_u8 = const volatile __attribute__((address_space(3))) uint8_t;
-    lds_u8 *hp = (lds_u8 *)(L.hap + kLdsPad - 1 - lane);  // address-space cast: C-style only
+
+// Per row, in the lanes whose haplotype byte differs from the row's base: a *= ratio.  EXEC is all ones
+// before and after (whole waves, uniform control flow); the s_nop completes the five wait states a DPP
+// needs after a VALU write of EXEC, which the compiler does not track across inline assembly.
+__device__ __forceinline__ void scale_mismatch(double (&a)[1], const double (&ratio)[1], uint32_t hb,
+                                               const uint32_t (&base)[1]) {
+    asm("v_cmpx_ne_u32_e32 vcc, %2, %3\n\t"
+        "v_mul_f64 %0, %0, %1\n\t"
+        "s_mov_b64 exec, -1\n\t"
+        "s_nop 2"
+        : "+v"(a[0])
+        : "v"(ratio[0]), "v"(hb), "v"(base[0])
+        : "vcc");
+}
+__device__ __forceinline__ void scale_mismatch(double (&a)[2], const double (&ratio)[2], uint32_t hb,
+                                               const uint32_t (&base)[2]) {
+    asm("v_cmpx_ne_u32_e32 vcc, %4, %5\n\t"
+        "v_mul_f64 %0, %0, %2\n\t"
+        "s_mov_b64 exec, -1\n\t"
+        "v_cmpx_ne_u32_e32 vcc, %4, %6\n\t"
+        "v_mul_f64 %1, %1, %3\n\t"
+        "s_mov_b64 exec, -1\n\t"
+        "s_nop 2"
+        : "+v"(a[0]), "+v"(a[1])
+        : "v"(ratio[0]), "v"(ratio[1]), "v"(hb), "v"(base[0]), "v"(base[1])
+        : "vcc");
+}
+__device__ __forceinline__ void scale_mismatch(double (&a)[4], const double (&ratio)[4], uint32_t hb,
+                                               const uint32_t (&base)[4]) {
+    asm("v_cmpx_ne_u32_e32 vcc, %8, %9\n\t"
+        "v_mul_f64 %0, %0, %4\n\t"
+        "s_mov_b64 exec, -1\n\t"
+        "v_cmpx_ne_u32_e32 vcc, %8, %10\n\t"
+        "v_mul_f64 %1, %1, %5\n\t"
+        "s_mov_b64 exec, -1\n\t"
+        "v_cmpx_ne_u32_e32 vcc, %8, %11\n\t"
+        "v_mul_f64 %2, %2, %6\n\t"
+        "s_mov_b64 exec, -1\n\t"
+        "v_cmpx_ne_u32_e32 vcc, %8, %12\n\t"
+        "v_mul_f64 %3, %3, %7\n\t"
+        "s_mov_b64 exec, -1\n\t"
+        "s_nop 2"
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3])
+        : "v"(ratio[0]), "v"(ratio[1]), "v"(ratio[2]), "v"(ratio[3]), "v"(hb), "v"(base[0]), "v"(base[1]),
+          "v"(base[2]), "v"(base[3])
+        : "vcc");
+}
+
+// Rows per lane of the stripe that starts with `left` rows to go.
+__device__ __forceinline__ int f64_stripe_rows(int left) {
+    return left > 3 * kWave ? 4 : left > kWave ? 2 : 1;
+}
+
+// What a row's M is multiplied with along a lane (fast path): g = pm' MM' g' of the row below it in the
+// lane, 1 for the lane's last row and above a pass-through row.  The row below takes A with pm' g'
+// folded in, so M's term in it has the factor 1 and costs no product.
+template <int kRows>
+__device__ __forceinline__ void f64_scales(const RowTrans<double> (&w)[kRows], const bool (&real)[kRows],
+                                           double (&g)[kRows]) {
+    g[kRows - 1] = 1.0;
+#pragma unroll
+    for (int j = kRows - 2; j >= 0; --j) g[j] = real[j + 1] ? w[j + 1].pm * w[j + 1].MM * g[j + 1] : 1.0;
+}
+
+// The factor folded into the sums that reach the row at read position p, the first of its lane in a
+// stripe of `rows` rows per lane (wave-uniform arguments).
+__device__ __forceinline__ double f64_first_fold(int p, int rows, int R, const uint8_t *__restrict__ rb,
+                                                 const uint8_t *__restrict__ rq, const uint8_t *__restrict__ ri,
+                                                 const uint8_t *__restrict__ rd, const uint8_t *__restrict__ rg,
+                                                 const DeviceTables &tab) {
+    double f = 1.0;
+    for (int j = 0; j < rows && p + j < R; ++j) {
+        const RowTrans<double> w = row_trans<double>(p + j, R, rb, rq, ri, rd, rg, tab);
+        f *= j == 0 ? w.pm : w.pm * w.MM;
+    }
+    return f;
+}
+
+// One stripe: rows of read positions p0 + kRows lane .. + kRows - 1.
+template <int kRows, bool kGeneric>
+__device__ __forceinline__ void f64_stripe(double *P, __attribute__((address_space(3))) double *const ring,
+                                           const volatile __attribute__((address_space(3))) uint8_t *hp, int lane,
+                                           int steps, int p0, int R, const uint8_t *__restrict__ rb,
+                                           const uint8_t *__restrict__ rq, const uint8_t *__restrict__ ri,
+                                           const uint8_t *__restrict__ rd, const uint8_t *__restrict__ rg,
+                                           const DeviceTables &tab) {
     using lds_f64 = __attribute__((address_space(3))) double;
-    lds_f64 *const ring = (lds_f64 *)L.ring;  // slot k: B at 2 k, A at 2 k + 1
     constexpr int kLag = kWave - 1;
     int zoff;
     asm volatile("v_mov_b32 %0, 0" : "=v"(zoff));
     const double *r0 = P + 2 * kLdsPad + zoff;
     // Copy-out: lane handles column offset v of the block's finished columns.
     const int v = lane & (kUnroll - 1);
-    for (int s = 0; s < n_stripes; ++s) {
-        const RowTrans<double> w = row_trans<double>(s * kWave + lane, R, rb, rq, ri, rd, rg, tab);
-        const RowTrans<double> wn = row_trans<double>(s * kWave + lane + 1, R, rb, rq, ri, rd, rg, tab);
-        // dd = D / MD: D(c) = D(c-1) DD + M(c-1) MD becomes dd(c) = dd(c-1) DD + M(c-1), and
-        // S = I + D = I + MD dd, one FMA each (rows past R have MD = DD = 0, so S = I there).
-        double m1 = 0, dd1 = 0;
-        double an1 = 0, an2 = 0, bn1 = 0;  // sums for the row below, one and two steps back
-        // The previous stripe's (or the initial) stores complete before this stripe reads them.
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-        double ab[2 * kUnroll];
-        __builtin_memcpy(ab, __builtin_assume_aligned(r0, 16), sizeof(ab));
-        for (int t0 = 0; t0 < steps; t0 += kUnroll) {
-            lds_f64 *wr = ring + 2 * ((t0 - lane) & 127);
-            uint32_t hbs[kUnroll];
+    // Row j's own MD, DD and priors; the transitions of the row below it (n).  Generic: px is the
+    // mismatch prior.  Fast: pm is folded into the sums, px is px / pm, M carries the factor g.
+    double MD[kRows], DD[kRows], pm[kRows], px[kRows], MMn[kRows], GMn[kRows], MIn[kRows], IIn[kRows];
+    uint32_t base[kRows];
+    {
+        RowTrans<double> w[kRows];
+        bool real[kRows];
+        double g[kRows];
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) hbs[u] = hp[t0 + u];
-            __builtin_amdgcn_wave_barrier();
+        for (int j = 0; j < kRows; ++j) {
+            w[j] = row_trans<double>(p0 + kRows * lane + j, R, rb, rq, ri, rd, rg, tab);
+            real[j] = p0 + kRows * lane + j < R;
+        }
+        f64_scales(w, real, g);
+        const int p_next = p0 + kRows * kWave;
+        double fold = 1.0;
+        if constexpr (!kGeneric) {
+            fold = f64_first_fold(p_next, f64_stripe_rows(R - p_next), R, rb, rq, ri, rd, rg, tab);
+            fold = wave_shl1(fold, real[0] ? w[0].pm * g[0] : 1.0);
+        }
+        const RowTrans<double> below = row_trans<double>(p0 + kRows * lane + kRows, R, rb, rq, ri, rd, rg, tab);
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                const uint32_t hb = hbs[u];
-                const bool match = (hb == w.base) || (kHapHasN && hb == 'N');
-                const double prior = match ? w.pm : w.px;
-                double a = ab[2 * u], i = ab[2 * u + 1];
-                a = wave_shr1(a, an2);  // lane 0 keeps its plane values
-                i = wave_shr1(i, bn1);
-                const double m = a * prior;
-                const double dd = fma(dd1, w.DD, m1);
-                const double sx = fma(dd, w.MD, i);
-                const double an = fma(sx, wn.GM, m * wn.MM);
-                const double bn = fma(i, wn.II, m * wn.MI);
-                wr[2 * u] = bn;
-                wr[2 * u + 1] = an;
-                an2 = an1;
-                an1 = an;
-                bn1 = bn;
-                m1 = m;
-                dd1 = dd;
-                // The next block's halves, loaded unconditionally (the slice has slots past the last
-                // block): with a fixed count of loads in the loop, the wait for a half is a counted
-                // one instead of a full drain at the block start.
-                if (u == kUnroll / 2 - 1)
-                    __builtin_memcpy(ab, __builtin_assume_aligned(r0 + 2 * (t0 + kUnroll), 16), sizeof(ab) / 2);
-                if (u == kUnroll - 1)
-                    __builtin_memcpy(ab + kUnroll, __builtin_assume_aligned(r0 + 2 * (t0 + kUnroll) + kUnroll, 16),
-                                     sizeof(ab) / 2);
+        for (int j = 0; j < kRows; ++j) {
+            const RowTrans<double> wn = j + 1 < kRows ? w[j + 1 < kRows ? j + 1 : 0] : below;
+            const double f = kGeneric ? 1.0 : j + 1 < kRows ? wn.pm * g[j + 1 < kRows ? j + 1 : 0] : fold;
+            const double inv_g = kGeneric || j + 1 == kRows ? 1.0 : 1.0 / g[j];
+            MMn[j] = wn.MM * f;
+            GMn[j] = wn.GM * f;
+            MIn[j] = wn.MI * inv_g;
+            IIn[j] = wn.II;
+            MD[j] = w[j].MD * inv_g;
+            DD[j] = w[j].DD;
+            pm[j] = w[j].pm;
+            px[j] = kGeneric ? w[j].px : real[j] ? w[j].px / w[j].pm : 0.0;
+            base[j] = kGeneric || real[j] ? w[j].base : 0x1FFu;  // a pass-through row matches nothing: M = 0
+        }
+    }
+    // dd = D / MD: D(c) = D(c-1) DD + M(c-1) MD becomes dd(c) = dd(c-1) DD + M(c-1), and
+    // S = I + D = I + MD dd, one FMA each (rows past R have MD = DD = 0, so S = I there).
+    double m[kRows] = {}, dd[kRows] = {};
+    double an1[kRows] = {}, an2 = 0, bn1 = 0;  // sums for the row below; the last row's two steps back
+    // The previous stripe's (or the initial) stores complete before this stripe reads them.
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    double ab[2 * kUnroll];
+    __builtin_memcpy(ab, __builtin_assume_aligned(r0, 16), sizeof(ab));
+    for (int t0 = 0; t0 < steps; t0 += kUnroll) {
+        lds_f64 *wr = ring + 2 * ((t0 - lane) & 127);
+        uint32_t hbs[kUnroll];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) hbs[u] = hp[t0 + u];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            const uint32_t hb = hbs[u];
+            double a[kRows];
+            double i = wave_shr1(ab[2 * u + 1], bn1);  // lane 0 keeps its plane values
+            a[0] = wave_shr1(ab[2 * u], an2);
+#pragma unroll
+            for (int j = 1; j < kRows; ++j) a[j] = an1[j - 1];
+            an2 = an1[kRows - 1];
+            if constexpr (!kGeneric) scale_mismatch(a, px, hb, base);
+            double an = 0, bn = 0;
+#pragma unroll
+            for (int j = 0; j < kRows; ++j) {
+                if constexpr (kGeneric) a[j] *= (hb == base[j] || hb == 'N') ? pm[j] : px[j];
+                dd[j] = fma(dd[j], DD[j], m[j]);
+                m[j] = a[j];
+                const double sx = fma(dd[j], MD[j], i);
+                an = fma(sx, GMn[j], kGeneric || j + 1 == kRows ? m[j] * MMn[j] : m[j]);
+                bn = fma(i, IIn[j], m[j] * MIn[j]);
+                an1[j] = an;
+                i = bn;
             }
-            __builtin_amdgcn_wave_barrier();
-            // Lane 63 finished columns t0 - 63 .. t0 - 56 in this block, at ring slots
-            // ((t0 - 63) mod 128) + v: (B(c), A(c + 1)) as they go to the plane.
-            {
-                const lds_f64 *rs = ring + 2 * (((t0 - kLag) & 127) + v);
-                const double ba[2] = {rs[0], rs[1]};
-                __builtin_memcpy(P + 2 * (kLdsPad + t0 - kLag + v) + 1, ba, sizeof(ba));
-            }
-            __builtin_amdgcn_wave_barrier();
+            bn1 = bn;
+            wr[2 * u] = bn;
+            wr[2 * u + 1] = an;
+            // The next block's halves, loaded unconditionally (the slice has slots past the last
+            // block): with a fixed count of loads in the loop, the wait for a half is a counted
+            // one instead of a full drain at the block start.
+            if (u == kUnroll / 2 - 1)
+                __builtin_memcpy(ab, __builtin_assume_aligned(r0 + 2 * (t0 + kUnroll), 16), sizeof(ab) / 2);
+            if (u == kUnroll - 1)
+                __builtin_memcpy(ab + kUnroll, __builtin_assume_aligned(r0 + 2 * (t0 + kUnroll) + kUnroll, 16),
+                                 sizeof(ab) / 2);
         }
         __builtin_amdgcn_wave_barrier();
+        // Lane 63 finished columns t0 - 63 .. t0 - 56 in this block, at ring slots
+        // ((t0 - 63) mod 128) + v: (B(c), A(c + 1)) as they go to the plane.
+        {
+            const lds_f64 *rs = ring + 2 * (((t0 - kLag) & 127) + v);
+            const double ba[2] = {rs[0], rs[1]};
+            __builtin_memcpy(P + 2 * (kLdsPad + t0 - kLag + v) + 1, ba, sizeof(ba));
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int kCols, bool kGeneric>
+__device__ double forward_pair_f64(const WaveLds<double> &L, int lane, int H, int R, const uint8_t *__restrict__ rb,
+                                   const uint8_t *__restrict__ rq, const uint8_t *__restrict__ ri,
+                                   const uint8_t *__restrict__ rd, const uint8_t *__restrict__ rg,
+                                   const DeviceTables &tab) {
+    const int steps = round_up(H + kWave, kUnroll);
+    double *P = L.bm;  // A(c) at 2 (kLdsPad + c), B(c) at 2 (kLdsPad + c) + 1
+    using lds_u8 = const volatile __attribute__((address_space(3))) uint8_t;
+    lds_u8 *hp = (lds_u8 *)(L.hap + kLdsPad - 1 - lane);  // address-space cast: C-style only
+    using lds_f64 = __attribute__((address_space(3))) double;
+    lds_f64 *const ring = (lds_f64 *)L.ring;  // slot k: B at 2 k, A at 2 k + 1
+    for (int p0 = 0; p0 < R;) {
+        const int rows = f64_stripe_rows(R - p0);
+        if (rows == 4)
+            f64_stripe<4, kGeneric>(P, ring, hp, lane, steps, p0, R, rb, rq, ri, rd, rg, tab);
+        else if (rows == 2)
+            f64_stripe<2, kGeneric>(P, ring, hp, lane, steps, p0, R, rb, rq, ri, rd, rg, tab);
+        else
+            f64_stripe<1, kGeneric>(P, ring, hp, lane, steps, p0, R, rb, rq, ri, rd, rg, tab);
+        p0 += rows * kWave;
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the last stripe's B values are complete
     double acc = 0.0;
@@ -370,14 +519,15 @@ __device__ double forward_pair_f64(const WaveLds<double> &L, int lane, int H, in
     return wave_sum(acc);
 }
 
-template <typename T, int kCols, bool kHapHasN>
+// kGeneric: the haplotype has an 'N' (FP64: or the read a base quality of 0).
+template <typename T, int kCols, bool kGeneric>
 __device__ __forceinline__ double forward_pair(const WaveLds<T> &L, int lane, int H, int R, const uint8_t *rb,
                                                const uint8_t *rq, const uint8_t *ri, const uint8_t *rd,
                                                const uint8_t *rg, const DeviceTables &tab) {
     if constexpr (sizeof(T) == sizeof(double))
-        return forward_pair_f64<kCols, kHapHasN>(L, lane, H, R, rb, rq, ri, rd, rg, tab);
+        return forward_pair_f64<kCols, kGeneric>(L, lane, H, R, rb, rq, ri, rd, rg, tab);
     else
-        return forward_pair_f32<T, kCols, kHapHasN>(L, lane, H, R, rb, rq, ri, rd, rg, tab);
+        return forward_pair_f32<T, kCols, kGeneric>(L, lane, H, R, rb, rq, ri, rd, rg, tab);
 }
 
 template <typename T, int kCols>
@@ -411,8 +561,21 @@ __device__ void process_pair(const DeviceBatch &b, const DeviceTables &tab, cons
     const T d0 = static_cast<T>(__builtin_ldexp(1.0, Scale<T>::kExp) / static_cast<double>(H));
     // Row 1's sums over row 0 (M = I = 0, D = 2^S / H from column 0 on): A(c) = d0 GM_1 for c >= 1,
     // B(c) = 0 (FP32: A in the M plane, B in the I plane; FP64: interleaved, A at 2 j, B at 2 j + 1).
-    const T gm1 = row_trans<T>(0, R, b.rd_bases + ro, b.rd_quals + ro, b.rd_ins + ro, b.rd_del + ro,
-                               b.rd_gcp + ro, tab).GM;
+    const RowTrans<T> row1 = row_trans<T>(0, R, b.rd_bases + ro, b.rd_quals + ro, b.rd_ins + ro, b.rd_del + ro,
+                                          b.rd_gcp + ro, tab);
+    bool generic = __any(has_n);
+    T gm1 = row1.GM;
+    if constexpr (sizeof(T) == sizeof(double)) {
+        // The fast path divides by match priors and MM: base quality 0 (pm = 0) and gap-open qualities
+        // under 4 (from there on MM >= 0.2) take the generic one.
+        int low = 0;
+        for (int p = lane; p < R; p += kWave)
+            low |= b.rd_quals[ro + p] == 0 || b.rd_ins[ro + p] < 4 || b.rd_del[ro + p] < 4;
+        generic = generic || __any(low);
+        if (!generic)
+            gm1 *= f64_first_fold(0, f64_stripe_rows(R), R, b.rd_bases + ro, b.rd_quals + ro, b.rd_ins + ro,
+                                  b.rd_del + ro, b.rd_gcp + ro, tab);
+    }
     for (int j = lane; j < kCols; j += kWave) {
         const T a0 = j >= kLdsPad + 1 ? d0 * gm1 : T(0);
         if constexpr (sizeof(T) == sizeof(float)) {
@@ -424,7 +587,7 @@ __device__ void process_pair(const DeviceBatch &b, const DeviceTables &tab, cons
         }
     }
     double sum;
-    if (__any(has_n))
+    if (generic)
         sum = forward_pair<T, kCols, true>(L, lane, H, R, b.rd_bases + ro, b.rd_quals + ro, b.rd_ins + ro, b.rd_del + ro,
                                     b.rd_gcp + ro, tab);
     else
@@ -445,7 +608,7 @@ __device__ void process_pair(const DeviceBatch &b, const DeviceTables &tab, cons
 }
 
 template <typename T, int kCols>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) == sizeof(double) ? 4 : 1)))
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) == sizeof(double) ? 3 : 1)))
 void forward_kernel(DeviceBatch b, DeviceTables tab, WorkSource ws, RescueSink rs) {
     extern __shared__ __align__(16) uint8_t lds_raw[];
     const int lane = threadIdx.x & (kWave - 1);

@@ -228,6 +228,41 @@ def test_fp64_kernel_random_shapes(engine64):
     assert np.max(np.abs(out[fin] - want[fin])) <= FP64_TOL
 
 
+@pytest.mark.parametrize("case", ["plain", "base_quality_0", "low_gap_open", "hap_n", "read_n"])
+def test_fp64_kernel_stripe_row_counts(engine64, case):
+    """The FP64 kernel against the oracle at 1e-9 where its stripes change between 4, 2 and 1 rows per lane
+    (64, 128, 192 and 256 rows to go) and on the inputs that leave its fast path: base quality 0, gap-open
+    qualities under 4, an 'N' in the haplotype; an 'N' in the read stays on it."""
+    rng = np.random.default_rng(31)
+    regions = []
+    for R in (1, 2, 3, 4, 5, 63, 64, 65, 127, 128, 129, 191, 192, 193, 194, 255, 256, 257, 319, 320, 321, 384, 385, 447,
+              448, 449, 450, 511, 512, 513):
+        haps = [rng.choice(list(b"ACGT"), H).astype(np.uint8) for H in (7, 150)]
+        bases = np.concatenate([haps[1]] * 4)[:R].copy()
+        bases[rng.integers(0, R, 3)] = ord("A")
+        q, ins, dele = (rng.integers(a, z, R).astype(np.uint8) for a, z in ((1, 41), (4, 60), (4, 60)))
+        at = rng.integers(0, R, 2)
+        if case == "base_quality_0":
+            q[at] = 0
+        elif case == "low_gap_open":
+            ins[at] = rng.integers(0, 4, 2)
+            dele[at[::-1]] = rng.integers(0, 4, 2)
+        elif case == "hap_n":
+            haps[1][rng.integers(0, 150, 2)] = ord("N")
+        elif case == "read_n":
+            bases[at] = ord("N")
+        regions.append((haps, [(bases, q, ins, dele, rng.integers(5, 20, R).astype(np.uint8))]))
+    b = pack_regions(regions)
+    want = oracle.logless_batch(b, n_threads=8)
+    dev = engine64.upload(b)
+    out = np.empty(b.n_pairs)
+    dev.forward(mode=_native.RUN_FP64, out=out)
+    dev.free()
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isfinite(out), fin)
+    assert np.max(np.abs(out[fin] - want[fin])) <= FP64_TOL
+
+
 def _repeat_pairs(read_unit, ref_unit, copies):
     """Reads and haplotypes of repeated units with the qualities of PairHMMUnitTest's big-read case
     (base 30, insertion 40, deletion 40, gap continuation 10)."""
