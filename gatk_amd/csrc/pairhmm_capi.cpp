@@ -1069,7 +1069,7 @@ extern "C" int32_t pairhmm_dragstr_impute_device(pairhmm_context *ctx, const dou
     if (!read_bases || !read_off || !read_len || !out_gop || !out_gcp)
         return fail(PAIRHMM_ERR_BAD_ARG, "null device pointer");
     HIP_TRY(hipSetDevice(ctx->device), PAIRHMM_ERR_KERNEL);
-    HIP_TRY(launch_dragstr_impute(read_bases, read_off, read_len, n_reads, t, out_gop, out_gcp, ctx->stream),
+    HIP_TRY(launch_dragstr_impute(read_bases, read_off, read_len, n_reads, max_read_len, t, out_gop, out_gcp, ctx->stream),
             PAIRHMM_ERR_KERNEL);
     HIP_TRY(hipStreamSynchronize(ctx->stream), PAIRHMM_ERR_KERNEL);
     return PAIRHMM_OK;

@@ -184,8 +184,8 @@ struct DragstrByteTables {
     uint8_t gop[512], gcp[512];
 };
 hipError_t launch_dragstr_impute(const uint8_t *bases, const int64_t *read_off, const int32_t *read_len,
-                                 int64_t n_reads, const DragstrByteTables &tables, uint8_t *out_gop, uint8_t *out_gcp,
-                                 hipStream_t stream);
+                                 int64_t n_reads, int max_read_len, const DragstrByteTables &tables, uint8_t *out_gop,
+                                 uint8_t *out_gcp, hipStream_t stream);
 int dragstr_max_read_length();
 
 // ---- partially determined PairHMM (pdhmm.hip) ----------------------------------------------

@@ -168,3 +168,66 @@ def test_dragstr_impute_device_matches_host(seed):
             prep.dragstr_impute(params, t(bases), t(off), t(lens), d_gop, d_gcp)
             np.testing.assert_array_equal(d_gop.cpu().numpy(), want_gop)
             np.testing.assert_array_equal(d_gcp.cpu().numpy(), want_gcp)
+
+
+def _edge_reads(rng):
+    """Reads whose lengths and repeat runs lie at the edges of the kernels' 64-position masks and of the
+    imputer's 512-position capacity: random bases with a tract of a 1-12 base unit placed around each
+    multiple of 64, homopolymers, and pure repeats."""
+    reads = []
+    for L in (1, 2, 3, 8, 9, 62, 63, 64, 65, 66, 127, 128, 129, 192, 193, 255, 256, 257, 300, 511, 512):
+        for unit in (1, 2, 3, 5, 8, 12):
+            s = rng.choice(list(b"ACGT"), L).astype(np.uint8)
+            motif = rng.choice(list(b"ACGT"), unit).astype(np.uint8)
+            for m in range(0, L, 64):
+                a = max(0, m - int(rng.integers(0, 40)))
+                tract = np.tile(motif, 12)[:max(0, min(L - a, int(rng.integers(unit, 90))))]
+                s[a:a + len(tract)] = tract
+            reads.append(s.tobytes())
+        reads += [b"A" * L, (b"ACG" * L)[:L], (b"ACGTTGCA" * L)[:L]]
+    return reads
+
+
+def test_pcr_error_model_at_mask_edges():
+    rng = np.random.default_rng(41)
+    reads = _edge_reads(rng)
+    bases, off, lens, _, ins, dels, _ = _pack(reads, rng)
+    t = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    d_ins, d_del = t(ins.copy()), t(dels.copy())
+    with ReadPrep() as prep:
+        prep.apply_pcr_error_model(t(bases), t(off), t(lens), d_ins, d_del, PCRErrorModel.CONSERVATIVE)
+    got_i, got_d = d_ins.cpu().numpy(), d_del.cpu().numpy()
+    for r, read in enumerate(reads):
+        o, L = int(off[r]), int(lens[r])
+        wi, wd = rp.apply_pcr_error_model(read, ins[o:o + L], dels[o:o + L], "CONSERVATIVE")
+        assert list(got_i[o:o + L]) == wi, read
+        assert list(got_d[o:o + L]) == wd, read
+
+
+@pytest.mark.parametrize("periods,repeats,longest,declared", [(8, 20, 512, 512), (1, 20, 512, 512), (16, 30, 512, 512),
+                                                              (70, 4, 512, 512), (8, 20, 4096, 4096),
+                                                              (8, 20, 600, 300)])
+def test_dragstr_impute_at_mask_edges(periods, repeats, longest, declared):
+    """Periods from 1 to more than a mask's 64 positions, reads up to both capacities, and reads over the
+    length the caller declared."""
+    from gatk_amd.dragstr import DragstrParams, DragstrPairHMMInputScoreImputator
+
+    rng = np.random.default_rng(periods + longest)
+    reads = _edge_reads(rng)
+    if longest > 512:
+        reads += [rng.choice(list(b"AC"), n).astype(np.uint8).tobytes() for n in (513, longest - 1, longest)]
+        reads += [b"G" * longest, (b"ACGTT" * longest)[:longest]]
+    bases, off, lens, *_ = _pack(reads, rng)
+
+    class _B:
+        read_bases, read_off, read_len = bases, off, lens
+
+    params = DragstrParams(rng.uniform(5, 50, (periods, repeats)), rng.uniform(2, 20, (periods, repeats)),
+                           np.zeros((periods, repeats)), name="random")
+    want_gop, want_gcp = DragstrPairHMMInputScoreImputator(params).impute_batch(_B)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    d_gop, d_gcp = (torch.zeros(len(bases), dtype=torch.uint8, device="cuda") for _ in range(2))
+    with ReadPrep() as prep:
+        prep.dragstr_impute(params, t(bases), t(off), t(lens), d_gop, d_gcp, declared)
+    np.testing.assert_array_equal(d_gop.cpu().numpy(), want_gop)
+    np.testing.assert_array_equal(d_gcp.cpu().numpy(), want_gcp)
