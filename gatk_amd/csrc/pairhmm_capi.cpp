@@ -1058,6 +1058,7 @@ extern "C" int32_t pairhmm_dragstr_impute_device(pairhmm_context *ctx, const dou
     DragstrByteTables t{};
     t.max_period = max_period;
     t.max_repeats = max_repeats;
+    t.max_read_len = max_read_len;
     for (int k = 0; k < max_period * max_repeats; ++k) {
         if (!(gop_table[k] >= 0.0 && std::isfinite(gop_table[k]) && gcp_table[k] >= 0.0 && std::isfinite(gcp_table[k])))
             return fail(PAIRHMM_ERR_BAD_ARG, "tables must hold finite values >= 0");
@@ -1069,7 +1070,7 @@ extern "C" int32_t pairhmm_dragstr_impute_device(pairhmm_context *ctx, const dou
     if (!read_bases || !read_off || !read_len || !out_gop || !out_gcp)
         return fail(PAIRHMM_ERR_BAD_ARG, "null device pointer");
     HIP_TRY(hipSetDevice(ctx->device), PAIRHMM_ERR_KERNEL);
-    HIP_TRY(launch_dragstr_impute(read_bases, read_off, read_len, n_reads, max_read_len, t, out_gop, out_gcp, ctx->stream),
+    HIP_TRY(launch_dragstr_impute(read_bases, read_off, read_len, n_reads, t, out_gop, out_gcp, ctx->stream),
             PAIRHMM_ERR_KERNEL);
     HIP_TRY(hipStreamSynchronize(ctx->stream), PAIRHMM_ERR_KERNEL);
     return PAIRHMM_OK;

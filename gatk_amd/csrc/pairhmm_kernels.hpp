@@ -181,11 +181,12 @@ hipError_t launch_cap_qualities(const int64_t *read_off, const int32_t *read_len
 // capped as the imputer does, row-major [max_period][max_repeats].
 struct DragstrByteTables {
     int32_t max_period, max_repeats;
+    int32_t max_read_len;  // longest read the caller expects: sizes a wave's LDS
     uint8_t gop[512], gcp[512];
 };
 hipError_t launch_dragstr_impute(const uint8_t *bases, const int64_t *read_off, const int32_t *read_len,
-                                 int64_t n_reads, int max_read_len, const DragstrByteTables &tables, uint8_t *out_gop,
-                                 uint8_t *out_gcp, hipStream_t stream);
+                                 int64_t n_reads, const DragstrByteTables &tables, uint8_t *out_gop, uint8_t *out_gcp,
+                                 hipStream_t stream);
 int dragstr_max_read_length();
 
 // ---- partially determined PairHMM (pdhmm.hip) ----------------------------------------------
@@ -200,6 +201,10 @@ int dragstr_max_read_length();
 constexpr uint32_t kPdAltA = 8, kPdAltC = 16, kPdAltG = 32, kPdAltT = 64;
 constexpr uint32_t kPdDelEnd = 1u << 24, kPdInsideRow1 = 1u << 25, kPdInsideLater = 1u << 26;
 constexpr uint32_t kPdSpecial = 1u << 27;
+// Classes of read base the column accepts: A, C, G, T, a, c, g, t from kPdAcceptA on (its own base, every
+// class of an 'N' base, both cases of an alternative), and any other base.  Exact for haplotype bytes
+// ACGTacgtN; PdBatch::odd_bases says that some haplotype of the call holds another.
+constexpr uint32_t kPdAcceptA = 1u << 16, kPdAcceptOther = 1u << 28;
 
 // Every read against every haplotype; out[r * n_haps + h] (read-major).
 struct PdBatch {

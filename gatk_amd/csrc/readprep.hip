@@ -307,11 +307,11 @@ static_assert(dragstr_lds_bytes(kDragstrMaxRead) <= 65536, "a read's LDS fits th
 }  // namespace
 
 hipError_t launch_dragstr_impute(const uint8_t *bases, const int64_t *read_off, const int32_t *read_len,
-                                 int64_t n_reads, int max_read_len, const DragstrByteTables &tables, uint8_t *out_gop,
-                                 uint8_t *out_gcp, hipStream_t stream) {
+                                 int64_t n_reads, const DragstrByteTables &tables, uint8_t *out_gop, uint8_t *out_gcp,
+                                 hipStream_t stream) {
     if (n_reads <= 0) return hipSuccess;
     const int64_t grid = n_reads < 65536 ? n_reads : 65536;
-    const int longest = max_read_len < kDragstrMaxRead ? max_read_len : kDragstrMaxRead;
+    const int longest = tables.max_read_len < kDragstrMaxRead ? tables.max_read_len : kDragstrMaxRead;
     const int cap = (longest < 1 ? 1 : (longest + kWave - 1) / kWave) * kWave;
     hipLaunchKernelGGL(dragstr_impute_kernel, dim3(static_cast<unsigned>(grid)), dim3(kWave), dragstr_lds_bytes(cap), stream,
                        bases, read_off, read_len, n_reads, tables, cap, out_gop, out_gcp);
