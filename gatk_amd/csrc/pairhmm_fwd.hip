@@ -311,7 +311,7 @@ __device__ __forceinline__ void scale_mismatch(double (&a)[1], const double (&ra
         "v_mul_f64 %0, %0, %1\n\t"
         "s_mov_b64 exec, -1\n\t"
         "s_nop 2"
-        : "+v"(a[0])
+        : "+&v"(a[0])
         : "v"(ratio[0]), "v"(hb), "v"(base[0])
         : "vcc");
 }
@@ -324,7 +324,7 @@ __device__ __forceinline__ void scale_mismatch(double (&a)[2], const double (&ra
         "v_mul_f64 %1, %1, %3\n\t"
         "s_mov_b64 exec, -1\n\t"
         "s_nop 2"
-        : "+v"(a[0]), "+v"(a[1])
+        : "+&v"(a[0]), "+&v"(a[1])
         : "v"(ratio[0]), "v"(ratio[1]), "v"(hb), "v"(base[0]), "v"(base[1])
         : "vcc");
 }
@@ -343,7 +343,7 @@ __device__ __forceinline__ void scale_mismatch(double (&a)[4], const double (&ra
         "v_mul_f64 %3, %3, %7\n\t"
         "s_mov_b64 exec, -1\n\t"
         "s_nop 2"
-        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3])
+        : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3])
         : "v"(ratio[0]), "v"(ratio[1]), "v"(ratio[2]), "v"(ratio[3]), "v"(hb), "v"(base[0]), "v"(base[1]),
           "v"(base[2]), "v"(base[3])
         : "vcc");

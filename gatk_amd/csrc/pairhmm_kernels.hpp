@@ -216,6 +216,7 @@ struct PdBatch {
     const int32_t *rd_len;
     int32_t n_haps;
     int32_t tristate;
+    int32_t odd_bases;         // some haplotype byte lies outside ACGTacgtN
     double *out;
     const uint32_t *order;     // launch order of the pairs (longest first), or null
 };

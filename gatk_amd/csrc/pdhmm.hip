@@ -20,22 +20,40 @@
 // starts NORMAL and every later row starts in the state the previous row ended in, which is the
 // same for all rows >= 2.  The host folds this into each column's code (pd_column_codes).
 //
-// Mapping: one pair per wave, stripes of 64 rows, lane k owns row 64 s + k + 1 and at step t
-// computes column c = t - k + 1.  Each lane forms, from its new E values and the transitions of the
-// row below (the next lane's row; for lane 63 the next stripe's first row), the two sums that row
-// needs:
+// Mapping: one pair per wave.  A lane owns kRows = 2 consecutive rows (a stripe of 128; 1 row for a last
+// part of up to 64) and at step t computes column c = t - lane + 1 of all of them.  Each row forms, from its new E values and the transitions of the
+// row below, the two sums that row needs:
 //   A(r+1, c+1) = E_M(r,c) MM' + (E_I(r,c) + E_D(r,c)) GM'    (so M(r+1,c+1) = prior' A)
 //   B(r+1, c)   = E_M(r,c) MI' + E_I(r,c) II'                 (so I(r+1,c) = B)
-// and the row below takes A two steps later and B one step later by DPP wave_shr:1: two doubles
-// cross lanes per step instead of the three E values.  Lane 0 reads its A and B from an LDS record
-// per column that lane 63 of the previous stripe wrote (stripe 0 starts from row 0: M = I = 0,
-// D = 2^1020 / H, so A(1,c) = D GM_1 and B(1,c) = 0); every lane reads its own column's code from an
-// LDS array.  Records are 16 bytes (A, B) plus the 4-byte code, so a wave holds 20 bytes of LDS per
-// column.  Steps run in blocks of 4; a block in which no lane is on a special column (the host's
-// kPdSpecial: a deletion end, a column inside a span, or the column before a span) skips the branch
-// update and hands on E = X, which is exact because a row's branch values are only read on special
-// columns and the column before each span sets them from E.  The row-R lane sums M + I over
-// columns 1..H in column order, as the reference does (:132-139), in the last stripe only.
+// Along a lane the row below takes B at once and A at the next step; the next lane's first row takes A
+// two steps later and B one step later by DPP wave_shr:1, so two doubles cross lanes per step for
+// kRows cells.  Lane 0 takes them from a 16-byte LDS record per column, (B(c), A(c+1)): every lane
+// stores its last row's record at its own column (no one-lane branch in the step; lane 63 writes a
+// column last), and lane 0 reads a block's records at its start, before any lane of the stripe
+// stores to them (A of the block's first column was read with the block before).  Stripe 0 starts
+// from row 0: M = I = 0, D = 2^1020 / H, so A(1,c) = D GM_1 and B(1,c) = 0.  A wave holds 20 bytes of LDS
+// per column with the column's 4-byte code.
+//
+// Steps run in blocks of 4; a block in which no lane is on a special column (the host's kPdSpecial: a
+// deletion end, a column inside a span, or the column before a span) skips the branch update and
+// hands on E = X, which is exact because a row's branch values are only read on special columns and
+// the column before each span sets them from E.
+//
+// The result is the sum of M + I (not E) of row R over columns 1..H: rows past R pass the row above
+// down (M = D = 0, I = B with MI' = II' = 1), and from row R on B is formed from the plain M and I, so the
+// records end holding it.
+//
+// The prior of the fast path (as in the FP64 forward kernel): the match prior is folded into the
+// transitions that form A, a mismatch multiplies by px / pm in the lanes that have one, and M carries
+// the factor its next row in the lane would multiply it with.  A column's code holds one bit per class
+// of read base that it accepts, a row the bit of its base, so the match test is one AND.  Haplotype
+// bytes outside ACGTacgtN and qualities whose match prior or MM is near 0 take selected priors.
+//
+// Bound by VALU issue: 21 instructions per step of two cells, 47 in a block with a special column, at up
+// to 4 waves per SIMD (20 bytes of LDS per column hold longer haplotypes to less), where one row per
+// lane took 16 to 18 and 39 per cell.  One region of 81 reads (100-250 bases) and 65 haplotypes of 377,
+// kernel under the profiler: 306 us, against 437.  Four rows per lane take 255 VGPRs (two waves per
+// SIMD) and were slower: a region's pairs are few, and their tail weighs.
 #include "pairhmm_device.hpp"
 #include "pairhmm_kernels.hpp"
 
@@ -44,15 +62,16 @@ namespace {
 
 using namespace dev;
 
-// One column of a wave's LDS records: A and B of the stripe's first row (the row below lane 63 of
-// the stripe before).  The column codes are a separate uint32 array after the records.
+// One column of a wave's LDS records: B of this column and A of the next one for the stripe's first
+// row (the row below lane 63's last row of the stripe before).  The column codes are a separate uint32
+// array after the records.
 struct alignas(16) PdRecord {
-    double a, b;
+    double b, a;
 };
 static_assert(sizeof(PdRecord) == 16, "PdRecord is one 16-byte LDS word");
 
 constexpr int kPdPadColumns = 68;  // records past H that lane 0 reads (c <= H + 66 with 4-step blocks)
-constexpr int kPdLowPad = 64;      // records below column 0, where lane 63's stores of columns < 0 land
+constexpr int kPdLowPad = 64;      // records below column 0, where stores of columns < 0 land
 constexpr int kPdU = 4;            // wave-steps per unrolled block
 
 // Read-base class bit (placed like the column code's alternative mask) of isBasePDMatching
@@ -68,15 +87,30 @@ __device__ __forceinline__ uint32_t read_base_bit(uint32_t x) {
     }
 }
 
-// Row parameters of read position p (row p + 1); rows past the read are zero.
+// The bit of a read base among the classes a column accepts (kPdAccept*).
+__device__ __forceinline__ uint32_t accept_bit(uint32_t x) {
+    switch (x) {
+    case 'A': return kPdAcceptA;
+    case 'C': return kPdAcceptA << 1;
+    case 'G': return kPdAcceptA << 2;
+    case 'T': return kPdAcceptA << 3;
+    case 'a': return kPdAcceptA << 4;
+    case 'c': return kPdAcceptA << 5;
+    case 'g': return kPdAcceptA << 6;
+    case 't': return kPdAcceptA << 7;
+    default: return kPdAcceptOther;
+    }
+}
+
+// Row parameters of read position p (row p + 1); rows past the read are the pass-through row.
 struct PdRow {
     double MM, GM, MI, II, MD, DD, pm, px;
-    uint32_t x, xbit;
+    uint32_t x;
 };
 
 __device__ __forceinline__ PdRow pd_row(const PdBatch &b, const DeviceTables &tab, int64_t ro, int R, int p) {
-    PdRow w{0, 0, 0, 0, 0, 0, 0, 0, 0u, 0u};
-    if (p < 0 || p >= R) return w;
+    PdRow w{0, 0, 1, 1, 0, 0, 0, 0, 0u};
+    if (p >= R) return w;
     w.x = b.rd_bases[ro + p];
     const int q = b.rd_quals[ro + p], qi = b.rd_ins[ro + p], qd = b.rd_del[ro + p], qc = b.rd_gcp[ro + p];
     const int mn = qi < qd ? qi : qd, mx = qi < qd ? qd : qi;
@@ -90,68 +124,195 @@ __device__ __forceinline__ PdRow pd_row(const PdBatch &b, const DeviceTables &ta
     w.pm = 1.0 - eq;
     w.px = b.tristate ? eq / 3.0 : eq;
     if (w.x == 'N') w.px = w.pm;
-    w.xbit = read_base_bit(w.x);
     return w;
 }
 
-// Lane state of a stripe: own E and branch values at column c-1, the row-below sums of the last
-// two steps, the last-row sum.  The D values (ED, bD) are carried divided by the row's MD:
-// D(c) = E_D(c-1) DD + E_M(c-1) MD becomes D/MD = (E_D/MD) DD + E_M, one FMA, and max() commutes with
-// the positive scale (rows past R have MD = DD = 0 and stay 0).
-struct PdLane {
-    double EM = 0, EI = 0, ED = 0, bM = 0, bI = 0, bD = 0;
-    double an1 = 0, an2 = 0, bn1 = 0, acc = 0;
-};
+// Rows per lane of the stripe that starts with `left` rows to go.
+__device__ __forceinline__ int pd_stripe_rows(int left) { return left > kWave ? 2 : 1; }
 
-// One step of a lane at column c.  kBranch: the full branch update; without it E = X and the branch
-// values are left alone, which is exact on a block where no lane's column is special: a row's branch
-// values are only read at its special columns, and a deletion start (special) sets them from E.
-template <bool kLast, bool kBranch>
-__device__ __forceinline__ void pd_step(PdLane &st, const PdRecord &cur, uint32_t code, int c, int H, int R, int row,
-                                        const PdRow &w, const PdRow &wn, uint32_t inside_bit, bool writer,
-                                        PdRecord *wr) {
-    const double a = wave_shr1(cur.a, st.an2);  // lane 0 keeps its record's values
-    const double I = wave_shr1(cur.b, st.bn1);
-    const bool match = ((code & 0xFFu) == w.x) || (code & w.xbit) != 0u;
-    const double M = (match ? w.pm : w.px) * a;
-    const double D = fma(st.ED, w.DD, st.EM);  // D / MD
-    if constexpr (kBranch) {
-        const bool inside = (code & inside_bit) != 0u;
-        st.bM = inside ? st.bM : st.EM;
-        st.bI = inside ? st.bI : st.EI;
-        st.bD = inside ? st.bD : st.ED;
-        const double f = (code & kPdDelEnd) ? 1.0 : 0.0;  // max(0, X) == X for the cells here
-        st.EM = fmax(st.bM * f, M);
-        st.EI = fmax(st.bI * f, I);
-        st.ED = fmax(st.bD * f, D);
-    } else {
-        st.EM = M;
-        st.EI = I;
-        st.ED = D;
+// The factor folded into the sums that reach the row at read position p, the first of its lane in a
+// stripe of `rows` rows per lane (wave-uniform arguments; fast path).
+__device__ __forceinline__ double pd_first_fold(const PdBatch &b, const DeviceTables &tab, int64_t ro, int R, int p,
+                                                int rows) {
+    double f = 1.0;
+    for (int j = 0; j < rows && p + j < R; ++j) {
+        const PdRow w = pd_row(b, tab, ro, R, p + j);
+        f *= j == 0 ? w.pm : w.pm * w.MM;
     }
-    const double an = fma(fma(st.ED, w.MD, st.EI), wn.GM, st.EM * wn.MM);
-    const double bn = fma(st.EI, wn.II, st.EM * wn.MI);
-    st.an2 = st.an1;
-    st.an1 = an;
-    st.bn1 = bn;
-    if (writer) {  // (B(c), A(c + 1)) of the row below; c >= -62 (low pad)
-        wr->b = bn;
-        wr[1].a = an;
-    }
-    if (kLast && row == R && c >= 1 && c <= H) st.acc += M + I;
+    return f;
 }
 
-// Steps of one stripe, in blocks of kPdU; kLast adds the row-R lane's sum of M + I.  Lane 0's
-// records of a block are read at its start (lane 63 writes record j at step j + 61 or later); every
-// lane reads its own columns' codes (cds[c], zero for c < 1 and c > H).  A block runs the branch
-// update only if some lane's column in it is special.
-template <bool kLast>
-__device__ __forceinline__ double pd_stripe(PdRecord *rec, const uint32_t *cds, int lane, int H, int R, int row,
-                                            const PdRow &w, const PdRow &wn, uint32_t inside_bit) {
-    PdLane st;
-    const bool writer = lane == kWave - 1;
+// A lane's rows: own MD, DD and priors, the transitions of the row below each (n), and the state: E and
+// branch values at the column before, the row-below sums.  The D values (ED, bD) are carried divided by
+// the row's MD: D(c) = E_D(c-1) DD + E_M(c-1) MD becomes D/MD = (E_D/MD) DD + E_M, one FMA, and max()
+// commutes with the positive scale (rows past R have MD = DD = 0 and stay 0).  M's factor g scales EM, bM,
+// ED and bD alike.
+template <int kRows>
+struct PdLane {
+    double MD[kRows], DD[kRows], pm[kRows], px[kRows], MMn, GMn[kRows], MIn[kRows], IIn[kRows];
+    double MMr[kRows];             // generic path: every row's own factor of E_M in A
+    uint32_t bit[kRows], x[kRows]; // fast: accepted-class bit; generic: alternative bit and base
+    uint32_t inside0;              // the inside bit of the lane's first row
+    uint64_t inner[kRows];         // lanes whose row comes before row R
+    double EM[kRows], EI[kRows], ED[kRows], bM[kRows], bI[kRows], bD[kRows];
+    double an1[kRows], an2, bn1;
+};
+
+// Per row, in the lanes whose column does not accept the row's base (m == 0): a *= ratio.  EXEC is all
+// ones before and after (a workgroup is one whole wave in uniform control flow); the s_nop completes the
+// five wait states a DPP needs after a VALU write of EXEC, which the compiler does not track across
+// inline assembly.
+__device__ __forceinline__ void scale_unaccepted(double (&a)[1], const double (&ratio)[1], const uint32_t (&m)[1]) {
+    asm("v_cmpx_eq_u32_e32 vcc, 0, %2\n\t"
+        "v_mul_f64 %0, %0, %1\n\t"
+        "s_mov_b64 exec, -1\n\t"
+        "s_nop 2"
+        : "+&v"(a[0])
+        : "v"(ratio[0]), "v"(m[0])
+        : "vcc");
+}
+__device__ __forceinline__ void scale_unaccepted(double (&a)[2], const double (&ratio)[2], const uint32_t (&m)[2]) {
+    asm("v_cmpx_eq_u32_e32 vcc, 0, %4\n\t"
+        "v_mul_f64 %0, %0, %2\n\t"
+        "s_mov_b64 exec, -1\n\t"
+        "v_cmpx_eq_u32_e32 vcc, 0, %5\n\t"
+        "v_mul_f64 %1, %1, %3\n\t"
+        "s_mov_b64 exec, -1\n\t"
+        "s_nop 2"
+        : "+&v"(a[0]), "+&v"(a[1])
+        : "v"(ratio[0]), "v"(ratio[1]), "v"(m[0]), "v"(m[1])
+        : "vcc");
+}
+// The branch update's two masked parts (EXEC as above; SALU writes of it need no wait states).  Outside
+// a span the branch values follow the E values of the column before:
+__device__ __forceinline__ void pd_hold(double &bM, double &bI, double &bD, double EM, double EI, double ED,
+                                        uint64_t outside) {
+    asm("s_mov_b64 exec, %6\n\t"
+        "v_mov_b64_e32 %0, %3\n\t"
+        "v_mov_b64_e32 %1, %4\n\t"
+        "v_mov_b64_e32 %2, %5\n\t"
+        "s_mov_b64 exec, -1"
+        : "+&v"(bM), "+&v"(bI), "+&v"(bD)
+        : "v"(EM), "v"(EI), "v"(ED), "s"(outside));
+}
+// At a deletion's end E is max(b, X), and B of the row below is formed from it except from row R on.
+__device__ __forceinline__ void pd_merge(double &EM, double &EI, double &ED, double &bn, double bM, double bI, double bD,
+                                         double MIn, double IIn, uint64_t ends, uint64_t ends_inner) {
+    asm("s_mov_b64 exec, %9\n\t"
+        "v_max_f64 %0, %0, %4\n\t"
+        "v_max_f64 %1, %1, %5\n\t"
+        "v_max_f64 %2, %2, %6\n\t"
+        "s_mov_b64 exec, %10\n\t"
+        "v_mul_f64 %3, %0, %7\n\t"
+        "v_fma_f64 %3, %1, %8, %3\n\t"
+        "s_mov_b64 exec, -1"
+        : "+&v"(EM), "+&v"(EI), "+&v"(ED), "+&v"(bn)
+        : "v"(bM), "v"(bI), "v"(bD), "v"(MIn), "v"(IIn), "s"(ends), "s"(ends_inner));
+}
+
+// One step of a lane at its column.  kBranch: the full branch update; without it E = X and the branch
+// values are left alone, which is exact on a block where no lane's column is special: a row's branch
+// values are only read at its special columns, and a deletion start (special) sets them from E.
+template <int kRows, bool kBranch, bool kGeneric>
+__device__ __forceinline__ PdRecord pd_step(PdLane<kRows> &st, double a0, double b0, uint32_t code) {
+    double a[kRows];
+    double I = wave_shr1(b0, st.bn1);  // lane 0 keeps its record's values
+    a[0] = wave_shr1(a0, st.an2);
+#pragma unroll
+    for (int j = 1; j < kRows; ++j) a[j] = st.an1[j - 1];
+    st.an2 = st.an1[kRows - 1];
+    if constexpr (!kGeneric) {
+        uint32_t accepted[kRows];
+#pragma unroll
+        for (int j = 0; j < kRows; ++j) accepted[j] = code & st.bit[j];
+        scale_unaccepted(a, st.px, accepted);
+    }
+    uint64_t ends = 0;
+    if constexpr (kBranch) ends = __ballot((code & kPdDelEnd) != 0u);
+    PdRecord r{0, 0};
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) {
+        if constexpr (kGeneric)
+            a[j] *= ((code & 0xFFu) == st.x[j] || (code & st.bit[j]) != 0u) ? st.pm[j] : st.px[j];
+        if constexpr (kBranch)
+            pd_hold(st.bM[j], st.bI[j], st.bD[j], st.EM[j], st.EI[j], st.ED[j],
+                    __ballot((code & (j == 0 ? st.inside0 : kPdInsideLater)) == 0u));
+        st.ED[j] = fma(st.ED[j], st.DD[j], st.EM[j]);  // D / MD
+        st.EM[j] = a[j];
+        st.EI[j] = I;
+        r.b = fma(I, st.IIn[j], a[j] * st.MIn[j]);
+        if constexpr (kBranch)
+            pd_merge(st.EM[j], st.EI[j], st.ED[j], r.b, st.bM[j], st.bI[j], st.bD[j], st.MIn[j], st.IIn[j], ends,
+                     ends & st.inner[j]);
+        const double s = fma(st.ED[j], st.MD[j], st.EI[j]);
+        r.a = fma(s, st.GMn[j], kGeneric ? st.EM[j] * st.MMr[j] : j + 1 == kRows ? st.EM[j] * st.MMn : st.EM[j]);
+        st.an1[j] = r.a;
+        I = r.b;
+    }
+    st.bn1 = r.b;
+    return r;
+}
+
+// Two 8-byte stores, kept apart: merged they are a 16-byte store, whose data registers must not be
+// written within two instructions of it (check_isa.py).
+__device__ __forceinline__ void pd_store(PdRecord *r, const PdRecord &v) {
+    r->b = v.b;
+    asm volatile("" ::: "memory");
+    r->a = v.a;
+}
+
+// One stripe: rows of read positions p0 + kRows lane .. + kRows - 1.
+template <int kRows, bool kGeneric>
+__device__ __forceinline__ void pd_stripe(const PdBatch &b, const DeviceTables &tab, PdRecord *rec, const uint32_t *cds,
+                                          int lane, int H, int64_t ro, int R, int p0) {
+    PdLane<kRows> st;
+    {
+        PdRow w[kRows];
+        bool real[kRows];
+        double g[kRows];
+        const int p = p0 + kRows * lane;
+#pragma unroll
+        for (int j = 0; j < kRows; ++j) {
+            w[j] = pd_row(b, tab, ro, R, p + j);
+            real[j] = p + j < R;
+        }
+        g[kRows - 1] = 1.0;
+#pragma unroll
+        for (int j = kRows - 2; j >= 0; --j) g[j] = real[j + 1] ? w[j + 1].pm * w[j + 1].MM * g[j + 1] : 1.0;
+        const int p_next = p0 + kRows * kWave;
+        double fold = 1.0;
+        if constexpr (!kGeneric) {
+            fold = pd_first_fold(b, tab, ro, R, p_next, pd_stripe_rows(R - p_next));
+            fold = wave_shl1(fold, real[0] ? w[0].pm * g[0] : 1.0);
+        }
+        const PdRow below = pd_row(b, tab, ro, R, p + kRows);
+        st.inside0 = p == 0 ? kPdInsideRow1 : kPdInsideLater;
+#pragma unroll
+        for (int j = 0; j < kRows; ++j) {
+            const PdRow wn = j + 1 < kRows ? w[j + 1 < kRows ? j + 1 : 0] : below;
+            const double f = kGeneric ? 1.0 : j + 1 < kRows ? wn.pm * g[j + 1 < kRows ? j + 1 : 0] : fold;
+            const double inv_g = kGeneric || j + 1 == kRows ? 1.0 : 1.0 / g[j];
+            st.MMr[j] = wn.MM * f;
+            if (j + 1 == kRows) st.MMn = wn.MM * f;
+            st.GMn[j] = wn.GM * f;
+            st.MIn[j] = wn.MI * inv_g;
+            st.IIn[j] = wn.II;
+            st.MD[j] = w[j].MD * inv_g;
+            st.DD[j] = w[j].DD;
+            st.pm[j] = w[j].pm;
+            st.px[j] = kGeneric ? w[j].px : real[j] ? w[j].px / w[j].pm : 0.0;
+            // A pass-through row accepts nothing: M = 0.
+            st.bit[j] = !real[j] ? 0u : kGeneric ? read_base_bit(w[j].x) : accept_bit(w[j].x);
+            st.x[j] = real[j] ? w[j].x : 0x1FFu;
+            st.inner[j] = __ballot(p + j < R - 1);
+            st.EM[j] = st.EI[j] = st.ED[j] = st.bM[j] = st.bI[j] = st.bD[j] = st.an1[j] = 0.0;
+        }
+        st.an2 = st.bn1 = 0.0;
+    }
     const int steps = round_up(H + kWave - 1, kPdU);
     const uint32_t *cp = cds + 1 - lane;  // column t - lane + 1 at step t
+    PdRecord *wr = rec + 1 - lane;
+    double a_first = rec[0].a;  // A of the block's first column
     for (int t0 = 0; t0 < steps; t0 += kPdU) {
         PdRecord cur[kPdU];
         uint32_t cc[kPdU];
@@ -162,23 +323,44 @@ __device__ __forceinline__ double pd_stripe(PdRecord *rec, const uint32_t *cds, 
             cc[u] = cp[t0 + u];
             any |= cc[u];
         }
-        PdRecord *wr = rec + (t0 - (kWave - 2));  // lane 63's column at step t0 is t0 - 62
-        const int c0 = t0 - lane + 1;
+        __builtin_amdgcn_wave_barrier();
         if (__builtin_amdgcn_ballot_w64((any & kPdSpecial) != 0u) != 0) {
 #pragma unroll
             for (int u = 0; u < kPdU; ++u)
-                pd_step<kLast, true>(st, cur[u], cc[u], c0 + u, H, R, row, w, wn, inside_bit, writer, wr + u);
+                pd_store(wr + t0 + u, pd_step<kRows, true, kGeneric>(st, u == 0 ? a_first : cur[u - 1].a, cur[u].b, cc[u]));
         } else {
 #pragma unroll
             for (int u = 0; u < kPdU; ++u)
-                pd_step<kLast, false>(st, cur[u], cc[u], c0 + u, H, R, row, w, wn, inside_bit, writer, wr + u);
+                pd_store(wr + t0 + u, pd_step<kRows, false, kGeneric>(st, u == 0 ? a_first : cur[u - 1].a, cur[u].b, cc[u]));
         }
+        a_first = cur[kPdU - 1].a;
+        __builtin_amdgcn_wave_barrier();
     }
-    return st.acc;
 }
 
-__global__ __launch_bounds__(kWave) void pd_forward_kernel(PdBatch b, DeviceTables tab, uint32_t n_pairs,
-                                                            int rec_columns) {
+__device__ __forceinline__ void pd_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Every stripe of a pair; the records end holding M(R,c) + I(R,c) in b.
+template <bool kGeneric>
+__device__ __forceinline__ void pd_pair(const PdBatch &b, const DeviceTables &tab, PdRecord *rec, const uint32_t *cds,
+                                        int lane, int H, int64_t ro, int R) {
+    for (int p0 = 0; p0 < R;) {
+        const int rows = pd_stripe_rows(R - p0);
+        if (rows == 2)
+            pd_stripe<2, kGeneric>(b, tab, rec, cds, lane, H, ro, R, p0);
+        else
+            pd_stripe<1, kGeneric>(b, tab, rec, cds, lane, H, ro, R, p0);
+        p0 += rows * kWave;
+        pd_wave_sync();
+    }
+}
+
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4))) void pd_forward_kernel(
+    PdBatch b, DeviceTables tab, uint32_t n_pairs, int rec_columns) {
     extern __shared__ PdRecord lds_rec[];
     PdRecord *const rec = lds_rec + kPdLowPad;
     uint32_t *const cds = reinterpret_cast<uint32_t *>(rec + rec_columns) + kPdLowPad;
@@ -191,43 +373,34 @@ __global__ __launch_bounds__(kWave) void pd_forward_kernel(PdBatch b, DeviceTabl
         const int h = static_cast<int>(pair % static_cast<uint32_t>(b.n_haps));
         const int R = b.rd_len[r], H = b.hap_len[h];
         if (R == 0) {  // no rows: the final sum over row 0's M and I is 0
-            if (lane == 0) b.out[pair] = -__builtin_inf();
+            b.out[pair] = -__builtin_inf();
             continue;
         }
         const uint32_t *codes = b.hap_code + b.hap_off[h];
         const int64_t ro = b.rd_off[r];
         const double d0 = ldexp(1.0, Scale<double>::kExp) / static_cast<double>(H);
+        // Base quality 0 (pm = 0) and gap-open qualities under 4 (from there on MM >= 0.2) leave the fast
+        // path, which divides by both.
+        int low = 0;
+        for (int p = lane; p < R; p += kWave)
+            low |= b.rd_quals[ro + p] == 0 || b.rd_ins[ro + p] < 4 || b.rd_del[ro + p] < 4;
+        const bool generic = b.odd_bases || __any(low);
         // Row 1's sums over row 0 (M = I = 0, D = d0 on columns 0..H): A(c) = d0 GM_1 for 1 <= c <= H + 1.
-        const double gm1 = pd_row(b, tab, ro, R, 0).GM;
+        const double gm1 = pd_row(b, tab, ro, R, 0).GM * (generic ? 1.0 : pd_first_fold(b, tab, ro, R, 0, pd_stripe_rows(R)));
         __builtin_amdgcn_wave_barrier();
         for (int c = lane; c < H + kPdPadColumns && c < rec_columns; c += kWave) {
-            // Two 8-byte stores (volatile, so they are not merged into one 16-byte store).
-            volatile double *v = &rec[c].a;
-            v[0] = (c >= 1 && c <= H + 1) ? d0 * gm1 : 0.0;
-            v[1] = 0.0;
+            pd_store(rec + c, PdRecord{0.0, c <= H ? d0 * gm1 : 0.0});
             cds[c] = (c >= 1 && c <= H) ? codes[c - 1] : 0u;
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-        const int n_stripes = (R + kWave - 1) / kWave;
+        pd_wave_sync();
+        if (generic)
+            pd_pair<true>(b, tab, rec, cds, lane, H, ro, R);
+        else
+            pd_pair<false>(b, tab, rec, cds, lane, H, ro, R);
         double acc = 0.0;
-        for (int s = 0; s < n_stripes; ++s) {
-            const int row = s * kWave + lane + 1;
-            const PdRow w = pd_row(b, tab, ro, R, row - 1);
-            const PdRow wn = pd_row(b, tab, ro, R, row);
-            const uint32_t inside_bit = row == 1 ? kPdInsideRow1 : kPdInsideLater;
-            if (s == n_stripes - 1)
-                acc = pd_stripe<true>(rec, cds, lane, H, R, row, w, wn, inside_bit);
-            else
-                (void)pd_stripe<false>(rec, cds, lane, H, R, row, w, wn, inside_bit);
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
-        const double total = __shfl(acc, (R - 1) & (kWave - 1), kWave);
-        if (lane == 0) b.out[pair] = log10(total) - log10_init;
+        for (int c = 1 + lane; c <= H; c += kWave) acc += rec[c].b;
+        // Every lane holds the same sum and stores the same value.
+        b.out[pair] = log10(wave_sum(acc)) - log10_init;
         __builtin_amdgcn_wave_barrier();
     }
 }

@@ -41,18 +41,31 @@ PdState pd_state_pass(const uint8_t *pd, int H, PdState state, uint32_t inside_b
 // Column codes of one haplotype (layout in pairhmm_kernels.hpp).  Row 1 starts NORMAL; every later
 // row starts in the state the row before ended in (the state variable lives outside the row loop,
 // :63), which is the same state for all rows >= 2.
-void pd_column_codes(const uint8_t *bases, const uint8_t *pd, int H, uint32_t *code) {
+// Returns whether every base is one of ACGTacgtN.
+bool pd_column_codes(const uint8_t *bases, const uint8_t *pd, int H, uint32_t *code) {
+    // Per base: itself, an 'N's alternatives and the read-base classes it accepts; 0 for other bytes.
+    static const std::array<uint32_t, 256> of_base = [] {
+        std::array<uint32_t, 256> t{};
+        const char known[] = "ACGTacgt";
+        for (int k = 0; k < 8; ++k) t[static_cast<uint8_t>(known[k])] = static_cast<uint8_t>(known[k]) | (kPdAcceptA << k);
+        // An 'N' haplotype base matches every read base (:163).
+        t['N'] = 'N' | (0xF8u << 8) | (0xFFu * kPdAcceptA) | kPdAcceptOther;
+        return t;
+    }();
+    bool known = true;
     for (int j = 0; j < H; ++j) {
-        const uint32_t y = bases[j];
-        uint32_t alt = (pd[j] & kPdSnp) ? (pd[j] & kPdAltMask) : 0u;
-        if (y == 'N') alt |= 0xF8u;  // an 'N' haplotype base matches every read base (:163)
-        code[j] = y | (alt << 8) | ((pd[j] & kPdDelEndByte) ? kPdDelEnd : 0u);
+        const uint32_t y = bases[j], alt = (pd[j] & kPdSnp) ? (pd[j] & kPdAltMask) : 0u;
+        known = known && of_base[y] != 0u;
+        // Alternatives A, C, G, T are bits 3..6 of the PD byte and accept both cases.
+        code[j] = (of_base[y] ? of_base[y] : y) | (alt << 8) | ((alt >> 3) * 0x11u * kPdAcceptA) |
+                  ((pd[j] & kPdDelEndByte) ? kPdDelEnd : 0u);
     }
     const PdState end1 = pd_state_pass(pd, H, PdState::Normal, kPdInsideRow1, code);
     pd_state_pass(pd, H, end1, kPdInsideLater, code);
     constexpr uint32_t inside = kPdInsideRow1 | kPdInsideLater;
     for (int j = 0; j < H; ++j)
         if ((code[j] & (inside | kPdDelEnd)) || (j + 1 < H && (code[j + 1] & inside))) code[j] |= kPdSpecial;
+    return known;
 }
 
 bool is_pd_base(uint8_t x) {
@@ -152,10 +165,11 @@ extern "C" int32_t pairhmm_pd_compute_likelihoods(pairhmm_context *ctx, const pa
         pos += rd.length;
     }
     pos = 0;
+    bool known_bases = true;
     for (int32_t h = 0; h < n_haps; ++h) {
         hoff[h] = pos;
         hlen[h] = haps[h].length;
-        pd_column_codes(haps[h].haplotype_bases, haps[h].haplotype_pd_bases, haps[h].length, hcode + pos);
+        known_bases &= pd_column_codes(haps[h].haplotype_bases, haps[h].haplotype_pd_bases, haps[h].length, hcode + pos);
         pos += haps[h].length;
     }
     // Workgroups are dispatched in order: longest reads first, and each read's haplotypes longest
@@ -186,6 +200,7 @@ extern "C" int32_t pairhmm_pd_compute_likelihoods(pairhmm_context *ctx, const pa
     b.rd_len = reinterpret_cast<const int32_t *>(ds + o_rlen);
     b.n_haps = n_haps;
     b.tristate = 1;
+    b.odd_bases = known_bases ? 0 : 1;
     b.out = reinterpret_cast<double *>(ds + o_out);
     DeviceTables tab{ctx->d_qual_err, ctx->d_mm_prob};
     // One wave per workgroup and per pair; the hardware dispatcher balances uneven pairs.

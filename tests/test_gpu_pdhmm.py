@@ -227,3 +227,43 @@ def test_vector_pd_hmm_mask_and_results_file():
         want = oracle.pd_logless(h, p, rd.read_bases, rd.read_quals, rd.insertion_gop, rd.deletion_gop,
                                  rd.overall_gcp)
         assert abs(val - want) <= 5e-7 * max(1.0, abs(want))  # %e keeps 7 significant digits
+
+
+@pytest.mark.parametrize("case", ["plain", "base_quality_0", "low_gap_open", "odd_hap_base", "lower_case", "read_n"])
+def test_stripe_row_counts_and_generic_inputs(case):
+    """Reads that end where the stripes change between 2 and 1 rows per lane (64, 128, 192, ... rows to go),
+    with deletion spans on the haplotypes' first and last columns, and the inputs that leave the kernel's
+    fast path (base quality 0, gap-open qualities under 4, haplotype bytes outside ACGTacgtN) or meet its
+    accepted-class bits (lower-case bases, 'N' reads and haplotypes)."""
+    rng = np.random.default_rng(77)
+    haps = [_pd_haplotype(rng, 40, 3, 2), _pd_haplotype(rng, 260, 6, 4, n_bases=2)]
+    edge = bytearray(200)
+    edge[0] |= DEL_START
+    edge[2] |= DEL_END
+    edge[-3] |= DEL_START
+    edge[-1] |= DEL_END
+    haps.append((_rand_seq(rng, 200), bytes(edge)))
+    if case == "odd_hap_base":
+        h, p = bytearray(haps[1][0]), bytearray(haps[1][1])
+        for j in (5, 100, 200):
+            h[j], p[j] = ord("R"), p[j] & ~(SNP | A | C | G | T) & 0xFF
+        haps[1] = (bytes(h), bytes(p))
+    if case == "lower_case":
+        haps[2] = (haps[2][0][:90].lower() + haps[2][0][90:], haps[2][1])
+    reads = []
+    for R in (1, 2, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257, 320):
+        rd = list(_read(rng, R, haps[1][0] if R <= 260 else None))
+        at = rng.integers(0, R, 2)
+        if case == "base_quality_0":
+            rd[1][at] = 0
+        elif case == "low_gap_open":
+            rd[2][at] = rng.integers(0, 4, 2)
+            rd[3][at[::-1]] = rng.integers(0, 4, 2)
+        elif case == "lower_case":
+            rd[0][: R // 2] = np.frombuffer(rd[0][: R // 2].tobytes().lower(), np.uint8)
+        elif case == "read_n":
+            rd[0][at] = ord("N")
+        for byte, by in (("R", "A"), ("n", "N")):  # the reference refuses other read bases on SNP columns
+            rd[0][rd[0] == ord(byte)] = ord(by)
+        reads.append(tuple(rd))
+    _check(reads, haps, f"row counts, {case}")
