@@ -31,6 +31,8 @@
 //     flag pairs whose scaled sum is below the underflow threshold for an FP64 recompute (S = 1020).
 //   * Launches are per LDS column class (kColClasses): a wave's LDS slice holds the haplotype and
 //     the planes for the class's longest haplotype, so short haplotypes get more waves per CU.
+#include <algorithm>
+
 #include "pairhmm_device.hpp"
 #include "pairhmm_kernels.hpp"
 
@@ -622,12 +624,17 @@ void forward_kernel(DeviceBatch b, DeviceTables tab, WorkSource ws, RescueSink r
     const WaveLds<T> L = carve<T, kCols>(lds_raw + kPerWave * wave, b, gwave);
     const uint32_t n_items = ws.n_items_dev ? *ws.n_items_dev : ws.n_items;
     if (ws.head) {
-        for (;;) {
-            // All lanes issue the atomic (lane 0 adds 1, the rest add 0), so the fetch has no
-            // lane-divergent branch; lane 0's pre-increment value is the wave's item.
-            const uint32_t it = __builtin_amdgcn_readfirstlane(atomicAdd(ws.head, lane == 0 ? 1u : 0u));
-            if (it >= n_items) break;
+        // A wave's first item is the one of its own number; the next ones come from the queue head.  So
+        // surplus waves of a rescue pass leave without touching the head (one address for the whole GPU,
+        // about 14 ns an atomic: 60 us for a launch's 4,096 waves, whatever the rescued pairs).
+        const uint32_t waves = std::min<uint32_t>(
+            gridDim.x * waves_per_block, sizeof(T) == sizeof(double) ? b.f64_plane_waves : 0xFFFFFFFFu);
+        for (uint32_t it = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(gwave)); it < n_items;) {
             process_pair<T, kCols>(b, tab, rs, L, lane, ws.items ? ws.items[it] : it);
+            if (n_items <= waves) break;
+            // All lanes issue the atomic (lane 0 adds 1, the rest add 0), so the fetch has no
+            // lane-divergent branch; lane 0's pre-increment value is the wave's next item.
+            it = waves + __builtin_amdgcn_readfirstlane(atomicAdd(ws.head, lane == 0 ? 1u : 0u));
         }
     } else {
         // The wave's index is wave-uniform; readfirstlane tells the compiler so, which keeps the
@@ -704,6 +711,8 @@ constexpr uint32_t kPackedChunk = 16;
 
 struct ChunkCursor {
     uint32_t next = 0, end = 0;  // items [next, end) of the wave's current chunk
+    uint32_t wave = 0, waves = 0;  // this wave's number in the launch, and their count
+    bool first = true;             // the wave's first chunk is the one of its own number
 };
 
 // Takes the next pair of the wave's current chunk; with new_chunk, first takes a new chunk when the
@@ -714,8 +723,12 @@ __device__ bool packed_fetch(const DeviceBatch &b, const WorkSource &ws, uint32_
     for (;;) {
         if (cc.next >= cc.end) {
             if (!new_chunk) return false;
-            // All lanes issue the atomic (lane 0 adds 1): the fetch has no lane-divergent branch.
-            const uint32_t c = __builtin_amdgcn_readfirstlane(atomicAdd(ws.head, lane == 0 ? 1u : 0u));
+            // All lanes issue the atomic (lane 0 adds 1): the fetch has no lane-divergent branch.  A wave's
+            // first chunk needs none: thousands of waves starting on one address take about 14 ns each.
+            const uint32_t c = cc.first
+                                   ? cc.wave
+                                   : cc.waves + __builtin_amdgcn_readfirstlane(atomicAdd(ws.head, lane == 0 ? 1u : 0u));
+            cc.first = false;
             const uint64_t first = static_cast<uint64_t>(c) * ws.chunk;
             if (first >= n_items) return false;
             cc.next = static_cast<uint32_t>(first);
@@ -885,8 +898,10 @@ __device__ __forceinline__ float packed_steps(const WaveLds<float> &L, const uin
 // loop body.
 template <int kCols, int kU>
 __device__ void packed_wave(const DeviceBatch &b, const DeviceTables &tab, const WorkSource &ws, uint32_t n_items,
-                            const RescueSink &rs, uint8_t *lds, int lane) {
+                            const RescueSink &rs, uint8_t *lds, int lane, uint32_t gwave, uint32_t waves) {
     ChunkCursor cc;
+    cc.wave = gwave;
+    cc.waves = waves;
     WaveLds<float> L;
     // Haplotype buffer k at lds + kHapGuard + k kCols (chosen by arithmetic, not by indexing an array
     // of pointers, so the compiler keeps them LDS pointers).
@@ -985,7 +1000,10 @@ __global__ __launch_bounds__(512) void forward_kernel_packed(DeviceBatch b, Devi
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
     const uint32_t n_items = ws.n_items_dev ? *ws.n_items_dev : ws.n_items;
-    packed_wave<kCols, kU>(b, tab, ws, n_items, rs, lds_raw + packed_lds_per_wave<kCols>() * wave, lane);
+    const uint32_t waves_per_block = blockDim.x / kWave;
+    packed_wave<kCols, kU>(b, tab, ws, n_items, rs, lds_raw + packed_lds_per_wave<kCols>() * wave, lane,
+                           __builtin_amdgcn_readfirstlane(blockIdx.x * waves_per_block + wave),
+                           gridDim.x * waves_per_block);
 }
 
 __global__ void zero_counters_kernel(uint32_t *c, int n) {

@@ -371,10 +371,9 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kLong ? 3
     SwScore *recs = lds_sw;
     uint8_t *lref = reinterpret_cast<uint8_t *>(lds_sw + (kLong ? kSwLow + b.max_ref_len + kSwHigh : 0));
     uint32_t *bt = reinterpret_cast<uint32_t *>(b.scratch + static_cast<size_t>(blockIdx.x) * b.scratch_per_wave);
-    for (;;) {
-        // All lanes issue the atomic (lane 0 adds 1): the fetch has no lane-divergent branch.
-        const uint32_t p = __builtin_amdgcn_readfirstlane(atomicAdd(b.queue_head, lane == 0 ? 1u : 0u));
-        if (p >= n_pairs) break;
+    // The first pair is the one of the wave's own number, the next ones come from the queue head (an atomic
+    // on one address, about 14 ns each).
+    for (uint32_t p = blockIdx.x; p < n_pairs;) {
         const int R = __builtin_amdgcn_readfirstlane(b.ref_len[p]), A = __builtin_amdgcn_readfirstlane(b.alt_len[p]);
         const uint8_t *ref = b.ref_bases + b.ref_off[p];
         __builtin_amdgcn_wave_barrier();
@@ -398,6 +397,9 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kLong ? 3
         else
             sw_pair<1, false>(b, lref, recs, bt, p, lane, R, A);
         __builtin_amdgcn_wave_barrier();
+        if (n_pairs <= gridDim.x) break;
+        // All lanes issue the atomic (lane 0 adds 1): the fetch has no lane-divergent branch.
+        p = gridDim.x + __builtin_amdgcn_readfirstlane(atomicAdd(b.queue_head, lane == 0 ? 1u : 0u));
     }
 }
 
