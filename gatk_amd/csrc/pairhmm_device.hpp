@@ -108,17 +108,19 @@ __device__ __forceinline__ double rfl(double x) {
 // Lanes 1..63: a = a0(lane k-1) * ma0 + a1(lane k-1) * ma1 and b = b0(lane k-1) * mb0 + b1(lane k-1) * mb1.
 // Lane 0 keeps the a and b it brings in: a DPP wave_shr:1 without bound_ctrl leaves a lane whose
 // source lies outside the wave unwritten.  Four VALU instructions, the lane exchange included; the
-// leading s_nop 4 provides the DPP wait states the compiler does not track across inline assembly
-// (2 after a VALU write of a DPP source, 5 after an EXEC write).
+// leading s_nop provides the DPP wait states the compiler does not track across inline assembly: kNop = 4
+// for 5, which also covers a VALU write of EXEC just before; kNop = 1 for the 2 after a VALU write of a DPP
+// source, where no VALU instruction nearby writes EXEC.
+template <int kNop = 4>
 __device__ __forceinline__ void dpp_upper2(float &a, float a0, float ma0, float a1, float ma1, float &b, float b0,
                                            float mb0, float b1, float mb1) {
-    asm("s_nop 4\n\t"
+    asm("s_nop %10\n\t"
         "v_mul_f32_dpp %0, %2, %3 wave_shr:1 row_mask:0xf bank_mask:0xf\n\t"
         "v_mul_f32_dpp %1, %6, %7 wave_shr:1 row_mask:0xf bank_mask:0xf\n\t"
         "v_fmac_f32_dpp %0, %4, %5 wave_shr:1 row_mask:0xf bank_mask:0xf\n\t"
         "v_fmac_f32_dpp %1, %8, %9 wave_shr:1 row_mask:0xf bank_mask:0xf"
         : "+&v"(a), "+&v"(b)
-        : "v"(a0), "v"(ma0), "v"(a1), "v"(ma1), "v"(b0), "v"(mb0), "v"(b1), "v"(mb1));
+        : "v"(a0), "v"(ma0), "v"(a1), "v"(ma1), "v"(b0), "v"(mb0), "v"(b1), "v"(mb1), "n"(kNop));
 }
 
 // a^k for 0 <= k < 128 by repeated squaring (exact to a few ulp, unlike exp2(k log2 a)).

@@ -145,24 +145,36 @@ __device__ __forceinline__ WaveLds<T> carve(uint8_t *base, const DeviceBatch &b,
 // on still hold what earlier passes left there and are read as M = I = 0.  Leftovers past a
 // shorter stripe's end, turned over again by every later pass, can grow to inf, and a summing row
 // that meets inf beyond its haplotype (times its prior 0) turns NaN.
-template <int kCols>
-__device__ __forceinline__ void side_pass_f32(float *P0, float *P1, int lane, float MM0, float GM0, float MI0,
-                                              float II0, float MDr, float DDr, int jmax, float cd0 = 0.f,
-                                              int wend = kCols) {
-    const float a1 = DDr, a2 = a1 * a1, a4 = a2 * a2, a8 = a4 * a4, a16 = a8 * a8, a32 = a16 * a16;
-    // DD'^((l mod 16) + 1) by the bits of l mod 16, then the row's 16-lane steps on top:
-    // p_in = DD'^(l+1), p_31 = DD'^(l-31) for l >= 32 (1 below).
-    float p_row = a1;
-    p_row = (lane & 1) ? p_row * a1 : p_row;
-    p_row = (lane & 2) ? p_row * a2 : p_row;
-    p_row = (lane & 4) ? p_row * a4 : p_row;
-    p_row = (lane & 8) ? p_row * a8 : p_row;
-    const float p_16 = (lane & 16) ? p_row * a16 : p_row;
-    const float p_in = (lane & 32) ? p_16 * a32 : p_16;
-    const float p_31 = (lane & 32) ? p_16 : 1.f;
-    float cm = 0.f, ci = 0.f, cd = cd0;  // M, I, D of column j0 - 1
-    __builtin_amdgcn_wave_barrier();
-    for (int j0 = 0; j0 < jmax; j0 += kWave) {
+//
+// SidePass holds what goes from chunk to chunk, so a wave that works on a row while another still
+// computes it (forward_kernel_split) can take the chunks one at a time.
+struct SidePass {
+    float MM0, GM0, MI0, II0, MDr;
+    float a1, a2, a4, a8, p_row, p_in, p_31;
+    float cm = 0.f, ci = 0.f, cd;  // M, I, D of column j0 - 1
+
+    __device__ __forceinline__ SidePass(int lane, float MM0, float GM0, float MI0, float II0, float MDr, float DDr,
+                                        float cd0)
+        : MM0(MM0), GM0(GM0), MI0(MI0), II0(II0), MDr(MDr), cd(cd0) {
+        a1 = DDr;
+        a2 = a1 * a1;
+        a4 = a2 * a2;
+        a8 = a4 * a4;
+        const float a16 = a8 * a8, a32 = a16 * a16;
+        // DD'^((l mod 16) + 1) by the bits of l mod 16, then the row's 16-lane steps on top:
+        // p_in = DD'^(l+1), p_31 = DD'^(l-31) for l >= 32 (1 below).
+        p_row = a1;
+        p_row = (lane & 1) ? p_row * a1 : p_row;
+        p_row = (lane & 2) ? p_row * a2 : p_row;
+        p_row = (lane & 4) ? p_row * a4 : p_row;
+        p_row = (lane & 8) ? p_row * a8 : p_row;
+        const float p_16 = (lane & 16) ? p_row * a16 : p_row;
+        p_in = (lane & 32) ? p_16 * a32 : p_16;
+        p_31 = (lane & 32) ? p_16 : 1.f;
+    }
+
+    // Chunk of slots j0 .. j0 + 63.
+    __device__ __forceinline__ void chunk(float *P0, float *P1, int lane, int j0, int wend) {
         const int j = j0 + lane;
         const bool written = j >= kLdsPad - (kWave - 1) && j < wend;
         const float mj = written ? P0[j] : 0.f, ij = written ? P1[j] : 0.f;
@@ -177,6 +189,15 @@ __device__ __forceinline__ void side_pass_f32(float *P0, float *P1, int lane, fl
         cd = lane63(dj);
         __builtin_amdgcn_wave_barrier();
     }
+};
+
+template <int kCols>
+__device__ __forceinline__ void side_pass_f32(float *P0, float *P1, int lane, float MM0, float GM0, float MI0,
+                                              float II0, float MDr, float DDr, int jmax, float cd0 = 0.f,
+                                              int wend = kCols) {
+    SidePass side(lane, MM0, GM0, MI0, II0, MDr, DDr, cd0);
+    __builtin_amdgcn_wave_barrier();
+    for (int j0 = 0; j0 < jmax; j0 += kWave) side.chunk(P0, P1, lane, j0, wend);
 }
 
 // One pass over a pair, stripe by stripe.  Returns the scaled last-row sum (FP64, every lane).
@@ -838,16 +859,48 @@ __device__ __forceinline__ PackedRow packed_row(int kind, int idx, const PackedP
     return x;
 }
 
-// One stripe of steps (the aligned schedule's step, per-lane haplotype pointers and 'N' bytes).
-// Returns the lane's D' after the last step (a SUM row's last-row sum).
+// A lane's cell one step back (1) and two steps back (2); d1 is D' = D / MD.
+struct PackedState {
+    float m1, i1, d1, s1, m2, s2;
+};
+
+__device__ __forceinline__ PackedState packed_start(const PackedRow &x) {
+    return PackedState{x.m1, 0.f, x.d1, x.s1, 0.f, x.s2};
+}
+
+// kU steps (the aligned schedule's step, per-lane haplotype bytes and 'N' bytes): lane 0's sums in av, bv,
+// the lanes' haplotype bytes in hbs, M and I to wm, wi.  kNop: wait states before the DPP products.
+template <bool kHapHasN, int kU, int kNop>
+__device__ __forceinline__ void packed_block(PackedState &st, const RowTrans<float> &w, uint32_t nval,
+                                             const float (&av)[kU], const float (&bv)[kU], const uint32_t (&hbs)[kU],
+                                             __attribute__((address_space(3))) float *wm,
+                                             __attribute__((address_space(3))) float *wi) {
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+        const uint32_t hb = hbs[u];
+        const bool match = (hb == w.base) || (kHapHasN && hb == nval);
+        const float prior = match ? w.pm : w.px;
+        float a = av[u], i = bv[u];
+        dpp_upper2<kNop>(a, st.m2, w.MM, st.s2, w.GM, i, st.m1, w.MI, st.i1, w.II);
+        const float m = a * prior;
+        const float d = fmaf(st.d1, w.DD, st.m1);
+        const float sx = fmaf(w.MD, d, i);
+        wm[u] = m;
+        wi[u] = i;
+        st.m2 = st.m1;
+        st.s2 = st.s1;
+        st.m1 = m;
+        st.i1 = i;
+        st.d1 = d;
+        st.s1 = sx;
+    }
+}
+
+// One stripe of steps.  Returns the lane's D' after the last step (a SUM row's last-row sum).
 template <int kCols, bool kHapHasN, int kU>
 __device__ __forceinline__ float packed_steps(const WaveLds<float> &L, const uint8_t *hap, int lane,
                                               const PackedRow &x, int steps) {
-    const float MM = x.w.MM, GM = x.w.GM, MI = x.w.MI, II = x.w.II, MD = x.w.MD, DD = x.w.DD, pm = x.w.pm,
-                px = x.w.px;
-    const uint32_t base = x.w.base, nval = x.nval;
-    float m1 = x.m1, i1 = 0.f, d1 = x.d1, s1 = x.s1;
-    float m2 = 0.f, s2 = x.s2;
+    PackedState st = packed_start(x);
     using lds_u8 = const volatile __attribute__((address_space(3))) uint8_t;
     lds_u8 *hp = (lds_u8 *)(hap + kLdsPad - 1 - lane + x.shift);  // address-space cast: C-style only
     // Every lane stores its M and I at its own column c = t - lane at step t, so the step has no
@@ -862,7 +915,6 @@ __device__ __forceinline__ float packed_steps(const WaveLds<float> &L, const uin
     // there makes every LDS wait in the loop a full lgkmcnt(0) instead of waiting for the first reads.
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
     for (int t0 = 0; t0 < steps; t0 += kU) {
-        lds_f32 *wmb = wm + t0, *wib = wi + t0;
         float av[kU], bv[kU];
         __builtin_memcpy(av, __builtin_assume_aligned(L.bm + kLdsPad + t0, 16), sizeof(av));
         __builtin_memcpy(bv, __builtin_assume_aligned(L.bi + kLdsPad + t0, 16), sizeof(bv));
@@ -870,28 +922,10 @@ __device__ __forceinline__ float packed_steps(const WaveLds<float> &L, const uin
 #pragma unroll
         for (int u = 0; u < kU; ++u) hbs[u] = hp[t0 + u];
         __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            const uint32_t hb = hbs[u];
-            const bool match = (hb == base) || (kHapHasN && hb == nval);
-            const float prior = match ? pm : px;
-            float a = av[u], i = bv[u];
-            dpp_upper2(a, m2, MM, s2, GM, i, m1, MI, i1, II);
-            const float m = a * prior;
-            const float d = fmaf(d1, DD, m1);
-            const float sx = fmaf(MD, d, i);
-            wmb[u] = m;
-            wib[u] = i;
-            m2 = m1;
-            s2 = s1;
-            m1 = m;
-            i1 = i;
-            d1 = d;
-            s1 = sx;
-        }
+        packed_block<kHapHasN, kU, 4>(st, x.w, x.nval, av, bv, hbs, wm + t0, wi + t0);
     }
     __builtin_amdgcn_wave_barrier();
-    return d1;
+    return st.d1;
 }
 
 // The packed-stripe FP32 pass of one wave over its share of a queue, kU wave-steps per unrolled
@@ -1006,6 +1040,249 @@ __global__ __launch_bounds__(512) void forward_kernel_packed(DeviceBatch b, Devi
                            gridDim.x * waves_per_block);
 }
 
+// ---- split stripes (FP32) ---------------------------------------------------------------------
+//
+// A small queue (one region's pairs) gives a packed wave one pair (ws.chunk = 1), whose stripes it then
+// computes one after another: the launch lasts as long as the longest pair's stripes in a row on a SIMD
+// that got five of them, and with fewer pairs than SIMDs most of the GPU waits for single waves.  Here
+// a workgroup of four waves works through pairs together, the unit of work being a stripe: the stripes of
+// the group's pairs, in order, go to its waves in turn.  The wave of stripe s + 1 follows the wave of
+// stripe s at the distance at which lane 63 has finished a 64-column chunk, runs the side pass over that
+// chunk and then 64 steps.  Stripes, rows and the operations on every cell are those of a packed wave
+// with a chunk of one pair, so results are the same bit for bit.
+//
+// The stripes of a pair share one pair of LDS planes: along the columns, from right to left, lie the
+// columns stripe s is writing, its finished row, the same row as stripe s + 1's sums A and B, the columns
+// stripe s + 1 is writing, and so on; no stripe passes the one before it.  A group holds kSlots pairs.
+// Every wait is for work that does not depend on the waiting wave, by waves of the same workgroup, which
+// are resident together: a stripe for the stripe before it, a reader of a pair's record for the wave that
+// takes its first stripe, and that wave, to reuse a slot, for all waves to have gone past the slot's pair
+// (so its stripes are done and its record is read).  A wave's LDS operations complete in the order they
+// are issued, so a word published after its data needs no further wait.
+//
+// Bound by the latency of a pair's stripes in small queues (about 100 cycles a step for a lone wave: LDS
+// round trips, dependent products) and by VALU issue in large ones.  8 steps per block (81 VGPRs, 20 waves
+// per CU) against 16 (105, 16 waves): 288 and 303 us at 5,265 pairs, equal at 1,024.
+constexpr int kSplitWaves = 4;
+constexpr int kSplitStepBits = 20;       // a stripe's progress is published as stripe << 20 | steps done
+constexpr uint32_t kSplitEnd = 0xFFFFFFFFu;  // n_stripes of the record that ends the queue
+
+using lds_u32 = volatile __attribute__((address_space(3))) uint32_t;
+
+// A pair's record, after its haplotype and planes.
+struct SplitRecord {
+    uint32_t seq;  // pair number + 1 once the record is valid
+    uint32_t n_stripes, pair, R, H, ro_lo, ro_hi, hap_n;
+    uint32_t done[kSplitWaves];  // progress of the latest stripe s with s mod 4 = k
+};
+
+template <int kCols>
+constexpr size_t split_slot_bytes() {
+    return kHapGuard + static_cast<size_t>(kCols) + kPlanes * static_cast<size_t>(plane_stride<kCols>()) * sizeof(float) +
+           sizeof(SplitRecord);
+}
+// Slots per group: four, or two where the longer haplotypes' planes would leave a CU less than its share
+// of groups.
+template <int kCols>
+constexpr int split_slots() { return kCols <= 1024 ? 4 : 2; }
+template <int kCols>
+constexpr size_t split_lds_bytes() { return split_slots<kCols>() * split_slot_bytes<kCols>() + kSplitWaves * sizeof(uint32_t); }
+
+__device__ __forceinline__ uint32_t lds_get(lds_u32 *p) {
+    return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(*p)));
+}
+
+// Stages a haplotype as packed_stage does, one wave, four bases a load.  Returns whether it has an 'N'.
+template <int kCols>
+__device__ __forceinline__ bool split_stage(const uint8_t *hap, int H, uint8_t *hbuf, int lane) {
+    using lds_w32 = __attribute__((address_space(3))) uint32_t;
+    using lds_w8 = __attribute__((address_space(3))) uint8_t;
+    lds_w32 *w = (lds_w32 *)hbuf;  // address-space casts: C-style only
+    for (int k = lane; k < kCols / 4; k += kWave) w[k] = 0u;
+    __builtin_amdgcn_wave_barrier();
+    int has_n = 0;
+    for (int c = 4 * lane; c < H; c += 4 * kWave) {
+        if (c + 4 <= H) {
+            uint32_t v;
+            __builtin_memcpy(&v, hap + c, 4);
+            w[kLdsPad / 4 + c / 4] = v;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) has_n |= ((v >> (8 * k)) & 0xFFu) == 'N';
+        } else {
+            for (int k = c; k < H; ++k) {
+                ((lds_w8 *)hbuf)[kLdsPad + k] = hap[k];
+                has_n |= hap[k] == 'N';
+            }
+        }
+    }
+    if (lane == 0) ((lds_w8 *)hbuf)[kLdsPad - 2] = kZeroRowMark;  // column -1
+    return __any(has_n);
+}
+
+// One stripe on one wave.  Returns the lane's D' after the last step.
+template <int kCols, bool kHapHasN, int kU>
+__device__ __forceinline__ float split_stripe(const DeviceBatch &b, const DeviceTables &tab, const PackedPair &p,
+                                              const WaveLds<float> &L, lds_u32 *done, int lane, int s) {
+    const int idx = s * kWave + lane;
+    const int kind = idx == 0 ? kRowConst : idx == 1 ? kRowZero : idx == p.R + 2 ? kRowSum : idx < p.R + 2 ? kRowRead : kRowIdle;
+    const PackedRow x = packed_row(kind, idx, p, b, tab, lane);
+    // Lane 63's row of the stripe before (a read row), wave-uniform.
+    const PackedRow up = packed_row(s > 0 ? kRowRead : kRowIdle, s * kWave - 1, p, b, tab, lane);
+    SidePass side(lane, rfl(x.w.MM), rfl(x.w.GM), rfl(x.w.MI), rfl(x.w.II), up.w.MD, up.w.DD, 0.f);
+    const int steps = __builtin_amdgcn_readfirstlane(round_up(p.H + kWave + 2, kU));
+    const int wend = kLdsPad - (kWave - 1) + steps;
+    const int jmax = plane_span<kCols>(steps);
+    PackedState st = packed_start(x);
+    using lds_u8 = const volatile __attribute__((address_space(3))) uint8_t;
+    lds_u8 *hp = (lds_u8 *)(L.hap + kLdsPad - 1 - lane + x.shift);  // address-space cast: C-style only
+    using lds_f32 = __attribute__((address_space(3))) float;
+    int lane_w = lane;
+    asm volatile("" : "+v"(lane_w));
+    lds_f32 *wm = (lds_f32 *)(L.bm + kLdsPad) - lane_w, *wi = (lds_f32 *)(L.bi + kLdsPad) - lane_w;
+    const uint32_t before = static_cast<uint32_t>(s - 1) << kSplitStepBits;
+    auto follow = [&](int need) {  // until the stripe before has done `need` steps
+        const uint32_t want = before + static_cast<uint32_t>(need < steps ? need : steps);
+        while (lds_get(done + (s - 1) % kSplitWaves) < want) __builtin_amdgcn_s_sleep(1);
+        asm volatile("" ::: "memory");
+    };
+    if (s > 0) {
+        follow(kWave);
+        side.chunk(L.bm, L.bi, lane, 0, wend);
+    }
+    for (int t1 = 0; t1 < steps; t1 += kWave) {
+        if (s > 0 && t1 + kWave < jmax) {
+            follow(t1 + 2 * kWave - 1);
+            side.chunk(L.bm, L.bi, lane, t1 + kWave, wend);
+        }
+        const int end = t1 + kWave < steps ? t1 + kWave : steps;
+        for (int t0 = t1; t0 < end; t0 += kU) {
+            float av[kU], bv[kU];
+            if (s > 0) {
+                __builtin_memcpy(av, __builtin_assume_aligned(L.bm + kLdsPad + t0, 16), sizeof(av));
+                __builtin_memcpy(bv, __builtin_assume_aligned(L.bi + kLdsPad + t0, 16), sizeof(bv));
+            } else {  // above the CONST row
+#pragma unroll
+                for (int u = 0; u < kU; ++u) av[u] = bv[u] = 0.f;
+            }
+            uint32_t hbs[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) hbs[u] = hp[t0 + u];
+            __builtin_amdgcn_wave_barrier();
+            packed_block<kHapHasN, kU, 1>(st, x.w, x.nval, av, bv, hbs, wm + t0, wi + t0);
+            asm volatile("" ::: "memory");  // a wave's LDS operations complete in the order they are issued
+            done[s % kSplitWaves] = (static_cast<uint32_t>(s) << kSplitStepBits) + static_cast<uint32_t>(t0 + kU);
+        }
+    }
+    return st.d1;
+}
+
+template <int kCols, int kU>
+__global__ __launch_bounds__(kSplitWaves * kWave) void forward_kernel_split(DeviceBatch b, DeviceTables tab, WorkSource ws,
+                                                                            RescueSink rs) {
+    extern __shared__ __align__(16) uint8_t lds_raw[];
+    constexpr int kSlots = split_slots<kCols>();
+    constexpr size_t kSlotBytes = split_slot_bytes<kCols>();
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    lds_u32 *const view = (lds_u32 *)(lds_raw + kSlots * kSlotBytes);  // the pair each wave has come to
+    auto record = [&](int slot) {
+        return (volatile __attribute__((address_space(3))) SplitRecord *)(lds_raw + (slot + 1) * kSlotBytes -
+                                                                         sizeof(SplitRecord));
+    };
+    const double scale_log10 = static_cast<double>(Scale<float>::kExp) * 0.30102999566398119521;
+    if (wave == 0) {
+        for (int k = 0; k < kSlots; ++k) record(k)->seq = 0u;
+        for (int k = 0; k < kSplitWaves; ++k) view[k] = 0u;
+    }
+    __syncthreads();
+    uint32_t j = 0, first = 0;  // pair number and the task number of its first stripe
+    for (uint32_t task = wave;; task += kSplitWaves) {
+        uint8_t *base;
+        volatile __attribute__((address_space(3))) SplitRecord *rec;
+        uint32_t n_stripes;
+        // The pair of this task, walking on from the wave's last one.
+        for (;;) {
+            const int slot = static_cast<int>(j % kSlots);
+            base = lds_raw + slot * kSlotBytes;
+            rec = record(slot);
+            if (task == first) {
+                // This wave takes the pair's first stripe: it fetches the pair and fills the slot.
+                for (int k = 0; k < kSplitWaves; ++k)
+                    while (lds_get(view + k) + kSlots <= j) __builtin_amdgcn_s_sleep(1);
+                // The group's first pair is the one of its own number; the next ones come from the queue head.
+                uint32_t it = blockIdx.x;
+                if (j > 0)
+                    it = ws.n_items <= gridDim.x
+                             ? ws.n_items
+                             : gridDim.x + static_cast<uint32_t>(
+                                               __builtin_amdgcn_readfirstlane(atomicAdd(ws.head, lane == 0 ? 1u : 0u)));
+                if (it < ws.n_items) {
+                    const uint32_t pair = __builtin_amdgcn_readfirstlane(ws.items ? ws.items[it] : it);
+                    int r, h;
+                    if (b.pair_read) {
+                        r = b.pair_read[pair];
+                        h = b.pair_hap[pair];
+                    } else {
+                        r = static_cast<int>(pair / static_cast<uint32_t>(b.n_haps));
+                        h = static_cast<int>(pair % static_cast<uint32_t>(b.n_haps));
+                    }
+                    const int R = b.rd_len[r], H = b.hap_len[h];
+                    const int64_t ro = b.rd_off[r];
+                    const bool hap_n = split_stage<kCols>(b.hap_bases + b.hap_off[h], H, base + kHapGuard, lane);
+                    rec->pair = pair;
+                    rec->R = static_cast<uint32_t>(R);
+                    rec->H = static_cast<uint32_t>(H);
+                    rec->ro_lo = static_cast<uint32_t>(ro);
+                    rec->ro_hi = static_cast<uint32_t>(ro >> 32);
+                    rec->hap_n = hap_n ? 1u : 0u;
+                    for (int k = 0; k < kSplitWaves; ++k) rec->done[k] = 0u;
+                    rec->n_stripes = R > 0 ? static_cast<uint32_t>((R + 3 + kWave - 1) / kWave) : 0u;
+                    if (R <= 0) {  // an empty read: L = 0, listed for the FP64 pass
+                        b.out[pair] = -__builtin_inf();
+                        if (rs.list != nullptr)
+                            rs.list[__builtin_amdgcn_readfirstlane(atomicAdd(rs.count, lane == 0 ? 1u : 0u))] = pair;
+                    }
+                } else {
+                    rec->n_stripes = kSplitEnd;
+                }
+                asm volatile("" ::: "memory");
+                rec->seq = j + 1;
+            } else {
+                while (lds_get(&rec->seq) != j + 1) __builtin_amdgcn_s_sleep(1);
+            }
+            asm volatile("" ::: "memory");
+            n_stripes = lds_get(&rec->n_stripes);
+            if (n_stripes == kSplitEnd || task - first < n_stripes) break;
+            first += n_stripes;
+            ++j;
+            view[wave] = j;
+        }
+        if (n_stripes == kSplitEnd) break;
+        PackedPair p{};
+        p.pair = lds_get(&rec->pair);
+        p.R = static_cast<int>(lds_get(&rec->R));
+        p.H = static_cast<int>(lds_get(&rec->H));
+        p.ro = static_cast<int64_t>((static_cast<uint64_t>(lds_get(&rec->ro_hi)) << 32) | lds_get(&rec->ro_lo));
+        WaveLds<float> L;
+        L.hap = base + kHapGuard;
+        L.bm = reinterpret_cast<float *>(base + kHapGuard + kCols);
+        L.bi = L.bm + plane_stride<kCols>();
+        const int s = static_cast<int>(task - first);
+        lds_u32 *const done = (lds_u32 *)rec->done;
+        const float dfin = lds_get(&rec->hap_n) ? split_stripe<kCols, true, kU>(b, tab, p, L, done, lane, s)
+                                                : split_stripe<kCols, false, kU>(b, tab, p, L, done, lane, s);
+        if (s == static_cast<int>(n_stripes) - 1) {
+            // The SUM lane's total to every lane; unscaling and log10 are FP64.
+            const float f = __builtin_bit_cast(
+                float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, dfin), (p.R + 2) & (kWave - 1)));
+            const double sum = static_cast<double>(f);
+            b.out[p.pair] = log10(sum) - scale_log10;
+            if (rs.list != nullptr && !(sum >= rs.threshold))
+                rs.list[__builtin_amdgcn_readfirstlane(atomicAdd(rs.count, lane == 0 ? 1u : 0u))] = p.pair;
+        }
+    }
+}
+
 __global__ void zero_counters_kernel(uint32_t *c, int n) {
     for (int i = threadIdx.x; i < n; i += blockDim.x) c[i] = 0u;
 }
@@ -1067,6 +1344,45 @@ hipError_t with_kernel(bool fp64, bool packed, int cols, int unroll, F &&f) {
 
 }  // namespace
 
+namespace {
+
+// The split kernel for every packed launch whose chunks are one pair (packed_chunk: fewer than eight pairs
+// for each wave of the grid), which is where a wave's pairs would not share stripes anyway.  Measured on
+// one call, packed and split: 1,024 pairs 158 and 129 us, 5,265 pairs 311 and 288, 18,000 pairs 863 and
+// 825, 38,400 pairs 1,189 and 1,196; 200 pairs of 250-600 rows on haplotypes of 1,500 862 and 322.
+hipError_t launch_split(const DeviceBatch &batch, const DeviceTables &tables, const WorkSource &ws, const RescueSink &rescue,
+                        int cols, hipStream_t stream) {
+    return dispatch_col_class(cols, [&](auto C) -> hipError_t {
+        constexpr int kC = decltype(C)::value;
+        if constexpr (kC > kMaxFp32Cols) {
+            return hipErrorInvalidValue;
+        } else {
+            static_assert(split_lds_bytes<kC>() <= 163840, "a workgroup's LDS fits a CU");
+            auto kernel = forward_kernel_split<kC, 8>;
+            if (split_lds_bytes<kC>() > 65536)
+                (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          static_cast<int>(split_lds_bytes<kC>()));
+            static const int per_cu = [&] {
+                int n = 0;
+                const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kSplitWaves * kWave,
+                                                                                  split_lds_bytes<kC>());
+                return e == hipSuccess && n > 0 ? n : 1;
+            }();
+            int dev = 0, cus = 0;
+            if (hipGetDevice(&dev) != hipSuccess ||
+                hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+                cus = 1;
+            const uint32_t grid = std::min<uint32_t>(ws.n_items, static_cast<uint32_t>(per_cu * cus));
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(kSplitWaves * kWave), split_lds_bytes<kC>(), stream, batch, tables,
+                               ws, rescue);
+            return hipGetLastError();
+        }
+    });
+}
+
+}  // namespace
+
 hipError_t launch_forward(bool fp64, const DeviceBatch &batch, const DeviceTables &tables, const WorkSource &work,
                           const RescueSink &rescue, int max_hap_len, const LaunchShape &shape, int grid_blocks,
                           hipStream_t stream) {
@@ -1075,6 +1391,8 @@ hipError_t launch_forward(bool fp64, const DeviceBatch &batch, const DeviceTable
     if (shape.packed && (fp64 || work.head == nullptr || work.n_items_dev != nullptr)) return hipErrorInvalidValue;
     WorkSource ws = work;
     if (shape.packed) ws.chunk = packed_chunk(work.n_items, static_cast<int64_t>(grid_blocks) * shape.waves_per_block);
+    if (shape.packed && ws.chunk == 1)
+        return launch_split(batch, tables, ws, rescue, lds_columns(max_hap_len), stream);
     const dim3 block(kWave * shape.waves_per_block);
     return with_kernel(fp64, shape.packed, lds_columns(max_hap_len), shape.unroll, [&](auto kernel) {
         if (shape.lds_bytes > 65536)

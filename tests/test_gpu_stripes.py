@@ -193,3 +193,35 @@ def test_tuning_round_trip_and_bad_values():
         assert eng.lib.pairhmm_get_tuning(eng.ctx, ctypes.byref(got)) == 0
         assert (got.waves_per_block, got.grid_percent, got.queue_order, got.stripe_schedule, got.step_unroll) == \
             (2, 150, 1, 0, 16)
+
+
+@pytest.mark.parametrize("hap_len", [1, 30, 200, 480, 700, 1000, 2300, 4800])
+def test_split_stripes(hap_len):
+    """Small queues split a pair's stripes over a workgroup's waves: pairs of 0 to 13 stripes in mixed order
+    (empty reads between others, several one-stripe pairs in a row), more pairs than resident groups at
+    the short lengths, every LDS class size on both sides of the four- and two-slot groups, 'N' bytes.
+    Against the oracle, and three passes bit for bit."""
+    rng = np.random.default_rng(hap_len)
+    lens = [0, 1, 2, 3, 60, 61, 62, 63, 64, 65, 124, 125, 126, 127, 188, 189, 190, 253, 254, 317, 400, 520, 800]
+    if hap_len <= 200:
+        lens += [5] * 40 + [0] * 3 + list(rng.integers(1, 130, 130))
+    elif hap_len > 2000:
+        lens = lens[:18]
+    regions = []
+    for k in range(2):
+        order = rng.permutation(lens)
+        regions.append(_region(rng, order, hap_n=k == 1 and hap_len >= 30, hap_len=hap_len, n_haps=1 if hap_len == 1 else 9 if hap_len <= 200 else 3))
+    b = pack_regions(regions)
+    want = oracle.logless_batch(b, n_threads=8)
+    with BatchEngine() as eng:
+        dev = eng.upload(b)
+        outs = []
+        for _ in range(3):
+            out = np.empty(b.n_pairs)
+            dev.forward(out=out)
+            outs.append(out)
+        dev.free()
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isfinite(outs[0]), fin)
+    assert np.max(np.abs(outs[0][fin] - want[fin])) <= 1e-4
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
