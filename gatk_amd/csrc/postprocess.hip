@@ -11,9 +11,9 @@
 //      dropped when its best likelihood is below ceil(L * rate) * -4 (at most 2 errors unless the
 //      DRAGEN dynamic threshold is on, which takes the lower of that and
 //      -0.1 (sum mean_q + K sqrt(sum var_q)) over the read's HMM base qualities).
-// One thread per read; a wave's 64 matrix rows and quality strings are staged through LDS with
-// coalesced loads.  FP64 with contraction off, so every sum and product rounds where Java's do (the
-// quality sums run in read order).
+// One thread per read.  A wave's 64 matrix rows are staged through LDS with coalesced loads; a lane reads
+// its own qualities, 64 bytes at a time.  FP64 with contraction off, so every sum and product rounds where
+// Java's do (the quality sums run in read order).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -38,10 +38,10 @@ __constant__ double kDynVar[40] = {
     2.791361596, 2.370765375, 2.008921719, 1.698687797, 1.433525748, 1.207526336, 1.015402928, 0.852465956,
     0.714585285, 0.598145851, 0.500000349, 0.41742159,  0.348056286, 0.289881373, 0.241163527, 0.200422214};
 
-constexpr int kPpWaves = 2;             // waves per workgroup, each over 64 consecutive reads
-constexpr int kQualStage = 10240;       // bytes of HBM qualities a wave stages in LDS
+constexpr int kPpWaves = 4;             // waves per workgroup, each over 64 consecutive reads
 constexpr int kRowStage = 512;          // likelihoods a wave stages in LDS (64 reads x 8 haplotypes)
-constexpr int kQualBatch = 10;          // quality words per lane in flight while staging
+constexpr int kNoQual = 256;            // table entry of a byte outside the read: adds 0
+constexpr int kGranules = 4;            // 16-byte granules of a lane's qualities in flight
 
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -49,31 +49,48 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Sums of the table's mean and variance over a read's qualities, in read order (the order the
-// reference adds them).  Unrolled so the reads of later bases issue ahead of the ordered FP64 sums.
-__device__ __forceinline__ void quality_sums(const uint8_t *src, int L, const double2 *tab, double &s_mean,
-                                             double &s_var) {
+// A lane's qualities, as 16-byte granules from the one that holds the first of them (whole granules around
+// valid bytes stay inside the allocation's pages): kGranules from granule k, those that hold any.
+__device__ __forceinline__ void load_granules(uint4 (&g)[kGranules], const uint4 *q, int k, int n) {
+#pragma unroll
+    for (int i = 0; i < kGranules; ++i)
+        if (k + i < n) g[i] = q[k + i];
+}
+
+// Adds the table entries of a granule's 16 bytes, in order.  kWhole: every byte belongs to the lane's read;
+// else byte b does if at + b lies in [0, L), and the others add entry kNoQual.
+template <bool kWhole>
+__device__ __forceinline__ void add_granule(const uint4 &g, int at, int L, const double2 *tab, double &s_mean,
+                                            double &s_var) {
 #pragma clang fp contract(off)
-#pragma unroll 8
-    for (int i = 0; i < L; ++i) {
-        const int bq = src[i];
-        const int e = bq <= 1 ? 0 : (bq < 40 ? bq : 40) - 1;
+    const uint32_t w[4] = {g.x, g.y, g.z, g.w};
+#pragma unroll
+    for (int b = 0; b < 16; ++b) {
+        uint32_t e = (w[b / 4] >> (8 * (b % 4))) & 0xFFu;
+        if (!kWhole) e = static_cast<uint32_t>(at + b) < static_cast<uint32_t>(L) ? e : kNoQual;
         const double2 mv = tab[e];
         s_mean += mv.x;
         s_var += mv.y;
     }
 }
 
+// The kernel is bound by HBM latency and by the LDS lookups, 16 bytes per quality at lane-random entries.
+// Staging the qualities in LDS too held a CU to ten waves, took only spans of up to 10,240 bytes per wave
+// (reads of 160 on average; longer ones went byte by byte from global memory) and ran 13 VALU instructions
+// per quality; a lane's own 64-byte loads touch each line about twice and leave 6.  400,000 reads x 8
+// haplotypes, 100-250 bases: a call takes 63 us, 95 with the staged qualities.
 __global__ __launch_bounds__(kPpWaves * 64) void postprocess_kernel(PostprocessArgs p) {
 #pragma clang fp contract(off)
-    // The table in LDS: per-base lookups differ lane to lane, which LDS serves far better than
-    // gathers from global memory.
-    __shared__ double2 tab[40];
-    // Each wave's reads are adjacent in the matrix and (usually) in the quality plane: both are
-    // brought into LDS with coalesced loads, worked on there, and the rows written back coalesced.
-    __shared__ uint32_t qstage[kPpWaves][kQualStage / 4];
+    // The table in LDS by quality byte: per-base lookups differ lane to lane, which LDS serves far better
+    // than gathers from global memory.
+    __shared__ double2 tab[kNoQual + 1];
+    // Each wave's rows are adjacent in the matrix: brought into LDS with coalesced loads, worked on there,
+    // and written back coalesced.
     __shared__ double rstage[kPpWaves][kRowStage];
-    if (threadIdx.x < 40) tab[threadIdx.x] = make_double2(kDynMean[threadIdx.x], kDynVar[threadIdx.x]);
+    for (int q = threadIdx.x; q <= kNoQual; q += blockDim.x) {
+        const int e = q <= 1 ? 0 : (q < 40 ? q : 40) - 1;
+        tab[q] = q == kNoQual ? make_double2(0.0, 0.0) : make_double2(kDynMean[e], kDynVar[e]);
+    }
     __syncthreads();
     const int w = static_cast<int>(threadIdx.x) / 64, lane = static_cast<int>(threadIdx.x) % 64;
     const int64_t r0 = (static_cast<int64_t>(blockIdx.x) * kPpWaves + w) * 64;
@@ -87,9 +104,8 @@ __global__ __launch_bounds__(kPpWaves * 64) void postprocess_kernel(PostprocessA
     double *const grow = p.likelihoods + r0 * A;
     const int L = has ? p.read_len[r] : 0;
     const uint8_t *q = p.base_quals + (has && p.dynamic ? p.read_off[r] : 0);
-    // Every HBM load of the wave is issued before the first wait: the row loads go to registers
-    // first (nr * A <= kRowStage = 8 * 64, so eight per lane), then the qualities are staged, then
-    // the rows are stored to LDS; one wave barrier covers both.
+    // The wave's first HBM loads are issued before the first wait: the rows (nr * A <= kRowStage = 8 * 64, so
+    // eight values per lane) and the first granules of each lane's qualities.
     double rt[kRowStage / 64];
     if (stage_rows) {
 #pragma unroll
@@ -98,60 +114,19 @@ __global__ __launch_bounds__(kPpWaves * 64) void postprocess_kernel(PostprocessA
             rt[u] = e < nr * A ? grow[e] : 0.0;
         }
     }
-    // The wave's quality span [lo, hi) in global addresses; staged when it fits, read in place
-    // otherwise.
-    bool stage_q = false;
-    uint64_t blo = 0;
-    uint8_t *const qb = reinterpret_cast<uint8_t *>(qstage[w]);
-    if (p.dynamic) {
-        uint64_t lo = has ? reinterpret_cast<uintptr_t>(q) : ~0ull, hi = has ? lo + L : 0ull;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const uint64_t olo = __shfl_xor(static_cast<unsigned long long>(lo), off, 64);
-            const uint64_t ohi = __shfl_xor(static_cast<unsigned long long>(hi), off, 64);
-            lo = olo < lo ? olo : lo;
-            hi = ohi > hi ? ohi : hi;
-        }
-        blo = lo & ~3ull;
-        stage_q = hi > lo && hi - blo <= static_cast<uint64_t>(kQualStage);
-        if (stage_q) {
-            const uint64_t wlo = (lo + 3) & ~3ull, whi = hi & ~3ull;
-            // Derived from the plane's pointer (not from the integer address) so the loads stay global.
-            const uint8_t *gb = p.base_quals + (blo - reinterpret_cast<uintptr_t>(p.base_quals));
-            if (wlo < whi) {
-                const __attribute__((address_space(1))) uint32_t *gw =
-                    (const __attribute__((address_space(1))) uint32_t *)(gb + (wlo - blo));
-                const int nw = static_cast<int>((whi - wlo) / 4), w0 = static_cast<int>((wlo - blo) / 4);
-                // Batches of kQualBatch loads per lane in flight before their stores.
-                for (int k0 = lane; k0 < nw; k0 += 64 * kQualBatch) {
-                    uint32_t t[kQualBatch];
-#pragma unroll
-                    for (int u = 0; u < kQualBatch; ++u) {
-                        const int k = k0 + 64 * u;
-                        t[u] = k < nw ? gw[k] : 0u;
-                    }
-#pragma unroll
-                    for (int u = 0; u < kQualBatch; ++u) {
-                        const int k = k0 + 64 * u;
-                        if (k < nw) qstage[w][w0 + k] = t[u];
-                    }
-                }
-                const int head = static_cast<int>(wlo - lo), tail = static_cast<int>(hi - whi);
-                if (lane < head) qb[lo - blo + lane] = gb[lo - blo + lane];
-                if (lane < tail) qb[whi - blo + lane] = gb[whi - blo + lane];
-            } else {
-                for (int k = lane; k < static_cast<int>(hi - lo); k += 64) qb[lo - blo + k] = gb[lo - blo + k];
-            }
-        }
-    }
+    const int skip = static_cast<int>(reinterpret_cast<uintptr_t>(q) & 15);  // bytes of the first granule before the read
+    const uint4 *const gq = reinterpret_cast<const uint4 *>(q - skip);
+    const int n_granules = p.dynamic && L > 0 ? (skip + L + 15) / 16 : 0;
+    uint4 g[kGranules] = {};
+    load_granules(g, gq, 0, n_granules);
     if (stage_rows) {
 #pragma unroll
         for (int u = 0; u < kRowStage / 64; ++u) {
             const int e = lane + 64 * u;
             if (e < nr * A) rstage[w][e] = rt[u];
         }
+        wave_lds_sync();
     }
-    if (stage_rows || stage_q) wave_lds_sync();
     double *v = !has ? rstage[w] : stage_rows ? &rstage[w][lane * A] : p.likelihoods + r * A;
 
     if (has && p.normalize && A >= 2) {
@@ -170,13 +145,22 @@ __global__ __launch_bounds__(kPpWaves * 64) void postprocess_kernel(PostprocessA
     const double errors = ceil(static_cast<double>(L) * p.max_error_per_base);
     double t = (p.dynamic ? errors : fmin(2.0, errors)) * -4.0;
     if (p.dynamic) {
-        // Sums in read order, as the reference adds them; two calls so each loop sees one address
-        // space (LDS or global) and its reads pipeline.
+        // Sums in read order, as the reference adds them, the next granules loading meanwhile.
         double s_mean = 0.0, s_var = 0.0;
-        if (stage_q)
-            quality_sums(qb + (reinterpret_cast<uintptr_t>(q) - blo), L, tab, s_mean, s_var);
-        else
-            quality_sums(q, L, tab, s_mean, s_var);
+        for (int k = 0; __any(k < n_granules); k += kGranules) {
+            uint4 next[kGranules] = {};
+            load_granules(next, gq, k + kGranules, n_granules);
+#pragma unroll
+            for (int i = 0; i < kGranules; ++i) {
+                const int at = 16 * (k + i) - skip;  // the granule's first byte in the read
+                if (__all(at >= 0 && at + 16 <= L))
+                    add_granule<true>(g[i], at, L, tab, s_mean, s_var);
+                else if (__any(at < L))
+                    add_granule<false>(g[i], at, L, tab, s_mean, s_var);
+            }
+#pragma unroll
+            for (int i = 0; i < kGranules; ++i) g[i] = next[i];
+        }
         const double d = (s_mean + p.scale * sqrt(s_var)) * -0.1;
         if (d < t) t = d;
     }

@@ -59,3 +59,27 @@ def test_engine_default_cap_and_argument_errors():
             p.normalize_and_filter(lk, ln, 5, -4.5)       # reference index out of range
         keep, _ = p.normalize_and_filter(lk, ln, 0, -4.5)
     assert keep.cpu().tolist() == [1, 1, 1, 1]
+
+
+@pytest.mark.parametrize("shift", [0, 1, 7, 15])
+def test_quality_granules(shift):
+    """Reads that begin and end on every byte of the kernel's 16-byte granules and around its 64-byte loads, in
+    a plane that begins `shift` bytes into its allocation, the reads in no order and some sharing bytes."""
+    rng = np.random.default_rng(shift)
+    lens = np.concatenate([np.arange(0, 140), [255, 256, 257, 1000], rng.integers(0, 300, 60)]).astype(np.int32)
+    plane = rng.integers(0, 256, 4096).astype(np.uint8)
+    off = np.array([int(rng.integers(0, len(plane) - n + 1)) for n in lens], np.int64)
+    off[:2] = 0, len(plane) - 1
+    lens[1] = 1
+    lk = -rng.exponential(15.0, (len(lens), 3))
+    dev = torch.from_numpy(np.concatenate([np.zeros(shift, np.uint8), plane])).cuda()[shift:]
+    d_lk, d_len, d_off = (torch.from_numpy(x).cuda() for x in (lk.copy(), lens, off))
+    th = torch.empty(len(lens), dtype=torch.float64, device="cuda")
+    with LikelihoodPostProcessor() as p:
+        keep, _ = p.normalize_and_filter(d_lk, d_len, 0, -4.5, False, dev, d_off, 0.02, True, 1.0, threshold=th)
+    torch.cuda.synchronize()
+    norm, want_keep, want_th = pp.postprocess(lk, [plane[o:o + n] for o, n in zip(off, lens)], -4.5, False, 0, True,
+                                              0.02, 1.0)
+    assert np.array_equal(d_lk.cpu().numpy(), norm)
+    assert np.array_equal(th.cpu().numpy(), want_th)
+    assert np.array_equal(keep.cpu().numpy().astype(bool), want_keep)
