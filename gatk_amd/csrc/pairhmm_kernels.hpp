@@ -191,7 +191,10 @@ int dragstr_max_read_length();
 
 // ---- partially determined PairHMM (pdhmm.hip) ----------------------------------------------
 
-// Column code of a partially determined haplotype (built on the host from the haplotype base and
+// PartiallyDeterminedHaplotype byte layout (PartiallyDeterminedHaplotype.java:59-66).
+constexpr uint32_t kPdByteSnp = 1, kPdByteDelStart = 2, kPdByteDelEnd = 4, kPdByteAlts = 0x78;
+
+// Column code of a partially determined haplotype (pd_codes_kernel, from the haplotype base and
 // its PartiallyDeterminedHaplotype byte): bits 0-7 the base; bits 8-15 the bases the column also
 // accepts (the SNP alternatives A/C/G/T at the PD byte's own bit positions, or every class bit for
 // an 'N' base); kPdDelEnd when the base ends a deletion span; kPdInsideRow1 / kPdInsideLater when
@@ -216,7 +219,7 @@ struct PdBatch {
     const int32_t *rd_len;
     int32_t n_haps;
     int32_t tristate;
-    int32_t odd_bases;         // some haplotype byte lies outside ACGTacgtN
+    const uint32_t *odd_bases; // device word: not 0 when some haplotype byte lies outside ACGTacgtN
     double *out;
     const uint32_t *order;     // launch order of the pairs (longest first), or null
 };
@@ -224,6 +227,9 @@ struct PdBatch {
 // LDS of one wave (one workgroup) for haplotypes up to max_hap_len: a 16-byte record and a 4-byte
 // column code per column.
 size_t pd_lds_bytes(int max_hap_len);
+// Codes of every haplotype; odd_bases (device) is set to 1 where one has a byte outside ACGTacgtN.
+hipError_t launch_pd_codes(const uint8_t *bases, const uint8_t *pd, const int64_t *hap_off, const int32_t *hap_len,
+                           int32_t n_haps, uint32_t *code, uint32_t *odd_bases, hipStream_t stream);
 hipError_t launch_pd_forward(const PdBatch &batch, const DeviceTables &tables, uint32_t n_pairs, int max_hap_len,
                              int grid_blocks, hipStream_t stream);
 

@@ -18,7 +18,7 @@
 // (in NORMAL and INSIDE_DEL the column before carries no DEL_END, so E = X there).  Only
 // INSIDE_DEL depends on the row: the state variable is declared outside the row loop (:63), so row 1
 // starts NORMAL and every later row starts in the state the previous row ended in, which is the
-// same for all rows >= 2.  The host folds this into each column's code (pd_column_codes).
+// same for all rows >= 2.  pd_codes_kernel folds this into each column's code.
 //
 // Mapping: one pair per wave.  A lane owns kRows = 2 consecutive rows (a stripe of 128; 1 row for a last
 // part of up to 64) and at step t computes column c = t - lane + 1 of all of them.  Each row forms, from its new E values and the transitions of the
@@ -34,7 +34,7 @@
 // from row 0: M = I = 0, D = 2^1020 / H, so A(1,c) = D GM_1 and B(1,c) = 0.  A wave holds 20 bytes of LDS
 // per column with the column's 4-byte code.
 //
-// Steps run in blocks of 4; a block in which no lane is on a special column (the host's kPdSpecial: a
+// Steps run in blocks of 4; a block in which no lane is on a special column (kPdSpecial: a
 // deletion end, a column inside a span, or the column before a span) skips the branch update and
 // hands on E = X, which is exact because a row's branch values are only read on special columns and
 // the column before each span sets them from E.
@@ -359,6 +359,67 @@ __device__ __forceinline__ void pd_pair(const PdBatch &b, const DeviceTables &ta
     }
 }
 
+// Column codes of one haplotype per workgroup (layout in pairhmm_kernels.hpp).  A column is processed inside
+// a deletion when the last column before it that starts or ends one starts one (and does not also end
+// it), LoglessPDPairHMM.java:63-136; row 1 begins outside, every later row in the state the row before
+// ended in (the state variable lives outside the row loop, :63), which is the same for all rows >= 2.  Bound by
+// latency (a few chunks of loads and ballots per haplotype); the same loop on the host was a fifth of the
+// call (81 reads of 100-250 by 65 haplotypes of 377: 467 us with it, 383 us with this kernel).
+__global__ __launch_bounds__(kWave) void pd_codes_kernel(const uint8_t *__restrict__ bases, const uint8_t *__restrict__ pd,
+                                                         const int64_t *__restrict__ hap_off,
+                                                         const int32_t *__restrict__ hap_len, uint32_t *code,
+                                                         uint32_t *odd_bases) {
+    const int lane = static_cast<int>(threadIdx.x);
+    const int64_t o = hap_off[blockIdx.x];
+    const int H = hap_len[blockIdx.x];
+    // Columns that start a deletion (and do not end one) and columns that start or end one, of a chunk.
+    auto events = [&](int j0, uint64_t &starts, uint64_t &any) {
+        const int j = j0 + lane;
+        const uint32_t v = j < H ? pd[o + j] : 0u;
+        starts = __ballot((v & (kPdByteDelStart | kPdByteDelEnd)) == kPdByteDelStart);
+        any = __ballot((v & (kPdByteDelStart | kPdByteDelEnd)) != 0u);
+        return v;
+    };
+    // Whether the last of the events `any` starts a deletion; `before` where there is none.
+    auto inside_after = [](uint64_t starts, uint64_t any, bool before) {
+        return any ? ((starts >> (kWave - 1 - __builtin_clzll(any))) & 1u) != 0u : before;
+    };
+    bool row1_end = false;
+    for (int j0 = 0; j0 < H; j0 += kWave) {
+        uint64_t starts, any;
+        events(j0, starts, any);
+        row1_end = inside_after(starts, any, row1_end);
+    }
+    bool row1 = false, later = row1_end;
+    bool odd = false;
+    const uint64_t below = lane == 0 ? 0ull : ~0ull >> (kWave - lane), upto = ~0ull >> (kWave - 1 - lane);
+    for (int j0 = 0; j0 < H; j0 += kWave) {
+        uint64_t starts, any;
+        const uint32_t v = events(j0, starts, any);
+        const int j = j0 + lane;
+        if (j < H) {
+            const uint32_t y = bases[o + j], alt = (v & kPdByteSnp) ? (v & kPdByteAlts) : 0u;
+            uint32_t c = y | (alt << 8) | ((alt >> 3) * 0x11u * kPdAcceptA);  // an alternative accepts both cases
+            if (y == 'N')  // an 'N' haplotype base matches every read base (:163)
+                c |= (0xF8u << 8) | (0xFFu * kPdAcceptA) | kPdAcceptOther;
+            else if (accept_bit(y) != kPdAcceptOther)
+                c |= accept_bit(y);
+            else
+                odd = true;
+            if (v & kPdByteDelEnd) c |= kPdDelEnd | kPdSpecial;
+            if (inside_after(starts & below, any & below, row1)) c |= kPdInsideRow1 | kPdSpecial;
+            if (inside_after(starts & below, any & below, later)) c |= kPdInsideLater | kPdSpecial;
+            // The column before one inside a span.
+            if (j + 1 < H && (inside_after(starts & upto, any & upto, row1) || inside_after(starts & upto, any & upto, later)))
+                c |= kPdSpecial;
+            code[o + j] = c;
+        }
+        row1 = inside_after(starts, any, row1);
+        later = inside_after(starts, any, later);
+    }
+    if (__any(odd)) *odd_bases = 1u;
+}
+
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4))) void pd_forward_kernel(
     PdBatch b, DeviceTables tab, uint32_t n_pairs, int rec_columns) {
     extern __shared__ PdRecord lds_rec[];
@@ -384,7 +445,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4))) void
         int low = 0;
         for (int p = lane; p < R; p += kWave)
             low |= b.rd_quals[ro + p] == 0 || b.rd_ins[ro + p] < 4 || b.rd_del[ro + p] < 4;
-        const bool generic = b.odd_bases || __any(low);
+        const bool generic = *b.odd_bases != 0u || __any(low);
         // Row 1's sums over row 0 (M = I = 0, D = d0 on columns 0..H): A(c) = d0 GM_1 for 1 <= c <= H + 1.
         const double gm1 = pd_row(b, tab, ro, R, 0).GM * (generic ? 1.0 : pd_first_fold(b, tab, ro, R, 0, pd_stripe_rows(R)));
         __builtin_amdgcn_wave_barrier();
@@ -411,6 +472,13 @@ int pd_record_columns(int max_hap_len) { return max_hap_len + kPdPadColumns; }
 
 size_t pd_lds_bytes(int max_hap_len) {
     return static_cast<size_t>(kPdLowPad + pd_record_columns(max_hap_len)) * (sizeof(PdRecord) + sizeof(uint32_t));
+}
+
+hipError_t launch_pd_codes(const uint8_t *bases, const uint8_t *pd, const int64_t *hap_off, const int32_t *hap_len,
+                           int32_t n_haps, uint32_t *code, uint32_t *odd_bases, hipStream_t stream) {
+    if (n_haps <= 0) return hipSuccess;
+    hipLaunchKernelGGL(pd_codes_kernel, dim3(n_haps), dim3(kWave), 0, stream, bases, pd, hap_off, hap_len, code, odd_bases);
+    return hipGetLastError();
 }
 
 hipError_t launch_pd_forward(const PdBatch &batch, const DeviceTables &tables, uint32_t n_pairs, int max_hap_len,

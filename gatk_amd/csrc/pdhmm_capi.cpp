@@ -8,7 +8,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <array>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -21,58 +20,37 @@ using namespace gatk_pairhmm::capi;
 
 namespace {
 
-// PartiallyDeterminedHaplotype byte layout (PartiallyDeterminedHaplotype.java:59-66).
-constexpr uint8_t kPdSnp = 1, kPdDelStart = 2, kPdDelEndByte = 4, kPdAltMask = 0x78;
-
-enum class PdState { Normal, InsideDel, AfterDel };  // LoglessPDPairHMM.java:22-31
-
-// One pass of LoglessPDPairHMM's state machine over a row (:63-136): ORs `inside_bit` into the code
-// of every column processed in INSIDE_DEL and returns the state the row ends in.
-PdState pd_state_pass(const uint8_t *pd, int H, PdState state, uint32_t inside_bit, uint32_t *code) {
-    for (int j = 0; j < H; ++j) {
-        if (state == PdState::InsideDel) code[j] |= inside_bit;
-        if (state == PdState::AfterDel) state = PdState::Normal;
-        if (pd[j] & kPdDelStart) state = PdState::InsideDel;
-        if (pd[j] & kPdDelEndByte) state = PdState::AfterDel;
-    }
-    return state;
-}
-
-// Column codes of one haplotype (layout in pairhmm_kernels.hpp).  Row 1 starts NORMAL; every later
-// row starts in the state the row before ended in (the state variable lives outside the row loop,
-// :63), which is the same state for all rows >= 2.
-// Returns whether every base is one of ACGTacgtN.
-bool pd_column_codes(const uint8_t *bases, const uint8_t *pd, int H, uint32_t *code) {
-    // Per base: itself, an 'N's alternatives and the read-base classes it accepts; 0 for other bytes.
-    static const std::array<uint32_t, 256> of_base = [] {
-        std::array<uint32_t, 256> t{};
-        const char known[] = "ACGTacgt";
-        for (int k = 0; k < 8; ++k) t[static_cast<uint8_t>(known[k])] = static_cast<uint8_t>(known[k]) | (kPdAcceptA << k);
-        // An 'N' haplotype base matches every read base (:163).
-        t['N'] = 'N' | (0xF8u << 8) | (0xFFu * kPdAcceptA) | kPdAcceptOther;
-        return t;
-    }();
-    bool known = true;
-    for (int j = 0; j < H; ++j) {
-        const uint32_t y = bases[j], alt = (pd[j] & kPdSnp) ? (pd[j] & kPdAltMask) : 0u;
-        known = known && of_base[y] != 0u;
-        // Alternatives A, C, G, T are bits 3..6 of the PD byte and accept both cases.
-        code[j] = (of_base[y] ? of_base[y] : y) | (alt << 8) | ((alt >> 3) * 0x11u * kPdAcceptA) |
-                  ((pd[j] & kPdDelEndByte) ? kPdDelEnd : 0u);
-    }
-    const PdState end1 = pd_state_pass(pd, H, PdState::Normal, kPdInsideRow1, code);
-    pd_state_pass(pd, H, end1, kPdInsideLater, code);
-    constexpr uint32_t inside = kPdInsideRow1 | kPdInsideLater;
-    for (int j = 0; j < H; ++j)
-        if ((code[j] & (inside | kPdDelEnd)) || (j + 1 < H && (code[j + 1] & inside))) code[j] |= kPdSpecial;
-    return known;
-}
-
 bool is_pd_base(uint8_t x) {
     switch (x) {
     case 'A': case 'a': case 'C': case 'c': case 'G': case 'g': case 'T': case 't': case 'N': return true;
     default: return false;
     }
+}
+
+// isBasePDMatching throws for a read base outside ACGTacgtN on a SNP column whose haplotype base is
+// neither that base nor 'N' (LoglessPDPairHMM.java:163, 195-196).
+int32_t check_read_bases(const pairhmm_read_data_holder *reads, int32_t n_reads,
+                         const pairhmm_pd_haplotype_data_holder *haps, int32_t n_haps) {
+    bool on_snp[256] = {}, known = false;  // haplotype bases on SNP columns, gathered at the first odd read base
+    for (int32_t r = 0; r < n_reads; ++r) {
+        const pairhmm_read_data_holder &rd = reads[r];
+        for (int i = 0; i < rd.length; ++i) {
+            const uint8_t x = rd.read_bases[i];
+            if (is_pd_base(x)) continue;
+            if (!known) {
+                for (int32_t h = 0; h < n_haps; ++h)
+                    for (int j = 0; j < haps[h].length; ++j)
+                        if (haps[h].haplotype_pd_bases[j] & kPdByteSnp) on_snp[haps[h].haplotype_bases[j]] = true;
+                known = true;
+            }
+            for (int y = 0; y < 256; ++y)
+                if (on_snp[y] && y != x && y != 'N')
+                    return fail(PAIRHMM_ERR_BAD_ARG, "read " + std::to_string(r) + " base " +
+                                                         std::to_string(static_cast<int>(x)) +
+                                                         " meets a SNP column: Found unexpected base in alt alleles");
+        }
+    }
+    return PAIRHMM_OK;
 }
 
 }  // namespace
@@ -93,33 +71,14 @@ extern "C" int32_t pairhmm_pd_compute_likelihoods(pairhmm_context *ctx, const pa
         if (st != PAIRHMM_OK) return st;
         read_bytes += rd.length;
     }
-    // isBasePDMatching throws for a read base outside ACGTacgtN on a SNP column whose haplotype base
-    // is neither that base nor 'N' (LoglessPDPairHMM.java:163, 195-196).  Haplotype side: which
-    // bases sit on SNP columns.
-    std::vector<std::array<bool, 256>> snp_bases(n_haps);
     for (int32_t h = 0; h < n_haps; ++h) {
         const pairhmm_pd_haplotype_data_holder &hp = haps[h];
         if (hp.length <= 0 || hp.haplotype_bases == nullptr || hp.haplotype_pd_bases == nullptr)
             return fail(PAIRHMM_ERR_BAD_ARG, "haplotype " + std::to_string(h) + " is empty or has a null array");
         hap_cols += hp.length;
         max_h = std::max(max_h, hp.length);
-        snp_bases[h].fill(false);
-        for (int j = 0; j < hp.length; ++j)
-            if (hp.haplotype_pd_bases[j] & kPdSnp) snp_bases[h][hp.haplotype_bases[j]] = true;
     }
-    for (int32_t r = 0; r < n_reads; ++r) {
-        const pairhmm_read_data_holder &rd = reads[r];
-        for (int i = 0; i < rd.length; ++i) {
-            const uint8_t x = rd.read_bases[i];
-            if (is_pd_base(x)) continue;
-            for (int32_t h = 0; h < n_haps; ++h)
-                for (int y = 0; y < 256; ++y)
-                    if (snp_bases[h][y] && y != x && y != 'N')
-                        return fail(PAIRHMM_ERR_BAD_ARG, "read " + std::to_string(r) + " base " +
-                                                             std::to_string(static_cast<int>(x)) +
-                                                             " meets a SNP column: Found unexpected base in alt alleles");
-        }
-    }
+    if (const int32_t st = check_read_bases(reads, n_reads, haps, n_haps); st != PAIRHMM_OK) return st;
     const int64_t n_pairs = static_cast<int64_t>(n_reads) * n_haps;
     if (n_pairs > 0xFFFFFFFFll) return fail(PAIRHMM_ERR_BAD_ARG, "too many pairs in one call");
     if (pd_lds_bytes(max_h) > max_lds_per_block())
@@ -132,11 +91,12 @@ extern "C" int32_t pairhmm_pd_compute_likelihoods(pairhmm_context *ctx, const pa
         return o;
     };
     const size_t o_rb = take(read_bytes), o_rq = take(read_bytes), o_ri = take(read_bytes), o_rd = take(read_bytes),
-                 o_rg = take(read_bytes), o_hc = take(sizeof(uint32_t) * hap_cols),
+                 o_rg = take(read_bytes), o_hb = take(hap_cols), o_hp = take(hap_cols),
                  o_roff = take(sizeof(int64_t) * n_reads), o_rlen = take(sizeof(int32_t) * n_reads),
                  o_hoff = take(sizeof(int64_t) * n_haps), o_hlen = take(sizeof(int32_t) * n_haps),
-                 o_order = take(sizeof(uint32_t) * n_pairs);
+                 o_order = take(sizeof(uint32_t) * n_pairs), o_odd = take(sizeof(uint32_t));
     const size_t in_bytes = off;
+    const size_t o_hc = take(sizeof(uint32_t) * hap_cols);  // column codes, made on the device
     const size_t o_out = take(sizeof(double) * n_pairs);
     const size_t total = off;
 
@@ -149,7 +109,6 @@ extern "C" int32_t pairhmm_pd_compute_likelihoods(pairhmm_context *ctx, const pa
     int32_t *rlen = reinterpret_cast<int32_t *>(hs + o_rlen);
     int64_t *hoff = reinterpret_cast<int64_t *>(hs + o_hoff);
     int32_t *hlen = reinterpret_cast<int32_t *>(hs + o_hlen);
-    uint32_t *hcode = reinterpret_cast<uint32_t *>(hs + o_hc);
     int64_t pos = 0;
     for (int32_t r = 0; r < n_reads; ++r) {
         const pairhmm_read_data_holder &rd = reads[r];
@@ -165,13 +124,14 @@ extern "C" int32_t pairhmm_pd_compute_likelihoods(pairhmm_context *ctx, const pa
         pos += rd.length;
     }
     pos = 0;
-    bool known_bases = true;
     for (int32_t h = 0; h < n_haps; ++h) {
         hoff[h] = pos;
         hlen[h] = haps[h].length;
-        known_bases &= pd_column_codes(haps[h].haplotype_bases, haps[h].haplotype_pd_bases, haps[h].length, hcode + pos);
+        std::memcpy(hs + o_hb + pos, haps[h].haplotype_bases, haps[h].length);
+        std::memcpy(hs + o_hp + pos, haps[h].haplotype_pd_bases, haps[h].length);
         pos += haps[h].length;
     }
+    *reinterpret_cast<uint32_t *>(hs + o_odd) = 0u;
     // Workgroups are dispatched in order: longest reads first, and each read's haplotypes longest
     // first, keeps the last wave of a launch short (outputs stay read-major).
     uint32_t *order = reinterpret_cast<uint32_t *>(hs + o_order);
@@ -200,11 +160,14 @@ extern "C" int32_t pairhmm_pd_compute_likelihoods(pairhmm_context *ctx, const pa
     b.rd_len = reinterpret_cast<const int32_t *>(ds + o_rlen);
     b.n_haps = n_haps;
     b.tristate = 1;
-    b.odd_bases = known_bases ? 0 : 1;
+    b.odd_bases = reinterpret_cast<const uint32_t *>(ds + o_odd);
     b.out = reinterpret_cast<double *>(ds + o_out);
     DeviceTables tab{ctx->d_qual_err, ctx->d_mm_prob};
     // One wave per workgroup and per pair; the hardware dispatcher balances uneven pairs.
     const int grid = static_cast<int>(std::min<int64_t>(n_pairs, 1 << 20));
+    HIP_TRY(launch_pd_codes(ds + o_hb, ds + o_hp, b.hap_off, b.hap_len, n_haps, reinterpret_cast<uint32_t *>(ds + o_hc),
+                            reinterpret_cast<uint32_t *>(ds + o_odd), ctx->stream),
+            PAIRHMM_ERR_KERNEL);
     HIP_TRY(launch_pd_forward(b, tab, static_cast<uint32_t>(n_pairs), max_h, grid, ctx->stream), PAIRHMM_ERR_KERNEL);
     HIP_TRY(hipMemcpyAsync(hs, ds + o_out, sizeof(double) * n_pairs, hipMemcpyDeviceToHost, ctx->stream),
             PAIRHMM_ERR_KERNEL);

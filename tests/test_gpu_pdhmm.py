@@ -132,6 +132,27 @@ def test_dense_deletion_spans():
     _check(reads, haps, "dense deletion spans")
 
 
+@pytest.mark.parametrize("hap_len", [1, 63, 64, 65, 128, 193])
+def test_column_codes_across_chunks(hap_len):
+    """Column codes are made 64 columns at a time: spans that start, end and stay open on both sides of
+    each multiple of 64 (also without an end, so that every later row begins inside one), with SNPs and
+    lower-case and ambiguity bases in between."""
+    rng = np.random.default_rng(hap_len)
+    haps = []
+    for span in ((62, 63), (63, 64), (63, 63), (64, 64), (10, 130), (0, 191), (192, None), (64, None), (0, None)):
+        hap, pd = _pd_haplotype(rng, hap_len, 2, 0)
+        hap = bytearray(hap)
+        hap[hap_len // 2] = b"acgtR"[len(haps) % 5]
+        pd = bytearray(b & ~(SNP | A | C | G | T) if hap[j] not in b"ACGT" else b for j, b in enumerate(pd))
+        start, end = span
+        pd[min(start, hap_len - 1)] |= DEL_START
+        if end is not None:
+            pd[min(end, hap_len - 1)] |= DEL_END
+        haps.append((bytes(hap), bytes(pd)))
+    reads = [_read(rng, R, haps[k % len(haps)][0]) for k, R in enumerate((1, 60, 130, 150))]
+    _check(reads, haps, f"column codes, {hap_len} bases")
+
+
 def test_long_haplotypes_and_reads():
     rng = np.random.default_rng(12)
     haps = [_pd_haplotype(rng, H, 8, 5) for H in (1000, 1500, 2000)]
