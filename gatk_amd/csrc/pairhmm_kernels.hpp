@@ -266,6 +266,7 @@ struct SwBatch {
     int32_t match, mismatch, open, extend;  // SWParameters
     int32_t strategy;                       // 0 SOFTCLIP, 1 INDEL, 2 LEADING_INDEL, 3 IGNORE
     int32_t max_ref_len, max_alt_len;
+    bool split;                             // several waves per pair (sw_splits; a workgroup per pair)
     uint8_t *scratch;                       // per wave: four bits per cell for the traceback
     size_t scratch_per_wave;
     uint32_t *queue_head;                   // next pair to take, 0 before the launch
@@ -279,6 +280,7 @@ struct SwBatch {
 // but a clip consumes an indel or a run of matches) is read from the full list.
 constexpr int kSwShortElems = 16;
 int sw_max_ref_len();
+bool sw_splits(uint32_t n_pairs, int max_ref_len, int max_alt_len, int num_cus);
 size_t sw_scratch_bytes_per_wave(int max_ref_len, int max_alt_len);
 hipError_t launch_sw(const SwBatch &batch, uint32_t n_pairs, int grid_blocks, hipStream_t stream);
 

@@ -30,7 +30,7 @@
 // Bound by VALU issue: 19 K + 10 instructions a step.  20,000 reads of 100-250 bases against
 // haplotypes of 150-600: 1.30 ms (980 GCUPS), where one column per lane, gap lengths carried as
 // values, a 2-byte store and LDS round trips every step took 4.23 ms; one region's 81 reads, a wave
-// each: 132 us against 773.
+// each: 126 us against 773 (few pairs: sw_split_kernel).
 #include "pairhmm_device.hpp"
 #include "pairhmm_kernels.hpp"
 
@@ -104,8 +104,8 @@ __device__ __forceinline__ void append_gt(uint32_t &w, int32_t a, int32_t b) {
 // before it starts, row R after it ends).  kA: the owner lane's index of column A.
 template <int K, bool kRec, bool kGuard>
 __device__ __forceinline__ void sw_block(SwLane<K> &st, SwEnds &ends, const SwBatch &b, const uint8_t *lref,
-                                         SwScore *recs, uint32_t *out, int lane, int t0, int R, int kA,
-                                         bool gap_edges) {
+                                         const SwScore *rec_in, SwScore *rec_out, uint32_t *out, int lane, int t0, int R,
+                                         int kA, bool gap_edges) {
     using lds_u8 = const volatile __attribute__((address_space(3))) uint8_t;
     lds_u8 *rp = (lds_u8 *)(lref + kSwLow - lane);  // address-space cast: C-style only
     uint32_t base[kSwBlock];
@@ -114,7 +114,7 @@ __device__ __forceinline__ void sw_block(SwLane<K> &st, SwEnds &ends, const SwBa
     for (int u = 0; u < kSwBlock; ++u) base[u] = rp[t0 + u];
     if constexpr (kRec) {
 #pragma unroll
-        for (int u = 0; u < kSwBlock; ++u) in[u] = recs[kSwLow + t0 + u + 1];
+        for (int u = 0; u < kSwBlock; ++u) in[u] = rec_in[kSwLow + t0 + u + 1];
         __builtin_amdgcn_wave_barrier();
     }
     uint32_t words[sw_words(K)];
@@ -155,7 +155,7 @@ __device__ __forceinline__ void sw_block(SwLane<K> &st, SwEnds &ends, const SwBa
         ends.col_step = better ? t : ends.col_step;
         if constexpr (kRec) {
             // Rows outside 1..R land in the low and high slots, or on rows that a later lane rewrites.
-            SwScore *r = recs + kSwLow + i;
+            SwScore *r = rec_out + kSwLow + i;
             r->sw = left;
             r->bgh = bgh;
         }
@@ -169,6 +169,38 @@ __device__ __forceinline__ void sw_block(SwLane<K> &st, SwEnds &ends, const SwBa
     __builtin_memcpy(__builtin_assume_aligned(out, sw_words(K) * 4), words, sizeof(words));
 }
 
+// A stripe's lanes before its first step.
+template <int K>
+__device__ __forceinline__ SwLane<K> sw_lane_start(const SwBatch &b, const uint8_t *alt, int j0, int A, bool gap_edges) {
+    SwLane<K> st;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        st.up[k] = edge_score(j0 + k + 1, gap_edges, b.open, b.extend);
+        st.bgv[k] = kLowInit;
+        st.alt[k] = j0 + k < A ? alt[j0 + k] : 0xFFFFu;
+    }
+    st.left = edge_score(j0, gap_edges, b.open, b.extend);
+    st.bgh = kLowInit;
+    st.s_last = st.up[K - 1];
+    st.h_last = kLowInit;
+    return st;
+}
+
+// Bottom-row candidates of a stripe's lane (columns j0 + 1 .. j0 + K).
+template <int K>
+__device__ __forceinline__ void sw_bottom(SwEnds &ends, const SwLane<K> &st, int j0, int R, int A) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int j = j0 + k + 1;
+        const int d = R - j < 0 ? j - R : R - j;
+        if (j <= A && better_end(st.up[k], d, j, ends.bot_best, ends.bot_dist, ends.bot_col)) {
+            ends.bot_best = st.up[k];
+            ends.bot_dist = d;
+            ends.bot_col = j;
+        }
+    }
+}
+
 // All stripes of a pair: cell bits into bt, the end-point candidates into `ends`.
 template <int K, bool kRec>
 __device__ __forceinline__ void sw_matrix(const SwBatch &b, const uint8_t *lref, SwScore *recs, uint32_t *bt, const uint8_t *alt,
@@ -178,17 +210,7 @@ __device__ __forceinline__ void sw_matrix(const SwBatch &b, const uint8_t *lref,
     const int n_blocks = sw_blocks(R);
     for (int s = 0; s < n_stripes; ++s) {
         const int j0 = s * kCols + lane * K;  // this lane's columns are j0 + 1 .. j0 + K
-        SwLane<K> st;
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            st.up[k] = edge_score(j0 + k + 1, gap_edges, b.open, b.extend);
-            st.bgv[k] = kLowInit;
-            st.alt[k] = j0 + k < A ? alt[j0 + k] : 0xFFFFu;
-        }
-        st.left = edge_score(j0, gap_edges, b.open, b.extend);
-        st.bgh = kLowInit;
-        st.s_last = st.up[K - 1];
-        st.h_last = kLowInit;
+        SwLane<K> st = sw_lane_start<K>(b, alt, j0, A, gap_edges);
         const bool last = s == n_stripes - 1;
         const int kA = last ? (A - 1) % K : 0;
         SwEnds col;
@@ -196,25 +218,16 @@ __device__ __forceinline__ void sw_matrix(const SwBatch &b, const uint8_t *lref,
         for (int tb = 0; tb < n_blocks; ++tb) {
             const int t0 = tb * kSwBlock;
             if (t0 < kWave - 1 || t0 + kSwBlock > R)
-                sw_block<K, kRec, true>(st, col, b, lref, recs, out, lane, t0, R, kA, gap_edges);
+                sw_block<K, kRec, true>(st, col, b, lref, recs, recs, out, lane, t0, R, kA, gap_edges);
             else
-                sw_block<K, kRec, false>(st, col, b, lref, recs, out, lane, t0, R, kA, gap_edges);
+                sw_block<K, kRec, false>(st, col, b, lref, recs, recs, out, lane, t0, R, kA, gap_edges);
             out += kWave * sw_words(K);
         }
         if (last) {
             ends.col_best = col.col_best;
             ends.col_step = col.col_step;
         }
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            const int j = j0 + k + 1;
-            const int d = R - j < 0 ? j - R : R - j;
-            if (j <= A && better_end(st.up[k], d, j, ends.bot_best, ends.bot_dist, ends.bot_col)) {
-                ends.bot_best = st.up[k];
-                ends.bot_dist = d;
-                ends.bot_col = j;
-            }
-        }
+        sw_bottom<K>(ends, st, j0, R, A);
         __builtin_amdgcn_wave_barrier();
     }
 }
@@ -403,6 +416,112 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kLong ? 3
     }
 }
 
+// Few pairs: a workgroup of kSplitWaves waves per pair, one stripe of 64 K columns per wave, K the least
+// of 1, 2, 4 that covers the alternate.  Wave w runs kSplitLag blocks behind wave w - 1, whose lane 63 has then
+// stored the records of the rows that the block reads; a barrier a block keeps the distance.  The record
+// arrays are a ring: the last wave's records, which nobody reads, land on rows that wave 0 read long before.
+// The cell bits lie as the one-wave kernel lays out stripes of K columns a lane, and wave 0 walks them.
+//
+// A lone wave is bound by its own issue, 19 K + 10 instructions a step; here four SIMDs share a pair, and a
+// step is bound by the latency of its chain of about eight dependent instructions and, once a block, of
+// the LDS round trip behind the barrier.  One region's 81 reads of 100-250 by haplotypes of 150-460: 126 us
+// with a wave per pair, 94 us with this; 81 haplotypes of up to 612 by references of up to 696, whole
+// call: 448 us and 222 us.
+constexpr int kSplitWaves = 4;
+constexpr int kSplitLag = (kWave + 2 * kSwBlock - 2) / kSwBlock;  // row t + 8 is complete 70 steps after step t
+
+struct SwSplitLds {
+    SwScore *recs;      // kSplitWaves arrays of `stride` records
+    int stride;
+    SwEnds *ends;       // kSplitWaves x 64
+    uint8_t *ref;
+};
+
+// LDS is all that the waves exchange inside the sweep: the barrier waits for LDS alone, stores of cell bits
+// stay in flight.
+__device__ __forceinline__ void sw_split_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+template <int K>
+__device__ __forceinline__ void sw_split_pair(const SwBatch &b, const SwSplitLds &L, uint32_t *bt, uint32_t p, int lane,
+                                              int wave, int R, int A) {
+    const bool gap_edges = b.strategy == 1 || b.strategy == 2;
+    const int n_stripes = (A + K * kWave - 1) / (K * kWave), n_blocks = sw_blocks(R);
+    const int j0 = wave * K * kWave + lane * K;
+    SwLane<K> st = sw_lane_start<K>(b, b.alt_bases + b.alt_off[p], j0, A, gap_edges);
+    const int kA = wave == n_stripes - 1 ? (A - 1) % K : 0;
+    const SwScore *rec_in = L.recs + wave * L.stride;
+    SwScore *rec_out = L.recs + (wave + 1) % kSplitWaves * L.stride;
+    SwEnds ends;
+    uint32_t *out = bt + (static_cast<size_t>(wave) * n_blocks * kWave + lane) * sw_words(K);
+    const int rounds = n_blocks + kSplitLag * (n_stripes - 1);
+    for (int g = 0; g < rounds; ++g) {
+        sw_split_barrier();  // the first one also ends the staging of the reference and the edges
+        const int tb = g - kSplitLag * wave;
+        if (wave >= n_stripes || tb < 0 || tb >= n_blocks) continue;
+        const int t0 = tb * kSwBlock;
+        if (t0 < kWave - 1 || t0 + kSwBlock > R)
+            sw_block<K, true, true>(st, ends, b, L.ref, rec_in, rec_out, out, lane, t0, R, kA, gap_edges);
+        else
+            sw_block<K, true, false>(st, ends, b, L.ref, rec_in, rec_out, out, lane, t0, R, kA, gap_edges);
+        out += kWave * sw_words(K);
+    }
+    if (wave < n_stripes) sw_bottom<K>(ends, st, j0, R, A);
+    L.ends[wave * kWave + lane] = ends;
+    // The cell bits too have to be out before wave 0 reads them, past lines that its L1 may hold.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (wave != 0) return;
+    for (int w = 1; w < n_stripes; ++w) {
+        const SwEnds e = L.ends[w * kWave + lane];
+        if (better_end(e.bot_best, e.bot_dist, e.bot_col, ends.bot_best, ends.bot_dist, ends.bot_col)) {
+            ends.bot_best = e.bot_best;
+            ends.bot_dist = e.bot_dist;
+            ends.bot_col = e.bot_col;
+        }
+    }
+    const SwEnds last = L.ends[(n_stripes - 1) * kWave + lane];
+    ends.col_best = last.col_best;
+    ends.col_step = last.col_step;
+    sw_traceback<K>(b, bt, p, lane, R, A, ends);
+}
+
+__global__ __launch_bounds__(kSplitWaves *kWave) void sw_split_kernel(SwBatch b) {
+    extern __shared__ SwScore lds_sw[];
+    const int lane = static_cast<int>(threadIdx.x) % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+    SwSplitLds L;
+    L.recs = lds_sw;
+    L.stride = kSwLow + b.max_ref_len + kSwHigh;
+    L.ends = reinterpret_cast<SwEnds *>(lds_sw + kSplitWaves * L.stride);
+    L.ref = reinterpret_cast<uint8_t *>(L.ends + kSplitWaves * kWave);
+    const uint32_t p = blockIdx.x;
+    uint32_t *bt = reinterpret_cast<uint32_t *>(b.scratch + static_cast<size_t>(p) * b.scratch_per_wave);
+    const int R = __builtin_amdgcn_readfirstlane(b.ref_len[p]), A = __builtin_amdgcn_readfirstlane(b.alt_len[p]);
+    const uint8_t *ref = b.ref_bases + b.ref_off[p];
+    const bool gap_edges = b.strategy == 1 || b.strategy == 2;
+    for (int i = static_cast<int>(threadIdx.x); i <= R; i += kSplitWaves * kWave) {
+        if (i < R) L.ref[kSwLow + i] = ref[i];  // rows outside 1..R read leftovers
+        L.recs[kSwLow + i] = SwScore{edge_score(i, gap_edges, b.open, b.extend), kLowInit};
+    }
+    if (A > 2 * kSplitWaves * kWave)
+        sw_split_pair<4>(b, L, bt, p, lane, wave, R, A);
+    else if (A > kSplitWaves * kWave)
+        sw_split_pair<2>(b, L, bt, p, lane, wave, R, A);
+    else
+        sw_split_pair<1>(b, L, bt, p, lane, wave, R, A);
+}
+
+size_t sw_split_lds_bytes(int max_ref_len) {
+    const size_t rows = static_cast<size_t>(kSwLow + max_ref_len + kSwHigh);
+    return rows * (kSplitWaves * sizeof(SwScore) + 1) + kSplitWaves * kWave * sizeof(SwEnds);
+}
+
 }  // namespace
 
 int sw_max_ref_len() {
@@ -421,11 +540,34 @@ size_t sw_scratch_bytes_per_wave(int max_ref_len, int max_alt_len) {
            sizeof(uint32_t);
 }
 
+// Whether a batch takes the split kernel: its alternates fit (1,024 bases), its LDS allows two workgroups
+// a CU, and its pairs are few.  Whole calls with a wave per pair and split, alternates of up to 250: 256
+// pairs 162 / 131 us, 512 pairs 173 / 149, 640 pairs 178 / 177, 1,024 pairs 190 / 209.  Alternates of more than
+// one sweep (up to 612), where a lone wave runs its stripes one after another: 1,024 pairs 499 / 417 us,
+// 2,048 pairs 811 / 733.
+bool sw_splits(uint32_t n_pairs, int max_ref_len, int max_alt_len, int num_cus) {
+    const uint32_t per_cu = max_alt_len > kSwMaxCols * kWave ? 8u : 2u;
+    return n_pairs <= per_cu * static_cast<uint32_t>(num_cus) && max_alt_len <= kSplitWaves * kSwMaxCols * kWave &&
+           sw_split_lds_bytes(max_ref_len) <= max_lds_per_block() / 2;
+}
+
 hipError_t launch_sw(const SwBatch &batch, uint32_t n_pairs, int grid_blocks, hipStream_t stream) {
     if (n_pairs == 0) return hipSuccess;
     if (batch.max_ref_len > sw_max_ref_len() || grid_blocks < 1) return hipErrorInvalidValue;
     const size_t lds = sw_lds_bytes(batch.max_ref_len, batch.max_alt_len);
     if (lds > max_lds_per_block()) return hipErrorInvalidValue;
+    if (batch.split) {
+        // A workgroup per pair, each with a wave's scratch.
+        const size_t bytes = sw_split_lds_bytes(batch.max_ref_len);
+        if (bytes > max_lds_per_block() || batch.max_alt_len > kSplitWaves * kSwMaxCols * kWave ||
+            static_cast<uint32_t>(grid_blocks) < n_pairs)
+            return hipErrorInvalidValue;
+        if (bytes > 65536)
+            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(sw_split_kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+        hipLaunchKernelGGL(sw_split_kernel, dim3(n_pairs), dim3(kSplitWaves * kWave), bytes, stream, batch);
+        return hipGetLastError();
+    }
     auto launch = [&](auto kernel) {
         if (lds > 65536)
             (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,

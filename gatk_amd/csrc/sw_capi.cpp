@@ -154,6 +154,7 @@ int32_t sw_run_batch(pairhmm_context *ctx, int64_t n_pairs, const uint8_t *ref_b
     b.strategy = overhang_strategy;
     b.max_ref_len = max_r;
     b.max_alt_len = max_a;
+    b.split = waves == n_pairs && sw_splits(static_cast<uint32_t>(n_pairs), max_r, max_a, cus);
     b.scratch = ds + o_scratch;
     b.scratch_per_wave = per_wave;
     b.queue_head = reinterpret_cast<uint32_t *>(ds + o_head);

@@ -178,3 +178,28 @@ def test_sweep_edges(binding, strategy):
     print(f"[sw] edges strategy={strategy.name} pairs={len(refs)}", flush=True)
     for k, (r, a, g) in enumerate(zip(refs, alts, binding.align_batch(refs, alts, params, strategy))):
         assert g == oracle.sw_align(r, a, _p(params), strategy.name), (k, len(r), len(a))
+
+
+@pytest.mark.parametrize("strategy", list(SWOverhangStrategy))
+@pytest.mark.parametrize("longest", [64, 256, 512, 1024, 1025])
+def test_few_and_many_pairs(binding, strategy, longest):
+    """A batch of few pairs shares each pair among the waves of a workgroup (alternates of up to 1,024
+    bases), a batch of many takes a wave per pair: both equal the oracle, at the edges of a wave's columns
+    and of the lag between waves."""
+    rng = np.random.default_rng(100 + longest + int(strategy))
+    base = lambda n: bytes(np.frombuffer(b"ACGT", np.uint8)[rng.integers(0, 4, n)])  # noqa: E731
+    refs, alts = [], []
+    for A in sorted({1, longest // 4, longest // 4 + 1, longest // 2 + 1, longest - 1, longest}):
+        for R in (1, 8, 65, 129, 700):
+            ref = base(R)
+            refs.append(ref)
+            alts.append((ref[R // 3:] + base(A))[:A] if R > 1 else base(A))
+    left, right, mid = base(longest // 4), base(longest // 4), base(longest // 2)
+    refs += [left + right, left + mid + right, base(700) + left + right]
+    alts += [left + mid + right, left + right, left + right]
+    params = NEW_SW_PARAMETERS
+    print(f"[sw] few and many longest={longest} strategy={strategy.name} pairs={len(refs)}", flush=True)
+    want = [oracle.sw_align(r, a, _p(params), strategy.name) for r, a in zip(refs, alts)]
+    assert list(binding.align_batch(refs, alts, params, strategy)) == want
+    times = 2100 // len(refs)
+    assert list(binding.align_batch(refs * times, alts * times, params, strategy)) == want * times
