@@ -12,8 +12,8 @@
 // Schedule (one pair per wave, 64-row stripes with the forward kernel's anti-diagonal skew):
 //   1. Forward over all stripes, top down, with lane 0 fed its sums of the row above (A, B) by a
 //      side pass, saving in per-wave global scratch, for every stripe, lane 0's A / B planes and,
-//      every kTile wave-steps, five values per lane (M, I, D one step back; M, S two steps back)
-//      as a checkpoint.
+//      every kTile wave-steps, four values per lane (M, I, D one step back and the pre-prior sum of
+//      the next step) as a checkpoint.
 //   2. Adjoint over the stripes bottom up.  Wave-steps run in reverse, so with the same skew lane k
 //      finds lane k+1's adjoints from one and two steps earlier (DPP wave_shl:1); lane 63 takes the
 //      row below the stripe (its X and gI) from LDS planes that lane 0 of the stripe underneath
@@ -29,6 +29,7 @@
 //   the lane below and they are moved down one lane when a stripe ends.  The last-row seed
 //   (d L / d M(R,c) = d L / d I(R,c) = 1) enters as a virtual row R+1 with gI = 1, X = 0 and
 //   MM = GM = 0, MI = II = 1, which also makes rows beyond R pass the seed up unchanged.
+//   (grad_adjoint's plain steps carry X and gM times the row's GM.)
 //   Scaling: forward cells carry 2^120 (FP32) / 2^1020 (FP64); the FP32 adjoint seed is 2^sigma with
 //   sigma = 30 - ilogb(L_scaled) so every accumulated product stays inside FP32's range; pairs whose
 //   L_scaled is below the forward's rescue threshold (1e-28) go to the FP64 kernel, as in the
@@ -42,7 +43,7 @@ namespace {
 
 using namespace dev;
 
-constexpr int kCk = 5;  // checkpoint: M, I, D one step back and M, S two steps back
+constexpr int kCk = 4;  // checkpoint: M, I, D one step back and the pre-prior sum of the next step
 
 template <typename T>
 struct AdjointScale;
@@ -101,6 +102,36 @@ __device__ __forceinline__ Row<T> load_row(const GradBatch &g, int64_t ro, int R
     return w;
 }
 
+// Rows the plain adjoint takes: it divides by GM, by the match prior and by the mismatch prior.  The bounds
+// (gap continuation of Q0.3 and more, base quality between Q0.3 and Q70) keep these far from 0.
+template <typename T>
+__device__ __forceinline__ bool plain_row(const Row<T> &w) {
+    return w.GM >= T(0.0625) && w.pm >= T(0.0625) && w.px >= T(3e-8);
+}
+
+// a += x y in the lanes of `mask`.
+__device__ __forceinline__ void fma_masked(float &a, float x, float y, uint64_t mask) {
+    uint64_t on;
+    asm("s_and_saveexec_b64 %1, %4\n\tv_fmac_f32 %0, %2, %3\n\ts_mov_b64 exec, %1"
+        : "+v"(a), "=&s"(on)
+        : "v"(x), "v"(y), "s"(mask)
+        : "scc");
+}
+__device__ __forceinline__ void fma_masked(double &a, double x, double y, uint64_t mask) {
+    uint64_t on;
+    asm("s_and_saveexec_b64 %1, %4\n\tv_fmac_f64 %0, %2, %3\n\ts_mov_b64 exec, %1"
+        : "+v"(a), "=&s"(on)
+        : "v"(x), "v"(y), "s"(mask)
+        : "scc");
+}
+
+// Lanes read what other lanes stored: the compiler keeps LDS accesses on their side of this (the hardware
+// takes a wave's in order).
+__device__ __forceinline__ void lds_order() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+}
+
 template <typename T, int kCols>
 struct GradLds {
     uint8_t *hap;
@@ -109,10 +140,16 @@ struct GradLds {
                       // M plane, which the adjoint no longer needs (four planes per wave, not five).
 };
 
+// Slots of a plane or of the haplotype that a pair's steps reach, pads included.
+__device__ __forceinline__ int used_columns(int H) { return H + 2 * kLdsPad + 32; }
+
 template <int kCols>
 constexpr int grad_stride() { return lds_plane_stride(kCols); }
 
 constexpr int kGradPlanes = 4;
+// A tile of the adjoint reads its row-below values from columns t0 - 62 (X) and t0 - 63 (gI) on: with these
+// shifts of the planes both are 16-byte aligned (the plane stride holds 4 elements more than the columns).
+constexpr int kBxShift = 2, kBgShift = 3;
 
 template <typename T, int kCols>
 constexpr size_t grad_lds_per_wave() {
@@ -126,114 +163,94 @@ __device__ __forceinline__ GradLds<T, kCols> grad_carve(uint8_t *base) {
     w.bm = reinterpret_cast<T *>(base + kCols);
     w.bi = w.bm + grad_stride<kCols>();
     w.bs = w.bi + grad_stride<kCols>();
-    w.bg = w.bs + grad_stride<kCols>();
-    w.bx = w.bm;
+    w.bg = w.bs + grad_stride<kCols>() + kBgShift;
+    w.bx = w.bm + kBxShift;
     return w;
 }
 
-// Lane 0's sums of the row above (A = M(c-1) MM + S(c-1) GM, B = M(c) MI + I(c) II) from the boundary
-// planes, in place: A over S, B over I, highest columns first so every read of index j-1 precedes
-// its overwrite.  The row above is in bm / bi / bs; MM0..II0 are lane 0's row parameters.
+// Lane 0's sums of the row above from the boundary planes, in place and into the scratch (dst), over the
+// stripe's columns 0 .. steps - 1: over S at column c the sum that column c + 1 multiplies by its prior,
+// A(c+1) = M(c) MM + S(c) GM, and over I the column's own insertion sum, B(c) = M(c) MI + I(c) II.  The row
+// above is in bm / bi / bs; MM0..II0 are lane 0's row parameters.
 template <typename T, int kCols>
-__device__ __forceinline__ void side_pass(const GradLds<T, kCols> &L, int lane, T MM0, T GM0, T MI0, T II0) {
-    __builtin_amdgcn_wave_barrier();
-    for (int j0 = kCols - kWave; j0 >= 0; j0 -= kWave) {
-        const int j = j0 + lane;
-        const T mj = L.bm[j], ij = L.bi[j];
-        const T mp = j > 0 ? L.bm[j - 1] : T(0), sp = j > 0 ? L.bs[j - 1] : T(0);
-        __builtin_amdgcn_wave_barrier();
-        L.bs[j] = fma(sp, GM0, mp * MM0);
-        L.bi[j] = fma(ij, II0, mj * MI0);
-        __builtin_amdgcn_wave_barrier();
+__device__ __forceinline__ void side_pass(const GradLds<T, kCols> &L, T *dst, int lane, int steps, T MM0, T GM0, T MI0,
+                                          T II0) {
+    lds_order();
+    for (int c = lane; c < steps; c += kWave) {
+        const int j = kLdsPad + c;
+        const T mj = L.bm[j], ij = L.bi[j], sj = L.bs[j];
+        const T a = fma(sj, GM0, mj * MM0), b = fma(ij, II0, mj * MI0);
+        L.bs[j] = a;
+        L.bi[j] = b;
+        dst[c] = a;
+        dst[kCols + c] = b;
     }
+    lds_order();
 }
 
-// One forward step of every lane (rows of a 64-row stripe, lane k at column t - k).  Lane 0 takes
-// its sums of the row above from a0 / b0; the other lanes take lane k-1's values by DPP.  Returns
-// the pre-prior sum a (for the base-error adjoint); updates the rolling state.
-template <typename T, bool kHapHasN>
-__device__ __forceinline__ T fwd_step(const Row<T> &w, T px, uint32_t hb, T a0, T b0, bool is_first, T &m1, T &i1,
-                                      T &d1, T &s1, T &m2, T &s2, T &m_out, T &i_out, T &d_out, T &s_out, T &p_out) {
-    const bool match = (hb == w.base) || (kHapHasN && hb == 'N');
-    const T prior = match ? w.pm : px;
-    T a, i;
+// One forward step of every lane (rows of a 64-row stripe, lane k at column t - k).  `a` is the step's
+// pre-prior sum; it becomes the next step's, which takes what lane k-1 had one step back (so one value
+// is carried, and checkpointed, for the diagonal instead of two).  Lane 0 takes its sums of the row above
+// from a0 (next step's) / b0; the other lanes take lane k-1's values by DPP.
+template <typename T>
+__device__ __forceinline__ void fwd_step(const Row<T> &w, T prior, T a0, T b0, bool is_first, T &a, T &m1, T &i1, T &d1,
+                                         T &s1) {
+    const T m = a * prior;
+    T i;
     if constexpr (sizeof(T) == sizeof(float)) {
         a = a0;
         i = b0;
-        dpp_upper2(a, m2, w.MM, s2, w.GM, i, m1, w.MI, i1, w.II);
+        dpp_upper2(a, m1, w.MM, s1, w.GM, i, m1, w.MI, i1, w.II);
     } else {
-        a = fma(from_prev_lane(s2), w.GM, from_prev_lane(m2) * w.MM);
+        a = fma(from_prev_lane(s1), w.GM, from_prev_lane(m1) * w.MM);
         i = fma(from_prev_lane(i1), w.II, from_prev_lane(m1) * w.MI);
         a = is_first ? a0 : a;
         i = is_first ? b0 : i;
     }
-    const T m = a * prior;
     // D carried divided by MD: D(c) = D(c-1) DD + M(c-1) MD becomes d(c) = d(c-1) DD + M(c-1), and
     // S = I + MD d, one FMA each (rows past R have MD = DD = 0, so d = 0 and S = I there).
-    const T d = fma(d1, w.DD, m1);
-    const T sx = fma(d, w.MD, i);
-    m_out = m;
-    i_out = i;
-    d_out = d;
-    s_out = sx;
-    p_out = prior;
-    m2 = m1;
-    s2 = s1;
+    d1 = fma(d1, w.DD, m1);
+    s1 = fma(d1, w.MD, i);
     m1 = m;
     i1 = i;
-    d1 = d;
-    s1 = sx;
-    return a;
 }
 
-// One pair: forward with checkpoints, then the adjoint.  Returns nothing; writes the outputs.
-//
-// Stripes of 64 rows, lane k = read position 64 s + k; rows past R pass the row above down
-// (MI = II = 1), in the forward and in the adjoint.  Scratch per stripe: the state registers every
-// kTile steps (checkpoints) and lane 0's A / B planes of the stripe.
+// Wave-steps of stripe s: until its last row (row R in the last stripe) has passed column H.
+template <int kTile>
+__device__ __forceinline__ int stripe_steps(int s, int n_stripes, int H, int R) {
+    return round_up(H + (s == n_stripes - 1 ? R - s * kWave : kWave), kTile);
+}
+
+// Forward over all stripes, top down, with checkpoints and lane 0's A / B planes in the scratch.  Returns
+// whether every row allows the plain adjoint (plain_row).
 template <typename T, int kCols, int kTile, bool kHapHasN>
-__device__ void grad_pair(const GradBatch &g, const GradLds<T, kCols> &L, T *__restrict__ scratch, int lane,
-                          uint32_t pair, int H, int R, int64_t ro, double weight, const RescueSink &rs) {
-    constexpr int kStripe = kWave;
-    constexpr int kLag = kWave - 1;
-    const int n_stripes = (R + kStripe - 1) / kStripe;
-    const int steps = round_up(H + kWave, kTile);
-    const int n_tiles = steps / kTile;
-    T *ck = scratch;                                                        // [stripe][tile][kCk][64]
-    T *abp = scratch + static_cast<size_t>(g.max_stripes) * g.max_tiles * kCk * kWave;  // [stripe][2][kCols]
-    const T d0 = static_cast<T>(__builtin_ldexp(1.0, Scale<T>::kExp) / static_cast<double>(H));
+__device__ __forceinline__ bool grad_forward(const GradBatch &g, const GradLds<T, kCols> &L, T *ck, T *abp, int lane,
+                                             int n_stripes, int H, int R, int64_t ro) {
     using lds_u8 = const volatile __attribute__((address_space(3))) uint8_t;
     lds_u8 *hp = (lds_u8 *)(L.hap + kLdsPad - 1 - lane);  // address-space cast: C-style only
-    int lane_w = lane, lane_r = lane, lane_x = lane;
-    asm volatile("" : "+v"(lane_w), "+v"(lane_r), "+v"(lane_x));
+    int lane_r = lane;
+    asm volatile("" : "+v"(lane_r));
     const bool is_first = lane_r == 0;
-
-    // ---- 1. forward, top down --------------------------------------------------------------
+    bool plain = true;
     for (int s = 0; s < n_stripes; ++s) {
-        const Row<T> w = load_row<T>(g, ro, R, s * kStripe + lane, true);
+        const int p = s * kWave + lane;
+        const int steps = stripe_steps<kTile>(s, n_stripes, H, R);
+        const Row<T> w = load_row<T>(g, ro, R, p, true);
+        plain = plain && (p >= R || plain_row(w));
         const T px = w.n_read ? w.pm : w.px;
-        side_pass<T, kCols>(L, lane, rfl(w.MM), rfl(w.GM), rfl(w.MI), rfl(w.II));
-        {
-            T *dst = abp + static_cast<size_t>(s) * 2 * kCols;
-            for (int j = lane; j < kCols; j += kWave) {
-                dst[j] = L.bs[j];
-                dst[kCols + j] = L.bi[j];
-            }
-        }
-        T m1 = 0, i1 = 0, d1 = 0, s1 = 0, m2 = 0, s2 = 0;
-        // Every lane stores its M, I and S at its own column c = t - lane at step t (no one-lane exec
-        // mask in the step): lane 63 writes column c last, at step c + 63, so the planes end with its
-        // row, and lane 0 has read A, B of column c by step c, before any lane overwrites it.
-        using lds_t = __attribute__((address_space(3))) T;
-        lds_t *wm = (lds_t *)(L.bm + kLdsPad) - lane_w, *wi = (lds_t *)(L.bi + kLdsPad) - lane_w,
-              *wsp = (lds_t *)(L.bs + kLdsPad) - lane_w;
+        side_pass<T, kCols>(L, abp + static_cast<size_t>(s) * 2 * kCols, lane, steps, rfl(w.MM), rfl(w.GM), rfl(w.MI),
+                            rfl(w.II));
+        T m1 = 0, i1 = 0, d1 = 0, s1 = 0, a = 0;
+        // The stripe's last row goes to the planes once a tile, from its own lane (one exec mask a tile; lane 0
+        // has read A, B of a column 63 steps before).
+        const int row_lane = s == n_stripes - 1 ? R - 1 - s * kWave : kWave - 1;
+        T *wm = L.bm + kLdsPad - row_lane, *wi = L.bi + kLdsPad - row_lane, *wsp = L.bs + kLdsPad - row_lane;
         T *ckp = ck + static_cast<size_t>(s) * g.max_tiles * kCk * kWave + lane;
         for (int t0 = 0; t0 < steps; t0 += kTile) {
             ckp[0 * kWave] = m1;  // S one step back is I + D, recomputed on restore
             ckp[1 * kWave] = i1;
             ckp[2 * kWave] = d1;
-            ckp[3 * kWave] = m2;
-            ckp[4 * kWave] = s2;
+            ckp[3 * kWave] = a;
             ckp += kCk * kWave;
             T av[kTile], bv[kTile];
             __builtin_memcpy(av, __builtin_assume_aligned(L.bs + kLdsPad + t0, 16), sizeof(av));
@@ -241,22 +258,244 @@ __device__ void grad_pair(const GradBatch &g, const GradLds<T, kCols> &L, T *__r
             uint32_t hbs[kTile];
 #pragma unroll
             for (int u = 0; u < kTile; ++u) hbs[u] = hp[t0 + u];
-            __builtin_amdgcn_wave_barrier();
-            lds_t *wmb = wm + t0, *wib = wi + t0, *wsb = wsp + t0;
+            T mv[kTile], iv[kTile], sv[kTile];
 #pragma unroll
             for (int u = 0; u < kTile; ++u) {
-                T m, i, d, sx, pr;
-                fwd_step<T, kHapHasN>(w, px, hbs[u], av[u], bv[u], is_first, m1, i1, d1, s1, m2, s2, m, i, d, sx, pr);
-                wmb[u] = m;
-                wib[u] = i;
-                wsb[u] = sx;
+                const bool match = (hbs[u] == w.base) || (kHapHasN && hbs[u] == 'N');
+                fwd_step<T>(w, match ? w.pm : px, av[u], bv[u], is_first, a, m1, i1, d1, s1);
+                mv[u] = m1;
+                iv[u] = i1;
+                sv[u] = s1;
             }
+            lds_order();
+            if (lane == row_lane) {
+#pragma unroll
+                for (int u = 0; u < kTile; ++u) {
+                    wm[t0 + u] = mv[u];
+                    wi[t0 + u] = iv[u];
+                    wsp[t0 + u] = sv[u];
+                }
+            }
+            lds_order();
         }
         __builtin_amdgcn_wave_barrier();
     }
+    return __all(plain);
+}
+
+// Adjoint over the stripes, bottom up, from the seed row in the bx / bg planes; adds the weighted results.
+// kPlain: no 'N' in the haplotype and plain_row for every row.  The steps then carry X times the row's own GM
+// and gM times GM, constants folded into the row's factors: gS is the X below as it comes, one product
+// less a step.  And d L / d e(qb) comes from two sums, gM M over all cells and over the mismatches alone
+// (one FMA under the mismatch mask), as M = a prior and the prior is one of two values: no weighted copy of
+// a is selected, multiplied and kept.
+template <typename T, int kCols, int kTile, bool kPlain>
+__device__ __forceinline__ void grad_adjoint(const GradBatch &g, const GradLds<T, kCols> &L, const T *ck, const T *abp,
+                                             int lane, int n_stripes, int H, int R, int64_t ro, T seed, T d0,
+                                             double norm) {
+    constexpr int kLag = kWave - 1;
+    using lds_u8 = const volatile __attribute__((address_space(3))) uint8_t;
+    lds_u8 *hp = (lds_u8 *)(L.hap + kLdsPad - 1 - lane);  // address-space cast: C-style only
+    int lane_r = lane;
+    asm volatile("" : "+v"(lane_r));
+    const bool is_first = lane_r == 0;
+    const double dq = -0.23025850929940456840;  // d e(q)/dq = dq * e(q)
+    for (int s = n_stripes - 1; s >= 0; --s) {
+        const int p = s * kWave + lane;
+        const int steps = stripe_steps<kTile>(s, n_stripes, H, R), n_tiles = steps / kTile;
+        const Row<T> w = load_row<T>(g, ro, R, p, true);
+        const T px = w.n_read ? w.pm : w.px;
+        // Next row's MM, GM, MI, II: lane k+1's own; lane 63's is the first row of the stripe below
+        // (a pass-through row below the last stripe).
+        const int p_below = (s + 1) * kWave;
+        const Row<T> below = load_row<T>(g, ro, R, p_below, true);
+        const T MMn = wave_shl1(below.MM, w.MM), GMn = wave_shl1(below.GM, w.GM);
+        const T MIn = wave_shl1(below.MI, w.MI), IIn = wave_shl1(below.II, w.II);
+        // Factors of GM gM (plain); X of a row past R is 0.
+        const T kD = w.GM * w.MD, kI = w.GM * MIn, kX = p + 1 < R ? w.GM * (MMn / GMn) : T(0);
+        // Lane 0's A / B planes of this stripe, for the recompute.
+        {
+            const T *src = abp + static_cast<size_t>(s) * 2 * kCols;
+            lds_order();
+            for (int c = lane; c < steps; c += kWave) {
+                L.bs[kLdsPad + c] = src[c];
+                L.bi[kLdsPad + c] = src[kCols + c];
+            }
+            lds_order();
+        }
+        // Lane 63 reads X(r+1, c+1) and gI(r+1, c) of the row below, a tile's values at its start; lane 0
+        // leaves X and gI of this stripe's first row for the stripe above (column c = t at step t), at the
+        // tile's end, 62 steps and more after lane 63 has read the column (steps run in reverse).
+        const T *bxr = L.bx + kLdsPad - (kLag - 1), *bgr = L.bg + kLdsPad - kLag;
+        // (Of an alignment that the compiler does not see: 8-byte stores.  The scheduler lets the data registers
+        // of 16-byte LDS stores be overwritten within two instructions, which has stored wrong values.)
+        int off_w = kLdsPad;
+        asm volatile("" : "+v"(off_w));
+        T *bxw = L.bx + off_w, *bgw = L.bg + off_w;
+        // Rows past R hold the seed as soon as they are inside the columns; the last stripe's steps begin
+        // when its row R enters them.
+        T X1 = 0, X2 = 0, gI1 = (p >= R && steps - lane >= 1 && steps - lane <= H) ? seed : T(0), gD1 = 0;
+        T aMMn = 0, aGMn = 0, aMIn = 0, aIIn = 0, aMD = 0, aDD = 0;
+        T aE = 0;  // plain: the sum of GM gM M
+        T aMis = 0;  // plain: its part on mismatches
+        const T *ckbase = ck + static_cast<size_t>(s) * g.max_tiles * kCk * kWave + lane;
+        // Checkpoints are read one tile ahead so the global load overlaps the current tile.
+        T cur[kCk], nxt[kCk];
+#pragma unroll
+        for (int k = 0; k < kCk; ++k) cur[k] = ckbase[(static_cast<size_t>(n_tiles - 1) * kCk + k) * kWave];
+        for (int tile = n_tiles - 1; tile >= 0; --tile) {
+            const int t0 = tile * kTile;
+            const int prev = tile > 0 ? tile - 1 : 0;
+#pragma unroll
+            for (int k = 0; k < kCk; ++k) nxt[k] = ckbase[(static_cast<size_t>(prev) * kCk + k) * kWave];
+            T m1 = cur[0], i1 = cur[1], d1 = cur[2], a = cur[3];
+            T s1 = fma(d1, w.MD, i1);
+            const T m_before = m1, d_before = d1;
+            T av[kTile], bv[kTile];
+            __builtin_memcpy(av, __builtin_assume_aligned(L.bs + kLdsPad + t0, 16), sizeof(av));
+            __builtin_memcpy(bv, __builtin_assume_aligned(L.bi + kLdsPad + t0, 16), sizeof(bv));
+            uint32_t hbs[kTile];
+#pragma unroll
+            for (int u = 0; u < kTile; ++u) hbs[u] = hp[t0 + u];
+            __builtin_amdgcn_wave_barrier();
+            T stM[kTile], stI[kTile], stD[kTile], stS[kTile], stP[kTile], stAW[kTile];
+            uint64_t mis[kTile];
+#pragma unroll
+            for (int u = 0; u < kTile; ++u) {
+                if constexpr (kPlain) {
+                    const bool differs = hbs[u] != w.base;
+                    mis[u] = __ballot(differs);
+                    stP[u] = differs ? px : w.pm;
+                } else {
+                    const bool hit = hbs[u] == w.base || hbs[u] == 'N';
+                    stP[u] = hit ? w.pm : px;
+                    stAW[u] = a * ((hit || w.n_read) ? T(-1) : T(1) / T(3));  // times d prior / d e(qb)
+                }
+                fwd_step<T>(w, stP[u], av[u], bv[u], is_first, a, m1, i1, d1, s1);
+                stM[u] = m1;
+                stI[u] = i1;
+                stD[u] = d1;
+                stS[u] = s1;
+            }
+            T xv[kTile], gv[kTile];
+            __builtin_memcpy(xv, __builtin_assume_aligned(bxr + t0, 16), sizeof(xv));
+            __builtin_memcpy(gv, __builtin_assume_aligned(bgr + t0, 16), sizeof(gv));
+            T xw[kTile], gw[kTile];
+#pragma unroll
+            for (int u = kTile - 1; u >= 0; --u) {
+                const T Xn2 = wave_shl1(xv[u], X2);   // X(r+1, c+1); plain: times GM of row r+1
+                const T gIn1 = wave_shl1(gv[u], gI1); // gI(r+1, c)
+                const T gS = kPlain ? Xn2 : GMn * Xn2;
+                const T gD = fma(w.DD, gD1, gS);
+                const T gI = fma(IIn, gIn1, gS);
+                const T gM = kPlain ? fma(kD, gD1, fma(kI, gIn1, kX * Xn2)) : fma(w.MD, gD1, fma(MIn, gIn1, MMn * Xn2));
+                const T X = stP[u] * gM;
+                const T Mp = (u > 0) ? stM[u - 1] : m_before;
+                const T Dp = (u > 0) ? stD[u - 1] : d_before;
+                aMMn = fma(Xn2, stM[u], aMMn);
+                aGMn = fma(Xn2, stS[u], aGMn);
+                aMIn = fma(gIn1, stM[u], aMIn);
+                aIIn = fma(gIn1, stI[u], aIIn);
+                aMD = fma(gD, Mp, aMD);
+                aDD = fma(gD, Dp, aDD);
+                if constexpr (kPlain) {
+                    aE = fma(gM, stM[u], aE);
+                    fma_masked(aMis, gM, stM[u], mis[u]);
+                } else {
+                    aE = fma(gM, stAW[u], aE);
+                }
+                xw[u] = X;
+                gw[u] = gI;
+                X2 = X1;
+                X1 = X;
+                gI1 = gI;
+                gD1 = gD;
+            }
+            lds_order();
+            if (lane == 0) {
+#pragma unroll
+                for (int u = 0; u < kTile; ++u) {
+                    bxw[t0 + u] = xw[u];
+                    bgw[t0 + u] = gw[u];
+                }
+            }
+            lds_order();
+#pragma unroll
+            for (int k = 0; k < kCk; ++k) cur[k] = nxt[k];
+        }
+        __builtin_amdgcn_wave_barrier();
+        // The next-row sums belong to the lane below: shift them down one lane.  Lane 63's belong to
+        // the first row of the stripe below; lane 0's own next-row terms come from the stripe above
+        // (or, for row 1, from row 0: S(0, c) = d0, so d L / d GM_1 = d0 sum_c X(1, c)).
+        double gMM = static_cast<double>(wave_shr1(T(0), aMMn));
+        double gGM = static_cast<double>(wave_shr1(T(0), aGMn));
+        const double gMI = static_cast<double>(wave_shr1(T(0), aMIn));
+        const double gII = static_cast<double>(wave_shr1(T(0), aIIn));
+        if (p < R) {
+            const double ei = static_cast<double>(w.MI), ed = static_cast<double>(w.MD), ec = static_cast<double>(w.II);
+            const double eb = 1.0 - static_cast<double>(w.pm);
+            double gE = static_cast<double>(aE);
+            if constexpr (kPlain) {
+                const double per_gm = 1.0 / static_cast<double>(w.GM);
+                gMM *= per_gm;
+                gGM *= per_gm;
+                const double mis = w.n_read ? 0.0 : static_cast<double>(aMis), hit = gE - mis;
+                gE = (mis / (3.0 * static_cast<double>(w.px)) - hit / static_cast<double>(w.pm)) * per_gm;
+            }
+            const double d_ei = (-gMM + gMI) * norm, d_ed = (-gMM + static_cast<double>(aMD)) * norm;
+            // aDD sums gD times D / MD (the forward's scaled D): d L / d DD = MD aDD.
+            const double d_ec = (-gGM + gII + static_cast<double>(aDD) * ed) * norm;
+            const double d_eb = gE * norm;
+            atomicAdd(&g.g_qi[ro + p], d_ei * dq * ei);
+            atomicAdd(&g.g_qd[ro + p], d_ed * dq * ed);
+            atomicAdd(&g.g_qc[ro + p], d_ec * dq * ec);
+            atomicAdd(&g.g_qb[ro + p], d_eb * dq * eb);
+            if (g.g_eb) atomicAdd(&g.g_eb[ro + p], d_eb);
+        }
+        if (lane == kLag && p_below < R) {
+            const double ei = static_cast<double>(below.MI), ed = static_cast<double>(below.MD);
+            const double ec = static_cast<double>(below.II);
+            const double per_gm = kPlain ? 1.0 / static_cast<double>(below.GM) : 1.0;
+            const double mmn = static_cast<double>(aMMn) * per_gm, gmn = static_cast<double>(aGMn) * per_gm;
+            atomicAdd(&g.g_qi[ro + p_below], (-mmn + static_cast<double>(aMIn)) * norm * dq * ei);
+            atomicAdd(&g.g_qd[ro + p_below], -mmn * norm * dq * ed);
+            atomicAdd(&g.g_qc[ro + p_below], (-gmn + static_cast<double>(aIIn)) * norm * dq * ec);
+        }
+        if (s == 0) {
+            double sx = 0.0;
+            for (int c = 1 + lane; c <= H; c += kWave) sx += static_cast<double>(L.bx[kLdsPad + c]);
+            sx = wave_sum(sx);
+            if (lane == 0) {
+                const double ec = static_cast<double>(w.II);
+                const double per_gm = kPlain ? 1.0 / static_cast<double>(w.GM) : 1.0;
+                atomicAdd(&g.g_qc[ro], -static_cast<double>(d0) * sx * per_gm * norm * dq * ec);
+            }
+        }
+    }
+}
+
+// One pair: forward with checkpoints, then the adjoint.  Returns nothing; writes the outputs.
+//
+// Stripes of 64 rows, lane k = read position 64 s + k; rows past R pass the row above down
+// (MI = II = 1), in the forward and in the adjoint.  Scratch per stripe: the state registers every
+// kTile steps (checkpoints) and lane 0's A / B planes of the stripe.
+template <typename T, int kCols, int kTile>
+__device__ __forceinline__ void grad_pair(const GradBatch &g, const GradLds<T, kCols> &L, T *__restrict__ scratch, int lane,
+                                          uint32_t pair, int H, int R, int64_t ro, double weight, bool hap_has_n,
+                                          const RescueSink &rs) {
+    const int n_stripes = (R + kWave - 1) / kWave;
+    T *ck = scratch;                                                        // [stripe][tile][kCk][64]
+    T *abp = scratch + static_cast<size_t>(g.max_stripes) * g.max_tiles * kCk * kWave;  // [stripe][2][kCols]
+    const T d0 = static_cast<T>(__builtin_ldexp(1.0, Scale<T>::kExp) / static_cast<double>(H));
+    const bool plain_rows = hap_has_n ? grad_forward<T, kCols, kTile, true>(g, L, ck, abp, lane, n_stripes, H, R, ro)
+                                      : grad_forward<T, kCols, kTile, false>(g, L, ck, abp, lane, n_stripes, H, R, ro);
+    // A last stripe of fewer than 64 rows rounds M + I to T (as rows past R would pass it down).
     double acc = 0.0;
-    for (int c = 1 + lane; c <= H; c += kWave)
-        acc += static_cast<double>(L.bm[kLdsPad + c]) + static_cast<double>(L.bi[kLdsPad + c]);
+    const bool whole = R % kWave == 0;
+    for (int c = 1 + lane; c <= H; c += kWave) {
+        const T m = L.bm[kLdsPad + c], i = L.bi[kLdsPad + c];
+        acc += whole ? static_cast<double>(m) + static_cast<double>(i) : static_cast<double>(m + i);
+    }
     const double l_scaled = wave_sum(acc);
     const double scale_log10 = static_cast<double>(Scale<T>::kExp) * 0.30102999566398119521;
 
@@ -278,159 +517,19 @@ __device__ void grad_pair(const GradBatch &g, const GradLds<T, kCols> &L, T *__r
     if (!(l_scaled > 0.0)) return;  // FP64 underflow: log10 L = -inf, no gradient
     const T seed = static_cast<T>(__builtin_ldexp(1.0, sigma));
     const double norm = weight / (l_scaled * __builtin_ldexp(1.0, sigma) * 2.30258509299404568402);
-    const double dq = -0.23025850929940456840;  // d e(q)/dq = dq * e(q)
 
     // Adjoint boundary below the last stripe: the seed row (gI = seed on columns 1..H, X = 0).  X
     // shares the M plane that the sum above just read.
     __builtin_amdgcn_wave_barrier();
-    for (int j = lane; j < kCols; j += kWave) {
+    for (int j = lane; j < used_columns(H); j += kWave) {
         const int c = j - kLdsPad;
         L.bx[j] = 0;
         L.bg[j] = (c >= 1 && c <= H) ? seed : T(0);
     }
-
-    // ---- 2. adjoint, bottom up -------------------------------------------------------------------
-    for (int s = n_stripes - 1; s >= 0; --s) {
-        const int p = s * kStripe + lane;
-        const Row<T> w = load_row<T>(g, ro, R, p, true);
-        const T px = w.n_read ? w.pm : w.px;
-        // Next row's MM, GM, MI, II: lane k+1's own; lane 63's is the first row of the stripe below
-        // (a pass-through row below the last stripe).
-        const int p_below = (s + 1) * kStripe;
-        const Row<T> below = load_row<T>(g, ro, R, p_below, true);
-        const T MMn = wave_shl1(below.MM, w.MM), GMn = wave_shl1(below.GM, w.GM);
-        const T MIn = wave_shl1(below.MI, w.MI), IIn = wave_shl1(below.II, w.II);
-        // Lane 0's A / B planes of this stripe, for the recompute.
-        {
-            const T *src = abp + static_cast<size_t>(s) * 2 * kCols;
-            __builtin_amdgcn_wave_barrier();
-            for (int j = lane; j < kCols; j += kWave) {
-                L.bs[j] = src[j];
-                L.bi[j] = src[kCols + j];
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-        // Lane 63 reads X(r+1, c+1) and gI(r+1, c) of the row below; lane 0 leaves X and gI of this
-        // stripe's first row for the stripe above (column c = t at step t).  Steps run in reverse, and
-        // every lane stores at its own column c = t - lane (no one-lane exec mask in the step): a
-        // column's stores come after lane 63 has read it, and lane 0's, at step c, come last.  Lane
-        // 63's X store alone would land before its own read of that column one step later; it goes
-        // one column right, onto the column it has just read.
-        // Volatile: single-dword LDS accesses at immediate offsets (paired ds_read2 / ds_write2 forms
-        // cannot reach the planes' offsets and cost an address add each).
-        using lds_t = volatile __attribute__((address_space(3))) T;
-        const lds_t *bxr = (const lds_t *)(L.bx + kLdsPad - (kLag - 1)), *bgr = (const lds_t *)(L.bg + kLdsPad - kLag);
-        lds_t *bxw = (lds_t *)(L.bx + kLdsPad) - lane_x + (lane_x == kLag ? 1 : 0);
-        lds_t *bgw = (lds_t *)(L.bg + kLdsPad) - lane_x;
-        T X1 = 0, X2 = 0, gI1 = 0, gD1 = 0;
-        T aMMn = 0, aGMn = 0, aMIn = 0, aIIn = 0, aMD = 0, aDD = 0, aE = 0;
-        const T *ckbase = ck + static_cast<size_t>(s) * g.max_tiles * kCk * kWave + lane;
-        // Checkpoints are read one tile ahead so the global load overlaps the current tile.
-        T cur[kCk], nxt[kCk];
-#pragma unroll
-        for (int k = 0; k < kCk; ++k) cur[k] = ckbase[(static_cast<size_t>(n_tiles - 1) * kCk + k) * kWave];
-        for (int tile = n_tiles - 1; tile >= 0; --tile) {
-            const int t0 = tile * kTile;
-            const int prev = tile > 0 ? tile - 1 : 0;
-#pragma unroll
-            for (int k = 0; k < kCk; ++k) nxt[k] = ckbase[(static_cast<size_t>(prev) * kCk + k) * kWave];
-            T m1 = cur[0], i1 = cur[1], d1 = cur[2], m2 = cur[3], s2 = cur[4];
-            T s1 = fma(d1, w.MD, i1);
-            const T m_before = m1, d_before = d1;
-            T av[kTile], bv[kTile];
-            __builtin_memcpy(av, __builtin_assume_aligned(L.bs + kLdsPad + t0, 16), sizeof(av));
-            __builtin_memcpy(bv, __builtin_assume_aligned(L.bi + kLdsPad + t0, 16), sizeof(bv));
-            uint32_t hbs[kTile];
-#pragma unroll
-            for (int u = 0; u < kTile; ++u) hbs[u] = hp[t0 + u];
-            // Lane 63's row-below values of the tile, read at its start: column c of the X plane is
-            // stored by lane k at step c + k (lane 63 at step c + 62, after its read there), and of
-            // the gI plane at step c + k, so no store of the tile reaches a column before the step
-            // that reads it (steps run t0 + kTile - 1 down to t0).
-            T xv[kTile], gv[kTile];
-#pragma unroll
-            for (int u = 0; u < kTile; ++u) {
-                xv[u] = bxr[t0 + u];
-                gv[u] = bgr[t0 + u];
-            }
-            __builtin_amdgcn_wave_barrier();
-            T stM[kTile], stI[kTile], stD[kTile], stS[kTile], stP[kTile], stAW[kTile];
-#pragma unroll
-            for (int u = 0; u < kTile; ++u) {
-                const T a = fwd_step<T, kHapHasN>(w, px, hbs[u], av[u], bv[u], is_first, m1, i1, d1, s1, m2, s2,
-                                                  stM[u], stI[u], stD[u], stS[u], stP[u]);
-                const bool hit = (hbs[u] == w.base) || (kHapHasN && hbs[u] == 'N');
-                const T wgt = (hit || w.n_read) ? T(-1) : T(1) / T(3);  // d prior / d e(qb)
-                stAW[u] = a * wgt;
-            }
-#pragma unroll
-            for (int u = kTile - 1; u >= 0; --u) {
-                const int t = t0 + u;
-                const T Xn2 = wave_shl1(xv[u], X2);   // X(r+1, c+1)
-                const T gIn1 = wave_shl1(gv[u], gI1); // gI(r+1, c)
-                const T gS = GMn * Xn2;
-                const T gD = fma(w.DD, gD1, gS);
-                const T gI = fma(IIn, gIn1, gS);
-                const T gM = fma(w.MD, gD1, fma(MIn, gIn1, MMn * Xn2));
-                const T X = stP[u] * gM;
-                const T Mp = (u > 0) ? stM[u - 1] : m_before;
-                const T Dp = (u > 0) ? stD[u - 1] : d_before;
-                aMMn = fma(Xn2, stM[u], aMMn);
-                aGMn = fma(Xn2, stS[u], aGMn);
-                aMIn = fma(gIn1, stM[u], aMIn);
-                aIIn = fma(gIn1, stI[u], aIIn);
-                aMD = fma(gD, Mp, aMD);
-                aDD = fma(gD, Dp, aDD);
-                aE = fma(gM, stAW[u], aE);
-                bxw[t] = X;
-                bgw[t] = gI;
-                X2 = X1;
-                X1 = X;
-                gI1 = gI;
-                gD1 = gD;
-            }
-#pragma unroll
-            for (int k = 0; k < kCk; ++k) cur[k] = nxt[k];
-        }
-        __builtin_amdgcn_wave_barrier();
-        // The next-row sums belong to the lane below: shift them down one lane.  Lane 63's belong to
-        // the first row of the stripe below; lane 0's own next-row terms come from the stripe above
-        // (or, for row 1, from row 0: S(0, c) = d0, so d L / d GM_1 = d0 sum_c X(1, c)).
-        const double gMM = static_cast<double>(wave_shr1(T(0), aMMn));
-        const double gGM = static_cast<double>(wave_shr1(T(0), aGMn));
-        const double gMI = static_cast<double>(wave_shr1(T(0), aMIn));
-        const double gII = static_cast<double>(wave_shr1(T(0), aIIn));
-        if (p < R) {
-            const double ei = static_cast<double>(w.MI), ed = static_cast<double>(w.MD), ec = static_cast<double>(w.II);
-            const double eb = 1.0 - static_cast<double>(w.pm);
-            const double d_ei = (-gMM + gMI) * norm, d_ed = (-gMM + static_cast<double>(aMD)) * norm;
-            // aDD sums gD times D / MD (the forward's scaled D): d L / d DD = MD aDD.
-            const double d_ec = (-gGM + gII + static_cast<double>(aDD) * ed) * norm;
-            const double d_eb = static_cast<double>(aE) * norm;
-            atomicAdd(&g.g_qi[ro + p], d_ei * dq * ei);
-            atomicAdd(&g.g_qd[ro + p], d_ed * dq * ed);
-            atomicAdd(&g.g_qc[ro + p], d_ec * dq * ec);
-            atomicAdd(&g.g_qb[ro + p], d_eb * dq * eb);
-            if (g.g_eb) atomicAdd(&g.g_eb[ro + p], d_eb);
-        }
-        if (lane == kLag && p_below < R) {
-            const double ei = static_cast<double>(below.MI), ed = static_cast<double>(below.MD);
-            const double ec = static_cast<double>(below.II);
-            const double mmn = static_cast<double>(aMMn);
-            atomicAdd(&g.g_qi[ro + p_below], (-mmn + static_cast<double>(aMIn)) * norm * dq * ei);
-            atomicAdd(&g.g_qd[ro + p_below], -mmn * norm * dq * ed);
-            atomicAdd(&g.g_qc[ro + p_below], (-static_cast<double>(aGMn) + static_cast<double>(aIIn)) * norm * dq * ec);
-        }
-        if (s == 0) {
-            double sx = 0.0;
-            for (int c = 1 + lane; c <= H; c += kWave) sx += static_cast<double>(L.bx[kLdsPad + c]);
-            sx = wave_sum(sx);
-            if (lane == 0) {
-                const double ec = static_cast<double>(w.II);
-                atomicAdd(&g.g_qc[ro], -static_cast<double>(d0) * sx * norm * dq * ec);
-            }
-        }
-    }
+    if (plain_rows && !hap_has_n)
+        grad_adjoint<T, kCols, kTile, true>(g, L, ck, abp, lane, n_stripes, H, R, ro, seed, d0, norm);
+    else
+        grad_adjoint<T, kCols, kTile, false>(g, L, ck, abp, lane, n_stripes, H, R, ro, seed, d0, norm);
 }
 
 template <typename T, int kCols, int kTile>
@@ -445,12 +544,12 @@ __device__ void grad_process(const GradBatch &g, const RescueSink &rs, uint8_t *
     // outside those bounds (or with an empty haplotype) gets NaN instead of touching memory.
     const int n_stripes = (R + kWave - 1) / kWave;
     const int n_tiles = round_up(H + kWave, kTile) / kTile;
-    if (H <= 0 || H + 2 * kLdsPad + 32 > kCols || n_stripes > g.max_stripes || n_tiles > g.max_tiles) {
+    if (H <= 0 || used_columns(H) > kCols || n_stripes > g.max_stripes || n_tiles > g.max_tiles) {
         g.out_log10[pair] = __builtin_nan("");
         return;
     }
     int has_n = 0;
-    for (int j = lane; j < kCols; j += kWave) {
+    for (int j = lane; j < used_columns(H); j += kWave) {
         const int c = j - kLdsPad + 1;
         uint8_t v = 0;
         if (c >= 1 && c <= H) {
@@ -460,7 +559,7 @@ __device__ void grad_process(const GradBatch &g, const RescueSink &rs, uint8_t *
         L.hap[j] = v;
     }
     const T d0 = static_cast<T>(__builtin_ldexp(1.0, Scale<T>::kExp) / static_cast<double>(H));
-    for (int j = lane; j < kCols; j += kWave) {
+    for (int j = lane; j < used_columns(H); j += kWave) {
         L.bm[j] = 0;
         L.bi[j] = 0;
         L.bs[j] = j >= kLdsPad ? d0 : T(0);
@@ -469,10 +568,7 @@ __device__ void grad_process(const GradBatch &g, const RescueSink &rs, uint8_t *
         g.out_log10[pair] = -__builtin_inf();
         return;
     }
-    if (__any(has_n))
-        grad_pair<T, kCols, kTile, true>(g, L, scratch, lane, pair, H, R, ro, weight, rs);
-    else
-        grad_pair<T, kCols, kTile, false>(g, L, scratch, lane, pair, H, R, ro, weight, rs);
+    grad_pair<T, kCols, kTile>(g, L, scratch, lane, pair, H, R, ro, weight, __any(has_n) != 0, rs);
 }
 
 template <typename T, int kCols, int kTile>
@@ -495,8 +591,14 @@ __device__ __forceinline__ void grad_loop(const GradBatch &g, const WorkSource &
     }
 }
 
-// FP32: held to 168 VGPRs (three waves per SIMD; the few values the allocator then keeps in scratch
-// are reloaded once per stripe, outside the step loops).
+// FP32: bound by VALU issue (91-93 % busy: 35 instructions a step of a 64-row stripe, 1.36 steps for each cell
+// that rows past R and the stripes' fill and drain leave useful) and close to it by the checkpoints' HBM
+// traffic (3 TB/s).  100 regions of reads of 100-250 by haplotypes of 136-607, 519,357 pairs, forward,
+// backward and autograd around them: 61.6 ms with 5 checkpoint values every 8 steps, planes written by every
+// lane every step and 40 instructions; 57.5 with the plain adjoint's sums and the shorter last stripe,
+// 54.2 with 4 values and the planes written once a tile, 50.6 with tiles of 12.  Held to 168 VGPRs, three
+// waves per SIMD (the values the allocator then keeps in scratch are reloaded outside the step loops);
+// two waves measured 58.0 (tiles of 12) and 57.0 (16), three waves with tiles of 16 spill inside the loops.
 template <int kCols, int kTile>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void grad_kernel_f32(GradBatch g, WorkSource ws,
                                                                                               RescueSink rs) {
@@ -580,7 +682,7 @@ hipError_t with_grad_kernel(bool fp64, int cols, F &&f) {
         if constexpr (kC > kMaxGradCols) {
             return hipErrorInvalidValue;
         } else {
-            return fp64 ? f(grad_kernel_f64<kC, kGradTile>) : f(grad_kernel_f32<kC, kGradTile>);
+            return fp64 ? f(grad_kernel_f64<kC, kGradTile>) : f(grad_kernel_f32<kC, kGradTileF32>);
         }
     });
 }
