@@ -155,7 +155,10 @@ extern "C" int32_t pairhmm_compute_likelihoods(pairhmm_context *ctx, const pairh
     const size_t total = off;
 
     HIP_TRY(hipSetDevice(ctx->device), PAIRHMM_ERR_KERNEL);
-    if (ctx->stage_host.reserve(in_bytes) != hipSuccess) return fail(PAIRHMM_ERR_OOM, "pinned staging allocation failed");
+    const size_t out_bytes = sizeof(double) * static_cast<size_t>(n_pairs);
+    const bool to_host = out_bytes <= kHostResultBytes;
+    if (ctx->stage_host.reserve(std::max(in_bytes, to_host ? out_bytes : 0)) != hipSuccess)
+        return fail(PAIRHMM_ERR_OOM, "pinned staging allocation failed");
     if (ctx->stage_dev.reserve(total) != hipSuccess) return fail(PAIRHMM_ERR_OOM, "device staging allocation failed");
     uint8_t *hs = static_cast<uint8_t *>(ctx->stage_host.ptr);
     int64_t *roff = reinterpret_cast<int64_t *>(hs + o_roff);
@@ -211,7 +214,7 @@ extern "C" int32_t pairhmm_compute_likelihoods(pairhmm_context *ctx, const pairh
     b.pair_read = nullptr;  // implicit read-major pairs
     b.pair_hap = nullptr;
     b.n_haps = n_haps;
-    b.out = reinterpret_cast<double *>(ds + o_out);
+    b.out = reinterpret_cast<double *>(to_host ? hs : ds + o_out);
     DeviceTables tab{ctx->d_qual_err, ctx->d_mm_prob};
     uint32_t *counters = reinterpret_cast<uint32_t *>(ds + o_cnt);
     uint32_t *rescue = reinterpret_cast<uint32_t *>(ds + o_rescue);
@@ -252,9 +255,10 @@ extern "C" int32_t pairhmm_compute_likelihoods(pairhmm_context *ctx, const pairh
         WorkSource again{rescue, 0, counters + 1, nullptr};
         HIP_TRY(launch_forward(true, b, tab, again, none, max_h, sh64, grid64, ctx->stream), PAIRHMM_ERR_KERNEL);
     }
-    HIP_TRY(hipMemcpyAsync(likelihoods, b.out, sizeof(double) * n_pairs, hipMemcpyDeviceToHost, ctx->stream),
-            PAIRHMM_ERR_KERNEL);
+    if (!to_host)
+        HIP_TRY(hipMemcpyAsync(likelihoods, b.out, out_bytes, hipMemcpyDeviceToHost, ctx->stream), PAIRHMM_ERR_KERNEL);
     HIP_TRY(hipStreamSynchronize(ctx->stream), PAIRHMM_ERR_KERNEL);
+    if (to_host) std::memcpy(likelihoods, hs, out_bytes);
     return PAIRHMM_OK;
 }
 

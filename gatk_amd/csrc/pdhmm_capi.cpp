@@ -161,7 +161,9 @@ extern "C" int32_t pairhmm_pd_compute_likelihoods(pairhmm_context *ctx, const pa
     b.n_haps = n_haps;
     b.tristate = 1;
     b.odd_bases = reinterpret_cast<const uint32_t *>(ds + o_odd);
-    b.out = reinterpret_cast<double *>(ds + o_out);
+    const size_t out_bytes = sizeof(double) * static_cast<size_t>(n_pairs);
+    const bool to_host = out_bytes <= kHostResultBytes;
+    b.out = reinterpret_cast<double *>(to_host ? hs : ds + o_out);
     DeviceTables tab{ctx->d_qual_err, ctx->d_mm_prob};
     // One wave per workgroup and per pair; the hardware dispatcher balances uneven pairs.
     const int grid = static_cast<int>(std::min<int64_t>(n_pairs, 1 << 20));
@@ -169,10 +171,10 @@ extern "C" int32_t pairhmm_pd_compute_likelihoods(pairhmm_context *ctx, const pa
                             reinterpret_cast<uint32_t *>(ds + o_odd), ctx->stream),
             PAIRHMM_ERR_KERNEL);
     HIP_TRY(launch_pd_forward(b, tab, static_cast<uint32_t>(n_pairs), max_h, grid, ctx->stream), PAIRHMM_ERR_KERNEL);
-    HIP_TRY(hipMemcpyAsync(hs, ds + o_out, sizeof(double) * n_pairs, hipMemcpyDeviceToHost, ctx->stream),
-            PAIRHMM_ERR_KERNEL);
+    if (!to_host)
+        HIP_TRY(hipMemcpyAsync(hs, ds + o_out, out_bytes, hipMemcpyDeviceToHost, ctx->stream), PAIRHMM_ERR_KERNEL);
     HIP_TRY(hipStreamSynchronize(ctx->stream), PAIRHMM_ERR_KERNEL);
-    std::memcpy(likelihoods, hs, sizeof(double) * n_pairs);
+    std::memcpy(likelihoods, hs, out_bytes);
     return PAIRHMM_OK;
 }
 

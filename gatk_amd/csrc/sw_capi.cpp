@@ -160,13 +160,16 @@ int32_t sw_run_batch(pairhmm_context *ctx, int64_t n_pairs, const uint8_t *ref_b
     b.queue_head = reinterpret_cast<uint32_t *>(ds + o_head);
     b.elems = reinterpret_cast<uint32_t *>(ds + o_elems);
     b.elem_off = reinterpret_cast<const int64_t *>(ds + o_eoff);
-    b.elems_short = reinterpret_cast<uint32_t *>(ds + o_short);
-    b.n_elems = reinterpret_cast<int32_t *>(ds + o_n);
-    b.offset = reinterpret_cast<int32_t *>(ds + o_off);
+    const bool to_host = out_bytes <= kHostResultBytes;
+    uint8_t *results = to_host ? hs : ds + out_begin;
+    b.elems_short = reinterpret_cast<uint32_t *>(results);
+    b.n_elems = reinterpret_cast<int32_t *>(results + (o_n - out_begin));
+    b.offset = reinterpret_cast<int32_t *>(results + (o_off - out_begin));
     HIP_TRY(launch_sw(b, static_cast<uint32_t>(n_pairs), static_cast<int>(waves), ctx->stream), PAIRHMM_ERR_KERNEL);
     // The input staging (in_bytes) has been consumed by the copy above before the kernel ran (same
     // stream), so the outputs can come back into the same pinned buffer.
-    HIP_TRY(hipMemcpyAsync(hs, ds + out_begin, out_bytes, hipMemcpyDeviceToHost, ctx->stream), PAIRHMM_ERR_KERNEL);
+    if (!to_host)
+        HIP_TRY(hipMemcpyAsync(hs, ds + out_begin, out_bytes, hipMemcpyDeviceToHost, ctx->stream), PAIRHMM_ERR_KERNEL);
     HIP_TRY(hipStreamSynchronize(ctx->stream), PAIRHMM_ERR_KERNEL);
     res.short_elems = reinterpret_cast<const uint32_t *>(hs);
     res.n_el = reinterpret_cast<const int32_t *>(hs + (o_n - out_begin));

@@ -518,3 +518,28 @@ def test_concurrent_contexts():
         t.join()
     assert not errors
     assert np.array_equal(results[0], results[1]) and np.array_equal(results[0], results[2])
+
+
+@pytest.mark.parametrize("use_double", [False, True])
+@pytest.mark.parametrize("n_reads", [1, 511, 512, 513])
+def test_results_on_both_sides_of_the_direct_store(n_reads, use_double):
+    """512 haplotypes: up to 512 reads (2 MB) the kernels store a call's results in pinned host memory, above
+    it they are copied back; the first rows equal the oracle either way and every result is written."""
+    rng = np.random.default_rng(12)
+    haps = [rng.choice(list(b"ACGT"), int(H)).astype(np.uint8) for H in rng.integers(8, 30, 512)]
+    reads = []
+    for k in range(n_reads):
+        R = int(rng.integers(1, 12))
+        reads.append((haps[k % 512][:R].copy() if R <= len(haps[k % 512]) else rng.choice(list(b"ACGT"), R).astype(np.uint8),
+                      *(rng.integers(10, 41, R).astype(np.uint8) for _ in range(4))))
+    binding = _binding(use_double)
+    out = np.full(n_reads * 512, np.nan)
+    try:
+        binding.compute_likelihoods([ReadDataHolder(*r) for r in reads], [HaplotypeDataHolder(h) for h in haps], out)
+    finally:
+        binding.done()
+    out = out.reshape(n_reads, 512)
+    assert np.isfinite(out).all()
+    rows = sorted({0, n_reads // 2, n_reads - 1})
+    want = oracle.logless_batch(pack_regions([(haps, [reads[r] for r in rows])]), n_threads=8).reshape(len(rows), 512)
+    assert np.max(np.abs(out[rows] - want)) <= (FP64_TOL if use_double else FP32_TOL)
