@@ -887,6 +887,9 @@ __device__ __forceinline__ void packed_block(PackedState &st, const RowTrans<flo
         const float sx = fmaf(w.MD, d, i);
         wm[u] = m;
         wi[u] = i;
+        // A column's last store has to come last, and the lanes' stores to it belong to different steps: the
+        // compiler, which sees one lane, may pair two steps' stores but not reorder pairs.
+        if (u % 2 == 1) asm volatile("" ::: "memory");
         st.m2 = st.m1;
         st.s2 = st.s1;
         st.m1 = m;
@@ -896,13 +899,42 @@ __device__ __forceinline__ void packed_block(PackedState &st, const RowTrans<flo
     }
 }
 
+// A lane's haplotype bytes in LDS, four columns a word: aligned words, shifted to the lane's own byte.  Byte
+// loads, one a step, kept a packed launch's LDS 71 % busy beside 90 % of its VALU issue, and each waited
+// for the other: 300 regions 39.7 ms with them, 36.7 ms with words; 128,000 pairs of one region 6.40 ms,
+// 5.87 ms; 5,265 pairs on the split kernel, whole call 293 us, 280 us.
+struct HapWords {
+    using lds_u32 = const __attribute__((address_space(3))) uint32_t;
+    uint32_t at, word;
+    lds_u32 *next;
+
+    __device__ __forceinline__ explicit HapWords(const uint8_t *first) {  // the byte of step 0
+        using lds_u8 = const __attribute__((address_space(3))) uint8_t;
+        at = (uint32_t)(uintptr_t)(lds_u8 *)first;  // address-space cast: C-style only
+        lds_u32 *w = (lds_u32 *)(uintptr_t)(at & ~3u);
+        word = w[0];
+        next = w + 1;
+    }
+    // The bytes of the kU steps from t0, of successive blocks.
+    template <int kU>
+    __device__ __forceinline__ void block(int t0, uint32_t (&hbs)[kU]) {
+#pragma unroll
+        for (int q = 0; q < kU / 4; ++q) {
+            const uint32_t w = next[t0 / 4 + q];
+            const uint32_t four = __builtin_amdgcn_alignbyte(w, word, at);
+            word = w;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) hbs[4 * q + u] = (four >> (8 * u)) & 0xFFu;
+        }
+    }
+};
+
 // One stripe of steps.  Returns the lane's D' after the last step (a SUM row's last-row sum).
 template <int kCols, bool kHapHasN, int kU>
 __device__ __forceinline__ float packed_steps(const WaveLds<float> &L, const uint8_t *hap, int lane,
                                               const PackedRow &x, int steps) {
     PackedState st = packed_start(x);
-    using lds_u8 = const volatile __attribute__((address_space(3))) uint8_t;
-    lds_u8 *hp = (lds_u8 *)(hap + kLdsPad - 1 - lane + x.shift);  // address-space cast: C-style only
+    HapWords bytes(hap + kLdsPad - 1 - lane + x.shift);
     // Every lane stores its M and I at its own column c = t - lane at step t, so the step has no
     // one-lane exec mask (no exec writes, no branch).  Lane 63 writes column c last, at step c + 63,
     // so the planes end with its row; lane 0 has read A and B of column c by step c, before any lane
@@ -919,8 +951,7 @@ __device__ __forceinline__ float packed_steps(const WaveLds<float> &L, const uin
         __builtin_memcpy(av, __builtin_assume_aligned(L.bm + kLdsPad + t0, 16), sizeof(av));
         __builtin_memcpy(bv, __builtin_assume_aligned(L.bi + kLdsPad + t0, 16), sizeof(bv));
         uint32_t hbs[kU];
-#pragma unroll
-        for (int u = 0; u < kU; ++u) hbs[u] = hp[t0 + u];
+        bytes.block(t0, hbs);
         __builtin_amdgcn_wave_barrier();
         packed_block<kHapHasN, kU, 4>(st, x.w, x.nval, av, bv, hbs, wm + t0, wi + t0);
     }
@@ -1133,8 +1164,7 @@ __device__ __forceinline__ float split_stripe(const DeviceBatch &b, const Device
     const int wend = kLdsPad - (kWave - 1) + steps;
     const int jmax = plane_span<kCols>(steps);
     PackedState st = packed_start(x);
-    using lds_u8 = const volatile __attribute__((address_space(3))) uint8_t;
-    lds_u8 *hp = (lds_u8 *)(L.hap + kLdsPad - 1 - lane + x.shift);  // address-space cast: C-style only
+    HapWords bytes(L.hap + kLdsPad - 1 - lane + x.shift);
     using lds_f32 = __attribute__((address_space(3))) float;
     int lane_w = lane;
     asm volatile("" : "+v"(lane_w));
@@ -1165,8 +1195,7 @@ __device__ __forceinline__ float split_stripe(const DeviceBatch &b, const Device
                 for (int u = 0; u < kU; ++u) av[u] = bv[u] = 0.f;
             }
             uint32_t hbs[kU];
-#pragma unroll
-            for (int u = 0; u < kU; ++u) hbs[u] = hp[t0 + u];
+            bytes.block(t0, hbs);
             __builtin_amdgcn_wave_barrier();
             packed_block<kHapHasN, kU, 1>(st, x.w, x.nval, av, bv, hbs, wm + t0, wi + t0);
             asm volatile("" ::: "memory");  // a wave's LDS operations complete in the order they are issued
