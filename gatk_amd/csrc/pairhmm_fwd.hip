@@ -43,6 +43,13 @@ using namespace dev;
 
 constexpr int kUnroll = 8;  // wave-steps per unrolled loop body
 
+// Every lane stores its cell at its own column, so a column is stored by all lanes, a step apart, and the last
+// store, lane 63's, has to come last.  The compiler sees one lane, whose stores are to different addresses,
+// and its schedulers reorder them unless the steps are held apart.  FP32 steps are held apart in pairs:
+// two steps' stores go out as one ds_write2, lower column first (single stores: 44.8 against 39.7 ms on 300
+// regions, LDS-bound).  check_isa.py checks the order in the assembly.
+__device__ __forceinline__ void store_order() { asm volatile("" ::: "memory"); }
+
 template <typename T>
 struct WaveLds {
     uint8_t *hap;      // [cols]: haplotype byte of column c (1-based) at kLdsPad + c - 1
@@ -268,6 +275,7 @@ __device__ double forward_pair_f32(const WaveLds<T> &L, int lane, int H, int R, 
                 const T sx = fma(MD, d, i);
                 wmb[u] = m;
                 wib[u] = i;
+                if (u % 2 == 1) store_order();
                 m2 = m1;
                 s2 = s1;
                 m1 = m;
@@ -493,6 +501,7 @@ __device__ __forceinline__ void f64_stripe(double *P, __attribute__((address_spa
             bn1 = bn;
             wr[2 * u] = bn;
             wr[2 * u + 1] = an;
+            store_order();
             // The next block's halves, loaded unconditionally (the slice has slots past the last
             // block): with a fixed count of loads in the loop, the wait for a half is a counted
             // one instead of a full drain at the block start.
@@ -887,9 +896,7 @@ __device__ __forceinline__ void packed_block(PackedState &st, const RowTrans<flo
         const float sx = fmaf(w.MD, d, i);
         wm[u] = m;
         wi[u] = i;
-        // A column's last store has to come last, and the lanes' stores to it belong to different steps: the
-        // compiler, which sees one lane, may pair two steps' stores but not reorder pairs.
-        if (u % 2 == 1) asm volatile("" ::: "memory");
+        if (u % 2 == 1) store_order();
         st.m2 = st.m1;
         st.s2 = st.s1;
         st.m1 = m;
@@ -1258,6 +1265,7 @@ __global__ __launch_bounds__(kSplitWaves * kWave) void forward_kernel_split(Devi
                     const int R = b.rd_len[r], H = b.hap_len[h];
                     const int64_t ro = b.rd_off[r];
                     const bool hap_n = split_stage<kCols>(b.hap_bases + b.hap_off[h], H, base + kHapGuard, lane);
+                    rec->n_stripes = R > 0 ? static_cast<uint32_t>((R + 3 + kWave - 1) / kWave) : 0u;
                     rec->pair = pair;
                     rec->R = static_cast<uint32_t>(R);
                     rec->H = static_cast<uint32_t>(H);
@@ -1265,7 +1273,6 @@ __global__ __launch_bounds__(kSplitWaves * kWave) void forward_kernel_split(Devi
                     rec->ro_hi = static_cast<uint32_t>(ro >> 32);
                     rec->hap_n = hap_n ? 1u : 0u;
                     for (int k = 0; k < kSplitWaves; ++k) rec->done[k] = 0u;
-                    rec->n_stripes = R > 0 ? static_cast<uint32_t>((R + 3 + kWave - 1) / kWave) : 0u;
                     if (R <= 0) {  // an empty read: L = 0, listed for the FP64 pass
                         b.out[pair] = -__builtin_inf();
                         if (rs.list != nullptr)

@@ -158,6 +158,7 @@ __device__ __forceinline__ void sw_block(SwLane<K> &st, SwEnds &ends, const SwBa
             SwScore *r = rec_out + kSwLow + i;
             r->sw = left;
             r->bgh = bgh;
+            asm volatile("" ::: "memory");  // the steps' stores stay in order: lane 63's to a row comes last
         }
         constexpr int kSpw = sw_steps_per_word(K);
         if (u % kSpw == kSpw - 1) {
