@@ -23,7 +23,7 @@ FORBIDDEN = re.compile(r"^\s*(s_store_|s_buffer_store|s_scratch_store|s_atomic_|
 FLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang",
          "-packed-fp32-ops", "--cuda-device-only", "-S"]
 # Per-file flags of the Makefile's object rules.
-FILE_FLAGS = {f: ["-mllvm", "-enable-post-misched=false"] for f in ("pairhmm_fwd.hip", "pdhmm.hip")}
+FILE_FLAGS = {"pairhmm_fwd.hip": ["-mllvm", "-enable-post-misched=false"]}
 WIDE_LDS_STORE = re.compile(r"^ds_(write|store)_b(96|128)\b")
 LDS_STORE = re.compile(r"^ds_(?:write|store)(2)?(st64)?_b(8|16|32|64|96|128)\s+(v\d+)")
 ORDER_WINDOW = 256  # bytes: 16 steps of up to 16 bytes; planes lie further apart

