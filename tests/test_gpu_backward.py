@@ -152,6 +152,33 @@ def test_adjoint_stripe_and_tile_edges(odd, use_double):
     assert _rel(got["eb"], want["eb"]) <= (1e-7 if use_double else 1e-3)
 
 
+@pytest.mark.parametrize("use_double", [False, True])
+@pytest.mark.parametrize("qb", [45, 50, 60, 70, 90])
+def test_gradient_of_high_base_qualities(qb, use_double):
+    """d log10 L / d qb is proportional to e(qb), which 1 - pm does not hold for high qualities (FP32: 3 % off at
+    Q60, 0 at Q90; FP64: 1e-7 off at Q90).  One error per read; the tolerances of the tests above, on d / d qb alone."""
+    rng = np.random.default_rng(qb)
+    regions = []
+    for R in (30, 64, 100, 150):
+        hap = rng.choice(list(b"ACGT"), R + 6).astype(np.uint8)
+        b = hap[3:3 + R].copy()
+        b[R // 2] = ord("A") if b[R // 2] != ord("A") else ord("C")
+        z = np.zeros(R, np.uint8)
+        regions.append(([hap], [(b, z, z, z, z)]))
+    batch = pack_regions(regions)
+    n = len(batch.read_bases)
+    q = {"qb": np.full(n, qb) + rng.uniform(-2, 2, n), "qi": rng.uniform(30, 50, n), "qd": rng.uniform(30, 50, n),
+         "qc": rng.uniform(8, 15, n)}
+    q = {k: v.astype(np.float32) for k, v in q.items()}
+    _, want = _oracle(batch, q)
+    _, got, _ = _run(batch, q, use_double=use_double)
+    assert _rel(got["qb"], want["qb"]) <= (1e-7 if use_double else 1e-3)
+    # Every position but the error's, whose term is the largest by far.
+    keep = np.ones(n, bool)
+    keep[batch.read_off + batch.read_len // 2] = False
+    assert _rel(got["qb"][keep], want["qb"][keep]) <= (1e-7 if use_double else 1e-3)
+
+
 def test_weighted_sum_of_pairs():
     batch, q = _problem(3)
     w = np.random.default_rng(0).uniform(-2, 2, batch.n_pairs)
