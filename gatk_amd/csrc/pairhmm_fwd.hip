@@ -1102,7 +1102,6 @@ __global__ __launch_bounds__(512) void forward_kernel_packed(DeviceBatch b, Devi
 // round trips, dependent products) and by VALU issue in large ones.  8 steps per block (81 VGPRs, 20 waves
 // per CU) against 16 (105, 16 waves): 288 and 303 us at 5,265 pairs, equal at 1,024.
 constexpr int kSplitWaves = 4;
-constexpr int kSplitStepBits = 20;       // a stripe's progress is published as stripe << 20 | steps done
 constexpr uint32_t kSplitEnd = 0xFFFFFFFFu;  // n_stripes of the record that ends the queue
 
 using lds_u32 = volatile __attribute__((address_space(3))) uint32_t;
@@ -1111,7 +1110,7 @@ using lds_u32 = volatile __attribute__((address_space(3))) uint32_t;
 struct SplitRecord {
     uint32_t seq;  // pair number + 1 once the record is valid
     uint32_t n_stripes, pair, R, H, ro_lo, ro_hi, hap_n;
-    uint32_t done[kSplitWaves];  // progress of the latest stripe s with s mod 4 = k
+    uint32_t done[kSplitWaves];  // split_progress of the latest stripe s with s mod 4 = k
 };
 
 template <int kCols>
@@ -1176,10 +1175,9 @@ __device__ __forceinline__ float split_stripe(const DeviceBatch &b, const Device
     int lane_w = lane;
     asm volatile("" : "+v"(lane_w));
     lds_f32 *wm = (lds_f32 *)(L.bm + kLdsPad) - lane_w, *wi = (lds_f32 *)(L.bi + kLdsPad) - lane_w;
-    const uint32_t before = static_cast<uint32_t>(s - 1) << kSplitStepBits;
     auto follow = [&](int need) {  // until the stripe before has done `need` steps
-        const uint32_t want = before + static_cast<uint32_t>(need < steps ? need : steps);
-        while (lds_get(done + (s - 1) % kSplitWaves) < want) __builtin_amdgcn_s_sleep(1);
+        const uint32_t want = split_progress(static_cast<uint32_t>(s - 1), static_cast<uint32_t>(need < steps ? need : steps));
+        while (!split_reached(lds_get(done + (s - 1) % kSplitWaves), want)) __builtin_amdgcn_s_sleep(1);
         asm volatile("" ::: "memory");
     };
     if (s > 0) {
@@ -1206,7 +1204,7 @@ __device__ __forceinline__ float split_stripe(const DeviceBatch &b, const Device
             __builtin_amdgcn_wave_barrier();
             packed_block<kHapHasN, kU, 1>(st, x.w, x.nval, av, bv, hbs, wm + t0, wi + t0);
             asm volatile("" ::: "memory");  // a wave's LDS operations complete in the order they are issued
-            done[s % kSplitWaves] = (static_cast<uint32_t>(s) << kSplitStepBits) + static_cast<uint32_t>(t0 + kU);
+            done[s % kSplitWaves] = split_progress(static_cast<uint32_t>(s), static_cast<uint32_t>(t0 + kU));
         }
     }
     return st.d1;

@@ -122,6 +122,14 @@ hipError_t launch_zero_counters(uint32_t *counters, int n, hipStream_t stream);
 // Sets n counters from a device array with a kernel (graph-capturable).
 hipError_t launch_copy_counters(uint32_t *counters, const uint32_t *init, int n, hipStream_t stream);
 
+// Progress of a split pair's stripe (forward_kernel_split): its number and the steps it has done in one word, the
+// number modulo 2^12.  Compared by signed difference, so reads of any length may wrap it: the word that a
+// stripe waits on belongs to the stripe before it or to one four stripes earlier or later.
+constexpr int kSplitStepBits = 20;
+static_assert(kMaxFp32Cols < (1 << kSplitStepBits), "a stripe's steps fit");
+constexpr uint32_t split_progress(uint32_t stripe, uint32_t steps) { return (stripe << kSplitStepBits) + steps; }
+constexpr bool split_reached(uint32_t progress, uint32_t want) { return static_cast<int32_t>(progress - want) >= 0; }
+
 // ---- forward + backward (adjoint) over continuous Phred parameters --------------------------
 
 // Wave-steps per recompute tile of the adjoint, i.e. between checkpoints: FP64 (the scratch is sized for it)

@@ -225,3 +225,27 @@ def test_split_stripes(hap_len):
     assert np.array_equal(np.isfinite(outs[0]), fin)
     assert np.max(np.abs(outs[0][fin] - want[fin])) <= 1e-4
     assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
+
+
+def test_split_stripes_of_a_very_long_read():
+    """A read of 4,100 stripes beside two short ones, on a haplotype of 40 bases.  After 40 bases all of it is one
+    insertion: gap continuation Q0 holds its probability, Q1 at one position of each of the last stripes lowers
+    it, so a stripe that took an unfinished row would miss factors and nothing underflows (no pair is redone
+    in FP64)."""
+    rng = np.random.default_rng(23)
+    hap = rng.choice(list(b"ACGT"), 40).astype(np.uint8)
+    reads = []
+    for R in (35, 64 * 4100 - 3, 130):
+        b = np.resize(hap, R).copy()
+        gcp = np.where(np.arange(R) < 38, 10, 0).astype(np.uint8)
+        gcp[64 * 4085::64] = 1
+        reads.append((b, np.full(R, 100, np.uint8), np.full(R, 40, np.uint8), np.full(R, 45, np.uint8), gcp))
+    b = pack_regions([([hap], reads)])
+    want = oracle.logless_batch(b, n_threads=3)
+    assert np.isfinite(want).all()
+    with BatchEngine() as eng:
+        dev = eng.upload(b)
+        o = np.empty(b.n_pairs)
+        assert dev.forward(mode=_native.RUN_PERSISTENT_EAGER, out=o).n_rescued == 0
+        dev.free()
+    assert np.max(np.abs(o - want)) <= 1e-4
