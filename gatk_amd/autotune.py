@@ -6,7 +6,8 @@ a CU's 160 KB), the persistent grid as a fraction of resident capacity, the work
 (descending cost vs submission order), the stripe schedule of the FP32 kernel: packed stripes
 (the rows of consecutive pairs share a wave's 64-row stripes) or aligned stripes (one pair per
 stripe, the read's last stripe padded to 64 rows), and the packed kernel's loop body (8 or 16
-wave-steps per unrolled block, or per LDS class by occupancy).  ``tune`` uploads a sample of the workload, times
+wave-steps per unrolled block, or per LDS class by occupancy).  Small queues share a pair among four waves
+unless the loop body or the waves are set.  ``tune`` uploads a sample of the workload, times
 every candidate's eager pass (FP32 forward plus FP64 rescue, HIP events, best of ``repeats``),
 re-times the fastest few on a larger sample, and returns the fastest.  Results are cached in a JSON
 file keyed by device and a coarse workload signature (haplotype / read length classes), so later

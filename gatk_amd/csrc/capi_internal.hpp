@@ -200,7 +200,7 @@ struct pairhmm_context {
     gatk_pairhmm::capi::HostPinned stage_host;
     gatk_pairhmm::capi::DevBuf grad_scratch32, grad_scratch64, grad_work;  // forward_backward scratch
     gatk_pairhmm::capi::DevBuf f64_planes;   // FP64 boundary planes of computeLikelihoods calls
-    int waves_per_block = 4;  // launch schedule (pairhmm_set_tuning)
+    int waves_per_block = gatk_pairhmm::kWavesPerBlock;  // launch schedule (pairhmm_set_tuning)
     int grid_percent = 100;
     int queue_order = 0;
     int stripe_schedule = 0;  // 0 packed stripes, 1 aligned stripes (FP32 pass)

@@ -463,8 +463,9 @@ hipError_t launch_fp32_slices(const pairhmm_context *ctx, const DeviceBatch &bat
         const QueueSlice &q = slices[k];
         const int64_t n32 = q.count - q.n_direct;
         if (n32 == 0) continue;  // an FP64-only slice, or every pair routed to FP64
-        const LaunchShape sh = forward_shape(false, q.max_hap_len, ctx->waves_per_block, packed, ctx->step_unroll);
+        LaunchShape sh = forward_shape(false, q.max_hap_len, ctx->waves_per_block, packed, ctx->step_unroll);
         if (sh.waves_per_block == 0) return hipErrorInvalidValue;
+        sh.grid_percent = ctx->grid_percent;  // as persistent_grid
         RescueSink rs{rescue_list + q.begin, slice_rescue_count(counters, k), kFp32RescueThreshold};
         WorkSource w{order + q.begin, static_cast<uint32_t>(n32), nullptr, slice_head(counters, k)};
         const hipError_t e = launch_forward(false, batch, tab, w, rs, q.max_hap_len, sh,
@@ -1083,7 +1084,7 @@ extern "C" int32_t pairhmm_dragstr_impute_device(pairhmm_context *ctx, const dou
 extern "C" int32_t pairhmm_set_tuning(pairhmm_context *ctx, const pairhmm_tuning *t) {
     if (!ctx) return fail(PAIRHMM_ERR_STATE, "context is null");
     if (!t) return fail(PAIRHMM_ERR_BAD_ARG, "null tuning");
-    const int wpb = t->waves_per_block == 0 ? 4 : t->waves_per_block;
+    const int wpb = t->waves_per_block == 0 ? kWavesPerBlock : t->waves_per_block;
     const int gp = t->grid_percent == 0 ? 100 : t->grid_percent;
     if (wpb < 1 || wpb > 8) return fail(PAIRHMM_ERR_BAD_ARG, "waves_per_block must be 1..8");
     if (gp < 1 || gp > 400) return fail(PAIRHMM_ERR_BAD_ARG, "grid_percent must be 1..400");

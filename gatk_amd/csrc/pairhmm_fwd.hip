@@ -737,8 +737,6 @@ constexpr size_t packed_lds_per_wave() {
 // the same results while the waves still balance their load dynamically.  The launch sets the chunk
 // (packed_chunk): at most kPackedChunk items, and few enough that every wave of the grid gets about
 // four chunks, so a small queue (one region's pairs) still spreads over the whole GPU.
-constexpr uint32_t kPackedChunk = 16;
-
 struct ChunkCursor {
     uint32_t next = 0, end = 0;  // items [next, end) of the wave's current chunk
     uint32_t wave = 0, waves = 0;  // this wave's number in the launch, and their count
@@ -1354,11 +1352,6 @@ size_t fp64_plane_bytes_per_wave(int max_hap_len) {
     return cols == 0 ? 0 : kPlanes * sizeof(double) * static_cast<size_t>(lds_plane_stride(cols));
 }
 
-uint32_t packed_chunk(int64_t n_items, int64_t waves) {
-    const int64_t c = n_items / (4 * (waves > 0 ? waves : 1));
-    return static_cast<uint32_t>(c < 1 ? 1 : c > kPackedChunk ? kPackedChunk : c);
-}
-
 namespace {
 
 template <typename F>
@@ -1380,12 +1373,12 @@ hipError_t with_kernel(bool fp64, bool packed, int cols, int unroll, F &&f) {
 
 namespace {
 
-// The split kernel for every packed launch whose chunks are one pair (packed_chunk: fewer than eight pairs
-// for each wave of the grid), which is where a wave's pairs would not share stripes anyway.  Measured on
-// one call, packed and split: 1,024 pairs 158 and 129 us, 5,265 pairs 311 and 288, 18,000 pairs 863 and
-// 825, 38,400 pairs 1,189 and 1,196; 200 pairs of 250-600 rows on haplotypes of 1,500 862 and 322.
+// The split kernel, for launches of fewer than eight pairs for each wave of a resident grid (takes_split).
+// Measured on one call, packed and split: 1,024 pairs 158 and 129 us, 5,265 pairs 311 and 288, 18,000 pairs
+// 863 and 825, 38,400 pairs 1,189 and 1,196; 200 pairs of 250-600 rows on haplotypes of 1,500 862 and 322.
+// Its groups have four waves and its loop body 8 steps; its grid is grid_percent of its own resident groups.
 hipError_t launch_split(const DeviceBatch &batch, const DeviceTables &tables, const WorkSource &ws, const RescueSink &rescue,
-                        int cols, hipStream_t stream) {
+                        int cols, int grid_percent, hipStream_t stream) {
     return dispatch_col_class(cols, [&](auto C) -> hipError_t {
         constexpr int kC = decltype(C)::value;
         if constexpr (kC > kMaxFp32Cols) {
@@ -1407,7 +1400,8 @@ hipError_t launch_split(const DeviceBatch &batch, const DeviceTables &tables, co
             if (hipGetDevice(&dev) != hipSuccess ||
                 hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
                 cus = 1;
-            const uint32_t grid = std::min<uint32_t>(ws.n_items, static_cast<uint32_t>(per_cu * cus));
+            const int64_t groups = std::max<int64_t>(1, static_cast<int64_t>(per_cu) * cus * grid_percent / 100);
+            const uint32_t grid = static_cast<uint32_t>(std::min<int64_t>(ws.n_items, groups));
             hipLaunchKernelGGL(kernel, dim3(grid), dim3(kSplitWaves * kWave), split_lds_bytes<kC>(), stream, batch, tables,
                                ws, rescue);
             return hipGetLastError();
@@ -1425,8 +1419,8 @@ hipError_t launch_forward(bool fp64, const DeviceBatch &batch, const DeviceTable
     if (shape.packed && (fp64 || work.head == nullptr || work.n_items_dev != nullptr)) return hipErrorInvalidValue;
     WorkSource ws = work;
     if (shape.packed) ws.chunk = packed_chunk(work.n_items, static_cast<int64_t>(grid_blocks) * shape.waves_per_block);
-    if (shape.packed && ws.chunk == 1)
-        return launch_split(batch, tables, ws, rescue, lds_columns(max_hap_len), stream);
+    if (takes_split(shape, work.n_items, grid_blocks))
+        return launch_split(batch, tables, ws, rescue, lds_columns(max_hap_len), shape.grid_percent, stream);
     const dim3 block(kWave * shape.waves_per_block);
     return with_kernel(fp64, shape.packed, lds_columns(max_hap_len), shape.unroll, [&](auto kernel) {
         if (shape.lds_bytes > 65536)
@@ -1472,6 +1466,7 @@ LaunchShape forward_shape(bool fp64, int max_hap_len, int requested_waves_per_bl
     sh.waves_per_block = wpb;
     sh.lds_bytes = per_wave * static_cast<size_t>(wpb);
     sh.packed = packed;
+    sh.tuned = requested_waves_per_block != kWavesPerBlock || unroll != 0;
     auto occupancy = [&](int u) {
         int blocks = 0;
         const hipError_t e = with_kernel(fp64, packed, cols, u, [&](auto kernel) {

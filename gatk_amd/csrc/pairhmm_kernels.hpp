@@ -86,14 +86,21 @@ int lds_columns(int max_hap_len);
 // LDS of one wave: FP32 aligned stripes (haplotype + two planes), FP32 packed stripes (two haplotype
 // buffers + two planes) or FP64 (haplotype; its planes live in global memory).
 size_t lds_bytes_per_wave(int max_hap_len, bool fp64, bool packed = false);
-// Items per queue chunk of a packed FP32 launch of `waves` waves over n_items items (1..16).
-uint32_t packed_chunk(int64_t n_items, int64_t waves);
+// Items per queue chunk of a packed FP32 launch of `waves` waves over n_items items.
+constexpr uint32_t kPackedChunk = 16;
+constexpr uint32_t packed_chunk(int64_t n_items, int64_t waves) {
+    const int64_t c = n_items / (4 * (waves > 0 ? waves : 1));
+    return static_cast<uint32_t>(c < 1 ? 1 : c > kPackedChunk ? kPackedChunk : c);
+}
 // Index of the LDS column class that holds haplotypes of this length (0 = smallest), -1 if none.
 // Queues split by class let short haplotypes run at the occupancy their smaller LDS slice allows.
 int lds_class_index(int hap_len);
 
 // Dynamic LDS budget per workgroup: the device's limit (queried once), at most 160 KB (gfx950).
 size_t max_lds_per_block();
+
+// Waves per workgroup unless the tuning asks for others.
+constexpr int kWavesPerBlock = 4;
 
 // Launch geometry of the forward kernel for one batch.
 struct LaunchShape {
@@ -102,10 +109,23 @@ struct LaunchShape {
     size_t lds_bytes = 0;     // dynamic LDS per block
     bool packed = false;      // FP32 packed-stripe schedule (rows of consecutive pairs share stripes)
     int unroll = 8;           // packed schedule: wave-steps per unrolled loop body (8 or 16)
+    bool tuned = false;       // waves per block or loop body were asked for
+    int grid_percent = 100;   // the tuning's share of resident capacity that the grid was made for
 };
 
+// Whether a packed launch of grid_blocks blocks takes the split kernel (forward_kernel_split): its chunks are
+// one pair, which is where a wave's pairs would not share stripes anyway, also at a grid of resident
+// capacity if the tuning asks for a larger one; and neither waves per block nor the loop body, which are the packed
+// kernel's, were asked for.
+constexpr bool takes_split(const LaunchShape &shape, uint32_t n_items, int grid_blocks) {
+    const int64_t waves = static_cast<int64_t>(grid_blocks) * shape.waves_per_block;
+    return shape.packed && !shape.tuned &&
+           packed_chunk(n_items, shape.grid_percent > 100 ? waves * 100 / shape.grid_percent : waves) == 1;
+}
+
 // Largest waves-per-block <= requested whose LDS fits kMaxLdsPerBlock, and its occupancy.  packed
-// selects the FP32 packed-stripe kernel (ignored for FP64), which takes its pairs from a queue;
+// selects the FP32 packed-stripe kernel (ignored for FP64), which takes its pairs from a queue
+// (small queues: see takes_split);
 // unroll picks its loop body: 8 or 16 wave-steps, or 0 for 16 where that keeps the occupancy of 8.
 LaunchShape forward_shape(bool fp64, int max_hap_len, int requested_waves_per_block, bool packed = false,
                           int unroll = 0);

@@ -168,6 +168,9 @@ typedef struct pairhmm_tuning {
                                 0 (default): per LDS class, 16 where its extra registers cost no
                                 occupancy (long haplotypes), else 8                              */
 } pairhmm_tuning;
+/* Small queues of packed stripes (fewer than eight pairs for each resident wave) share a pair among the
+ * four waves of a workgroup, on grid_percent of the resident groups, unless step_unroll or other
+ * than four waves_per_block are asked for; likelihoods are the same bit for bit. */
 
 int32_t pairhmm_set_tuning(pairhmm_context *ctx, const pairhmm_tuning *tuning);
 int32_t pairhmm_get_tuning(pairhmm_context *ctx, pairhmm_tuning *tuning);

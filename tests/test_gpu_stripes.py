@@ -227,6 +227,50 @@ def test_split_stripes(hap_len):
     assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
 
 
+@pytest.mark.parametrize("queue_order", [0, 1])
+def test_packed_chunks_of_several_pairs_match_oracle(queue_order):
+    """Chunks of 16 pairs (one wave per workgroup on one percent of the grid), so stripes hold the end of one
+    pair and the start of the next: the edge regions over and over, with rows ending at lane 62 and 63, empty
+    reads and 'N' bytes between other pairs.  Both loop bodies, which agree bit for bit."""
+    rng = np.random.default_rng(31)
+    regions = []
+    for _ in range(12):
+        regions += [_region(rng, [1, 2, 3, 5, 9, 17, 30]), _region(rng, [61, 62, 63, 64, 65, 125, 126, 128]),
+                    _region(rng, [0, 40, 0, 150], hap_n=True), _region(rng, [60, 61, 61, 61, 61, 100], n_haps=1),
+                    _region(rng, [100, 170, 250], hap_len=600, n_haps=7), _region(rng, [5] * 40)]
+    b = pack_regions(regions)
+    want = oracle.logless_batch(b, n_threads=8)
+    outs = []
+    with BatchEngine() as eng:
+        for unroll in (8, 16):
+            Schedule(waves_per_block=1, grid_percent=1, queue_order=queue_order, step_unroll=unroll).apply(eng)
+            dev = eng.upload(b)
+            o = np.empty(b.n_pairs)
+            dev.forward(mode=_native.RUN_PERSISTENT_EAGER, out=o)
+            dev.free()
+            outs.append(o)
+    inf = np.isinf(want)
+    assert inf.any() and np.array_equal(np.isinf(outs[0]), inf)
+    assert np.max(np.abs(outs[0][~inf] - want[~inf])) <= 1e-4
+    assert np.array_equal(outs[0].view(np.int64), outs[1].view(np.int64))
+
+
+def test_split_results_do_not_depend_on_the_grid():
+    """A small queue on a part of the grid, and on more than the resident one: a group takes several pairs, or
+    some groups start late.  The same bits as by default."""
+    b = _batch(37)
+    outs = {}
+    with BatchEngine() as eng:
+        for percent in (100, 1, 50, 400):
+            Schedule(grid_percent=percent).apply(eng)
+            dev = eng.upload(b)
+            outs[percent] = np.empty(b.n_pairs)
+            dev.forward(out=outs[percent])
+            dev.free()
+    for percent in (1, 50, 400):
+        assert np.array_equal(outs[percent].view(np.int64), outs[100].view(np.int64)), percent
+
+
 def test_split_stripes_of_a_very_long_read():
     """A read of 4,100 stripes beside two short ones, on a haplotype of 40 bases.  After 40 bases all of it is one
     insertion: gap continuation Q0 holds its probability, Q1 at one position of each of the last stripes lowers
