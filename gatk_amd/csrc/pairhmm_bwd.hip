@@ -429,8 +429,9 @@ __device__ __forceinline__ void grad_adjoint(const GradBatch &g, const GradLds<T
         const double gII = static_cast<double>(wave_shr1(T(0), aIIn));
         if (p < R) {
             const double ei = static_cast<double>(w.MI), ed = static_cast<double>(w.MD), ec = static_cast<double>(w.II);
-            // Not 1 - pm: rounding below 1 leaves that 3 % off at Q60 in FP32, 0 at Q90.
-            const double eb = 3.0 * static_cast<double>(w.px);
+            // e(qb): 1 - pm is off by up to 2^-25 in FP32, which is more than the gradients' 1e-3 from Q45 on (23 % at
+            // Q70, all of it at Q90).  Lower qualities keep it, and with it the bits of their gradients.
+            const double eb = w.px < T(1e-5) ? 3.0 * static_cast<double>(w.px) : 1.0 - static_cast<double>(w.pm);
             double gE = static_cast<double>(aE);
             if constexpr (kPlain) {
                 const double per_gm = 1.0 / static_cast<double>(w.GM);
