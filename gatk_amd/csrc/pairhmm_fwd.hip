@@ -501,7 +501,9 @@ __device__ __forceinline__ void f64_stripe(double *P, __attribute__((address_spa
             bn1 = bn;
             wr[2 * u] = bn;
             wr[2 * u + 1] = an;
-            store_order();
+            // Holds this step's stores before the next one's (store_order), as the address may be any other one from
+            // here on; a barrier would hold the loads too (75 pairs, one after another's latency: 143 and 146 us).
+            asm("" : "+v"(wr));
             // The next block's halves, loaded unconditionally (the slice has slots past the last
             // block): with a fixed count of loads in the loop, the wait for a half is a counted
             // one instead of a full drain at the block start.
