@@ -282,6 +282,20 @@ struct PostprocessArgs {
     uint8_t *keep;              // [n_reads]
     double *threshold;          // [n_reads] or null
 };
+// A read's qualities are loaded 16 at a time, as granules of a span that begins quality_lead bytes before the read: at
+// the 16-byte boundary before it (aligned loads), unless that lies before the plane or the span would still be
+// shorter than a granule.  Granule k is the span's bytes 16 k .. 16 k + 15, the last one its last 16: no load leaves a
+// span of 16 bytes or more.  The first quality_granule_skip bytes of a granule (0 or less: none) lie before the read
+// or belong to the granule before; 16 or more past the last granule.
+constexpr int quality_lead(uint64_t read, int len, uint64_t plane) {
+    const int lead = static_cast<int>(read & 15);
+    return read - plane >= static_cast<uint64_t>(lead) && lead + len >= 16 ? lead : 0;
+}
+constexpr int quality_granule_at(int span, int k) { return 16 * k + 16 < span ? 16 * k : span - 16; }
+constexpr int quality_granule_skip(int span, int lead, int k) {
+    const int again = 16 * k + 16 - span, before = lead - 16 * k;
+    return again > before ? again : before;
+}
 hipError_t launch_postprocess(const PostprocessArgs &args, hipStream_t stream);
 
 // ---- Smith-Waterman (sw.hip) ----------------------------------------------------------------

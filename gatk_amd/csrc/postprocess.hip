@@ -49,25 +49,33 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// A lane's qualities, as 16-byte granules from the one that holds the first of them (whole granules around
-// valid bytes stay inside the allocation's pages): kGranules from granule k, those that hold any.
-__device__ __forceinline__ void load_granules(uint4 (&g)[kGranules], const uint4 *q, int k, int n) {
+// A lane's qualities as 16-byte granules of a span of `len` bytes (quality_lead): kGranules from granule k, those that
+// hold any.
+__device__ __forceinline__ void load_granules(uint4 (&g)[kGranules], const uint8_t *span, int k, int len) {
 #pragma unroll
     for (int i = 0; i < kGranules; ++i)
-        if (k + i < n) g[i] = q[k + i];
+        if (16 * (k + i) < len) __builtin_memcpy(&g[i], span + quality_granule_at(len, k + i), 16);
 }
 
-// Adds the table entries of a granule's 16 bytes, in order.  kWhole: every byte belongs to the lane's read;
-// else byte b does if at + b lies in [0, L), and the others add entry kNoQual.
+// The granule of a span of fewer than 16 bytes: the read's bytes come last, as in a longer span's last granule.
+__device__ __forceinline__ uint4 load_short(const uint8_t *q, int L) {
+    uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int b = 1; b < 16; ++b)
+        if (b >= 16 - L) w[b / 4] |= static_cast<uint32_t>(q[b - (16 - L)]) << (8 * (b % 4));
+    return uint4{w[0], w[1], w[2], w[3]};
+}
+
+// Adds the table entries of a granule's 16 bytes, in order; its first `skip` bytes add entry kNoQual.  kWhole:
+// none is skipped.
 template <bool kWhole>
-__device__ __forceinline__ void add_granule(const uint4 &g, int at, int L, const double2 *tab, double &s_mean,
-                                            double &s_var) {
+__device__ __forceinline__ void add_granule(const uint4 &g, int skip, const double2 *tab, double &s_mean, double &s_var) {
 #pragma clang fp contract(off)
     const uint32_t w[4] = {g.x, g.y, g.z, g.w};
 #pragma unroll
     for (int b = 0; b < 16; ++b) {
         uint32_t e = (w[b / 4] >> (8 * (b % 4))) & 0xFFu;
-        if (!kWhole) e = static_cast<uint32_t>(at + b) < static_cast<uint32_t>(L) ? e : kNoQual;
+        if (!kWhole) e = b >= skip ? e : kNoQual;
         const double2 mv = tab[e];
         s_mean += mv.x;
         s_var += mv.y;
@@ -78,7 +86,8 @@ __device__ __forceinline__ void add_granule(const uint4 &g, int at, int L, const
 // Staging the qualities in LDS too held a CU to ten waves, took only spans of up to 10,240 bytes per wave
 // (reads of 160 on average; longer ones went byte by byte from global memory) and ran 13 VALU instructions
 // per quality; a lane's own 64-byte loads touch each line about twice and leave 6.  400,000 reads x 8
-// haplotypes, 100-250 bases: a call takes 63 us, 95 with the staged qualities.
+// haplotypes, 100-250 bases: a call takes 64 us, 95 with the staged qualities (63 with last granules that may end
+// after the plane).
 __global__ __launch_bounds__(kPpWaves * 64) void postprocess_kernel(PostprocessArgs p) {
 #pragma clang fp contract(off)
     // The table in LDS by quality byte: per-base lookups differ lane to lane, which LDS serves far better
@@ -116,11 +125,13 @@ __global__ __launch_bounds__(kPpWaves * 64) void postprocess_kernel(PostprocessA
             rt[u] = e < nr * A ? grow[e] : 0.0;
         }
     }
-    const int skip = static_cast<int>(reinterpret_cast<uintptr_t>(q) & 15);  // bytes of the first granule before the read
-    const uint4 *const gq = reinterpret_cast<const uint4 *>(q - skip);
-    const int n_granules = p.dynamic && L > 0 ? (skip + L + 15) / 16 : 0;
+    const int n_quals = p.dynamic && L > 0 ? L : 0;
+    const int lead = quality_lead(reinterpret_cast<uintptr_t>(q), n_quals, reinterpret_cast<uintptr_t>(p.base_quals));
+    const int span_len = lead + n_quals;
     uint4 g[kGranules] = {};
-    load_granules(g, gq, 0, n_granules);
+    const int wide_len = span_len >= 16 ? span_len : 0;
+    load_granules(g, q - lead, 0, wide_len);
+    if (n_quals > 0 && span_len < 16) g[0] = load_short(q, n_quals);
     if (stage_rows) {
 #pragma unroll
         for (int u = 0; u < kRowStage / 64; ++u) {
@@ -149,16 +160,16 @@ __global__ __launch_bounds__(kPpWaves * 64) void postprocess_kernel(PostprocessA
     if (p.dynamic) {
         // Sums in read order, as the reference adds them, the next granules loading meanwhile.
         double s_mean = 0.0, s_var = 0.0;
-        for (int k = 0; __any(k < n_granules); k += kGranules) {
+        for (int k = 0; __any(16 * k < span_len); k += kGranules) {
             uint4 next[kGranules] = {};
-            load_granules(next, gq, k + kGranules, n_granules);
+            load_granules(next, q - lead, k + kGranules, wide_len);
 #pragma unroll
             for (int i = 0; i < kGranules; ++i) {
-                const int at = 16 * (k + i) - skip;  // the granule's first byte in the read
-                if (__all(at >= 0 && at + 16 <= L))
-                    add_granule<true>(g[i], at, L, tab, s_mean, s_var);
-                else if (__any(at < L))
-                    add_granule<false>(g[i], at, L, tab, s_mean, s_var);
+                const int skip = quality_granule_skip(span_len, lead, k + i);
+                if (__all(skip <= 0))
+                    add_granule<true>(g[i], skip, tab, s_mean, s_var);
+                else if (__any(skip < 16))
+                    add_granule<false>(g[i], skip, tab, s_mean, s_var);
             }
 #pragma unroll
             for (int i = 0; i < kGranules; ++i) g[i] = next[i];
