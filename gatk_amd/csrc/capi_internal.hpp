@@ -98,8 +98,6 @@ inline bool haps_packable(const uint8_t *hap, int64_t n) {
                       std::memchr(hap, 1, static_cast<size_t>(n)) == nullptr);
 }
 
-// PairHMM.computeReadLikelihoodGivenHaplotypeLog10 argument checks (PairHMM.java:284-292) and
-// PairHMMModel.qualToTransProbs sign checks (PairHMMModel.java:108-111).
 // Results of a call up to this size are stored by the kernels straight into the call's pinned staging (its
 // inputs are on the device before the first kernel runs), larger ones on the device and copied: the copy
 // is a launch and a wait of its own.  Stored directly / copied: 1,024 pairs' likelihoods 109 / 118 us, 5,265
@@ -107,6 +105,8 @@ inline bool haps_packable(const uint8_t *hap, int64_t n) {
 // larger ones are not measured and keep the copy.
 constexpr size_t kHostResultBytes = size_t(2) << 20;
 
+// PairHMM.computeReadLikelihoodGivenHaplotypeLog10 argument checks (PairHMM.java:284-292) and
+// PairHMMModel.qualToTransProbs sign checks (PairHMMModel.java:108-111).
 inline int32_t validate_read(const uint8_t *b, const uint8_t *q, const uint8_t *ins, const uint8_t *del, const uint8_t *gcp,
                       int64_t len, int64_t idx) {
     if (len < 0) return fail(PAIRHMM_ERR_BAD_ARG, "read " + std::to_string(idx) + " has negative length");

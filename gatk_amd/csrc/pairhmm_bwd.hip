@@ -589,9 +589,9 @@ __device__ __forceinline__ void grad_loop(const GradBatch &g, const WorkSource &
     }
 }
 
-// FP32: bound by VALU issue (91-93 % busy: 35 instructions a step of a 64-row stripe, 1.36 steps for each cell
-// that rows past R and the stripes' fill and drain leave useful) and close to it by the checkpoints' HBM
-// traffic (3 TB/s).  100 regions of reads of 100-250 by haplotypes of 136-607, 519,357 pairs, forward,
+// FP32: bound by VALU issue (90-93 % of one instruction per four cycles: 35 instructions a step of a 64-row
+// stripe, 1.36 steps for each cell that rows past R and the stripes' fill and drain leave useful) and close to it
+// by the checkpoints' HBM traffic (3 TB/s).  100 regions of reads of 100-250 by haplotypes of 136-607, 519,357 pairs, forward,
 // backward and autograd around them: 61.6 ms with 5 checkpoint values every 8 steps, planes written by every
 // lane every step and 40 instructions; 57.5 with the plain adjoint's sums and the shorter last stripe,
 // 54.2 with 4 values and the planes written once a tile, 50.6 with tiles of 12.  Held to 168 VGPRs, three

@@ -907,9 +907,9 @@ __device__ __forceinline__ void packed_block(PackedState &st, const RowTrans<flo
 }
 
 // A lane's haplotype bytes in LDS, four columns a word: aligned words, shifted to the lane's own byte.  Byte
-// loads, one a step, kept a packed launch's LDS 71 % busy beside 90 % of its VALU issue, and each waited
-// for the other: 300 regions 39.7 ms with them, 36.7 ms with words; 128,000 pairs of one region 6.40 ms,
-// 5.87 ms; 5,265 pairs on the split kernel, whole call 293 us, 280 us.
+// loads, one a step, were a third of a packed launch's LDS instructions (0.23 a VALU instruction, 0.15 with
+// words), and VALU and LDS each waited for the other: 300 regions 39.7 ms with them, 36.7 ms with words; 128,000
+// pairs of one region 6.40 ms, 5.87 ms; 5,265 pairs on the split kernel, whole call 293 us, 280 us.
 struct HapWords {
     using lds_u32 = const __attribute__((address_space(3))) uint32_t;
     uint32_t at, word;

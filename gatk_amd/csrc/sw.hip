@@ -423,11 +423,13 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kLong ? 3
 // arrays are a ring: the last wave's records, which nobody reads, land on rows that wave 0 read long before.
 // The cell bits lie as the one-wave kernel lays out stripes of K columns a lane, and wave 0 walks them.
 //
-// A lone wave is bound by its own issue, 19 K + 10 instructions a step; here four SIMDs share a pair, and a
-// step is bound by the latency of its chain of about eight dependent instructions and, once a block, of
-// the LDS round trip behind the barrier.  One region's 81 reads of 100-250 by haplotypes of 150-460: 126 us
-// with a wave per pair, 94 us with this; 81 haplotypes of up to 612 by references of up to 696, whole
-// call: 448 us and 222 us.
+// A lone wave is bound by its own issue, 19 K + 10 instructions a step; here four SIMDs share a pair, and waits
+// bound it: 29 % of the waves' cycles issue a VALU instruction, 56 % wait.  Cycle stamps in a pair (which cost some
+// themselves): 1,400 to 1,500 a block of 8 steps (1,800 to 1,900 where lanes lie outside the rows), of which
+// about 900 are issue and the rest LDS reads and the chain; about 160 more at the barrier; and after 120,000 to
+// 170,000 of sweep 14,000 to 69,000 of traceback, whose reads depend on each other.  One region's 81 reads of
+// 100-250 by haplotypes of 150-460: 126 us with a wave per pair, 94 us with this; 81 haplotypes of up to 612 by
+// references of up to 696, whole call: 448 us and 222 us.
 constexpr int kSplitWaves = 4;
 constexpr int kSplitLag = (kWave + 2 * kSwBlock - 2) / kSwBlock;  // row t + 8 is complete 70 steps after step t
 
@@ -526,7 +528,8 @@ size_t sw_split_lds_bytes(int max_ref_len) {
 }  // namespace
 
 int sw_max_ref_len() {
-    // The longest reference taken: 12 bytes of LDS a row.
+    // What the entry points take: a twelfth of the LDS, in rows.  The sweep needs less (sw_lds_bytes: 9 bytes a row and
+    // 1,224 in all, or 1 a row), the split kernel, which needs 33, is left out where they don't fit (sw_splits).
     return static_cast<int>(max_lds_per_block() / 12) - 66;
 }
 

@@ -17,7 +17,7 @@ using namespace gatk_pairhmm::capi;
 
 namespace {
 
-constexpr int kMaxSwLength = 32767;       // backtrack codes are int16
+constexpr int kMaxSwLength = 32767;       // what the entry points take; the kernels' cell bits hold any length
 constexpr int32_t kMaxSwPenalty = 1000000;  // keeps every score far from int32 overflow
 constexpr size_t kSwScratchBudget = size_t(2) << 30;
 

@@ -1,6 +1,6 @@
 """The PD-HMM kernel skips the branch update on step blocks where no lane's column is special
-(pdhmm.hip: pd_step<kBranch = false>; special columns are set by pd_column_codes in
-pdhmm_capi.cpp: DEL_END, either inside bit, or the column before an inside column).
+(pdhmm.hip: pd_step<kBranch = false>; special columns are set by pd_codes_kernel there: DEL_END, either
+inside bit, or the column before an inside column).
 
 This pins the argument on the CPU with a restatement of the kernel's recurrence in which every cell
 of a non-special column takes the skipping path (the most skipping any block schedule can do): its
